@@ -212,7 +212,7 @@ mpf_status mpf_device_state(mpf_ctx* ctx, void** count, void** index, void** val
 
 /* Kernel timing of the last mpf_step call (timing on), average per step in ms, measured with HIP
  * events on the context's stream: the main step kernel (with the driving-force averaging
- * kernels when they run), and the rest of the step - the deferred-cell kernels and the grain
+ * kernels when they run), and the rest of the step - the deferred-cell kernel and the grain
  * kernel - in `rest_ms`. */
 mpf_status mpf_last_timing(mpf_ctx* ctx, double* step_kernel_ms, double* rest_ms);
 
@@ -268,7 +268,7 @@ mpf_status mpf_adjoint_step(mpf_ctx* ctx, double dt, const double* lam_next, dou
  * three active axes) - plane tiles of 64-256 cells (2D: 64 / 128 / 256 along the active plane
  * axis; 3D: 4x64, 8x32, 16x16, 4x32) times 1 / 4 / 16 / the default number of planes per block,
  * and the per-cell kernel; (2) the XCD-contiguous block order of the step kernel on/off times
- * 256 / 1024 / 4096 / 16384 blocks for the deferred-cell kernels. Results do not depend on the
+ * 256 / 1024 / 4096 / 16384 blocks for the deferred-cell kernel. Results do not depend on the
  * shape. The chosen launch shape is returned through the optional out pointers, the tile by
  * mpf_get_tile_shape. */
 mpf_status mpf_autotune(mpf_ctx* ctx, double dt, int32_t steps, int32_t* xcd_order, int32_t* deferred_grid);
@@ -306,7 +306,7 @@ void mpf_ensemble_destroy(mpf_ensemble* ens);
  * the context's own state is not touched, its grain records (Volume, VolumeRatio, ...) become
  * those of the output state. The step's scratch (deferred-cell work lists, volume accumulators,
  * status words) is one static device array per GPU, cleared at the start of every call: at most
- * 2^19 cells per call (MPF_ERR_UNSUPPORTED beyond, and with driving-force averaging), 10 MiB per
+ * 2^19 cells per call (MPF_ERR_UNSUPPORTED beyond, and with driving-force averaging), 8 MiB per
  * GPU held until the process ends. Calls that overlap on one GPU (other threads, other streams)
  * race on that array. Synchronises on the context's stream and returns the step's status. */
 mpf_status mpf_step_into(mpf_ctx* ctx, double dt, const void* count_in, const void* index_in, const void* value_in,

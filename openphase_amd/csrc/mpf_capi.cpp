@@ -325,6 +325,13 @@ unsigned grain_blocks(const mpf_ctx* c)
     return static_cast<unsigned>((n + mpf::kGrainBlock - 1) / mpf::kGrainBlock);
 }
 
+// Wavefronts of the deferred-cell kernel: no more than one per 32 cells of the domain, which is one
+// per round of four cells while up to an eighth of the cells are deferred.
+int deferred_blocks(const mpf_ctx* c)
+{
+    return static_cast<int>(std::min<int64_t>(c->deferred_grid, (c->ncells + 31) / 32));
+}
+
 // Makes the device copies of the kernel arguments current for time step dt (both parities).
 // Uploads only when something changed (dt, tables, launch shape, grains); then it waits for the
 // copies, so the host arrays can be reused.
@@ -401,14 +408,14 @@ mpf_status launch_step_part(mpf_ctx* c, hipStream_t stream)
 mpf_status launch_rest_part(mpf_ctx* c, hipStream_t stream)
 {
     const bool full = full_variant(c);
-    mpf_status st = c->hip(static_cast<hipError_t>(mpf::launch_deferred(c->d_args + c->cur, 1, c->deferred_grid, c->fp32,
-                                                                        full, stream)), "deferred-cell kernels");
+    mpf_status st = c->hip(static_cast<hipError_t>(mpf::launch_deferred(c->d_args + c->cur, 1, deferred_blocks(c), c->fp32,
+                                                                        full, stream)), "deferred-cell kernel");
     if (!st) st = c->hip(static_cast<hipError_t>(mpf::launch_grains(c->d_gargs, c->d_gfirst, 1, grain_blocks(c), stream)),
                          "grain kernel");
     return st;
 }
 
-// Enqueues one step (step kernel, deferred-cell kernels, grain kernel) on `stream` and flips the
+// Enqueues one step (step kernel, deferred-cell kernel, grain kernel) on `stream` and flips the
 // double buffer.
 mpf_status enqueue_step(mpf_ctx* c, double dt, hipStream_t stream)
 {
@@ -472,8 +479,7 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
         return bail(MPF_ERR_UNSUPPORTED, "at most 2^28 - 1 cells per device (e.g. 645^3)");
     c->slots = grid->slots;
     c->fp32 = grid->precision == MPF_FP32;
-    // deferred-cell grid: 16384 blocks from 4M cells on (256^3 FP64 step 3.98 ms at 4096 blocks,
-    // 3.92 at 8192, 3.85 at 16384: the level-0 list then needs one pass), 4096 below
+    // deferred-cell grid: 16384 wavefronts from 4M cells on, 4096 below
     c->deferred_grid = c->ncells >= (int64_t{1} << 22) ? 4 * mpf::kWideGrid : mpf::kWideGrid;
     c->nphases = params->nphases;
     const size_t np2 = static_cast<size_t>(c->nphases) * c->nphases;
@@ -611,7 +617,7 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
         c->hip(dalloc(&c->d_dgmode_off, np2), "tables") ||
         c->hip(dalloc(&c->d_status, mpf::kStatusWords), "status") ||
         c->hip(dalloc(&c->d_first_overflow, 1), "status") || c->hip(dalloc(&c->d_warnings, 1), "status") ||
-        c->hip(dalloc(&c->d_work_list, 4 * N), "work list") || c->hip(dalloc(&c->d_work_count, 4), "work list") ||
+        c->hip(dalloc(&c->d_work_list, 3 * N), "work list") || c->hip(dalloc(&c->d_work_count, 4), "work list") ||
         c->hip(dalloc(&c->d_stats, 2), "statistics") || c->hip(dalloc(&c->d_obs, 4), "statistics"))
         return bail(MPF_ERR_NOMEM, c->err.c_str());
     if (c->reg_active && c->reg_average) {
@@ -1403,7 +1409,7 @@ mpf_status mpf_autotune(mpf_ctx* c, double dt, int32_t steps, int32_t* xcd_order
         c->tile_y = best_ty;
         c->tile_z = best_tz;
     }
-    // 2. block order of the step kernel x grid of the deferred-cell kernels
+    // 2. block order of the step kernel x grid of the deferred-cell kernel
     const int grids[4] = {256, 1024, mpf::kWideGrid, 4 * mpf::kWideGrid};
     best = 1e30f;
     int best_x = x0, best_g = g0;
@@ -1525,7 +1531,7 @@ bool build_args(mpf_ensemble* e, const double* dt)
             // deferred-cell blocks per member: at most 256 (a 64-domain 2D ensemble: 7.0e9
             // cell-updates/s at 256, 6.8e9 at 512, 6.5e9 at 1024, 6.2e9 at 128; most blocks of a
             // small domain find no deferred cell)
-            per = std::max(per, std::min(c->deferred_grid, 256));
+            per = std::max(per, std::min(deferred_blocks(c), 256));
         }
         auto differs = [](const void* x, const void* y, size_t bytes) { return std::memcmp(x, y, bytes) != 0; };
         if (g.h_a1.size() != n || differs(a1.data(), g.h_a1.data(), n * sizeof(mpf::StepArgs)) ||
@@ -1732,9 +1738,9 @@ constexpr size_t kOffStatus = align256(kOffCount + 4 * sizeof(unsigned));       
 constexpr size_t kOffWords = align256(kOffStatus + mpf::kStatusWords * sizeof(int32_t));  // 8 x u64
 constexpr size_t kOffAcc = align256(kOffWords + 8 * sizeof(unsigned long long));
 constexpr size_t kOffList = align256(kOffAcc + size_t{kScratchGrains} * mpf::kLimbs * sizeof(unsigned long long));
-constexpr size_t kScratchBytes = align256(kOffList + 4 * size_t{kScratchCells} * sizeof(uint32_t));
+constexpr size_t kScratchBytes = align256(kOffList + 3 * size_t{kScratchCells} * sizeof(uint32_t));
 
-// 10 MiB + 2.2 KiB per GPU
+// 8 MiB + 2.2 KiB per GPU
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1836,8 +1842,8 @@ mpf_status mpf_step_into(mpf_ctx* c, double dt, const void* count_in, const void
     mpf_status st = c->hip(launch_main(c, a, c->stream), "step kernel");
     if (!st)
         st = c->hip(static_cast<hipError_t>(mpf::launch_deferred(reinterpret_cast<const mpf::StepArgs*>(base + kOffStepArgs), 1,
-                                                                 c->deferred_grid, c->fp32, full, c->stream)),
-                    "deferred-cell kernels");
+                                                                 deferred_blocks(c), c->fp32, full, c->stream)),
+                    "deferred-cell kernel");
     if (!st)
         st = c->hip(static_cast<hipError_t>(mpf::launch_grains(reinterpret_cast<const mpf::GrainArgs*>(base + kOffGrainArgs),
                                                                reinterpret_cast<const uint32_t*>(base + kOffFirst), 1, gblocks,

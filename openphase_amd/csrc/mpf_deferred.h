@@ -1,0 +1,620 @@
+// Deferred cells of the step: the cells whose neighbourhood the main step kernels cannot hold
+// (merged lists of more than four entries, neighbours with long lists, too many grains in a tile).
+// Included by mpf_kernels_variant.hip.
+//
+// A group of lanes takes one cell: 16 lanes, four cells per wavefront. What bounds such a cell is
+// latency - one chain of dependent loads, list searches and divisions - so its work is spread over
+// the group instead of run by one lane: every lane fetches the lists of its two neighbours of the
+// 3^d box (two round trips for the whole cell), the merged list (PhaseField::CalculateDerivativesSR,
+// src/PhaseField.cpp:566-615) is formed with one ballot per appended grain, and then lane t holds
+// entry t (Laplacian, limiter bounds, merge, finalize) and the pair increments are dealt to the
+// lanes. Sums that the reference forms in an order are formed by one lane in that order (stencil
+// order, list order, pair order), so every value equals the one-lane form bit for bit.
+//
+// Lists are held in LDS with run-time lengths, so one kernel takes every length: a cell of more
+// than kGroupCap merged entries, or next to a list of more than kGroupCap, is done again by the
+// whole wavefront with room for kWideSlots. Measured against one thread per cell with register
+// lists in three launches (2-6, 7-10 and up to 16 entries), mid-run states, FP64: 20 us instead of
+// 114 at 2D 512^2 and 22 instead of 120 at 96^2 (a few hundred cells that waited on their own
+// latency), 1.56 ms instead of 2.62 at 256^3; 64 FP32 domains in one launch 84 us instead of 354.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <float.h>
+#include <stdint.h>
+
+#include "mpf_device.h"
+#include "mpf_lists.h"
+#include "mpf_step_ops.h"
+
+namespace mpf {
+
+namespace {
+
+constexpr int kGroupLanes = 16;  // lanes per cell
+constexpr int kGroupCap = 8;     // merged entries a group has room for
+constexpr int kVolSlots = 32;    // grains of the wavefront's volume table
+
+// One cell's list and tables in LDS.
+template <typename TC, bool GRAD, int CAP> struct GroupMem {
+    union {
+        TC a[CAP][27];                 // value of merged entry t at box position k
+        struct {
+            double psi[CAP][CAP + 1];  // increment of (t, u), antisymmetric
+            TC sig[CAP][CAP + 1];      // interface energy of (t, u)
+        } p;
+    };
+    TC gr[GRAD ? CAP : 1][3];
+    double phi[CAP];
+    TC lap[CAP];
+    TC ev[CAP];                        // value in the stencil arithmetic
+    double lim1[CAP], lim2[CAP];
+    double vr[CAP];
+    int ph[CAP];
+    uint32_t eid[CAP];
+};
+
+struct VolTable {
+    int32_t key[kVolSlots];
+    unsigned long long acc[kVolSlots][kLimbs];
+};
+
+// Adds one entry's value to the wavefront's table of exact volume sums, or to the global sums
+// when the table is full.
+__device__ __forceinline__ void table_volume_add(VolTable& V, uint32_t g, double v, unsigned long long* acc, bool& bad)
+{
+    unsigned long long l[kLimbs];
+    value_limbs(v, l, bad);
+    unsigned long long* dst = acc + static_cast<int64_t>(g) * kLimbs;
+    uint32_t h = (g * 0x9E3779B1u) >> 27;
+    for (int i = 0; i < kVolSlots; ++i, h = (h + 1u) & (kVolSlots - 1)) {
+        int k = *static_cast<volatile int32_t*>(&V.key[h]);
+        if (k == -1) {
+            k = atomicCAS(&V.key[h], -1, static_cast<int>(g));
+            if (k == -1) k = static_cast<int>(g);
+        }
+        if (k == static_cast<int>(g)) {
+            dst = V.acc[h];
+            break;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kLimbs; ++i)
+        if (l[i]) atomicAdd(&dst[i], l[i]);
+}
+
+// Largest n over the wavefront's groups of G lanes (n uniform within a group), in a scalar.
+template <int G> __device__ __forceinline__ int wave_max(int n)
+{
+#pragma unroll
+    for (int k = G; k < 64; k <<= 1) n = max(n, __shfl_xor(n, k));
+    return __builtin_amdgcn_readfirstlane(n);
+}
+
+// The ballot's bits of this lane's group, shifted to bit 0.
+template <int G> __device__ __forceinline__ unsigned long long group_bits(unsigned long long m)
+{
+    if (G == 64) return m;
+    const int lane = static_cast<int>(threadIdx.x) & 63;
+    return (m >> (lane & ~(G - 1))) & ((1ull << (G & 63)) - 1ull);
+}
+
+// The step of cell c (when `run`) by the G lanes of this lane's group. Returns true (uniform in
+// the group) when the cell needs more than CAP entries: nothing was written then. All lanes of the
+// wavefront call it together; loops run to the longest list of its groups.
+template <typename TV, typename TC, bool GRAD, bool DG, int G, int CAP>
+__device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t c, GroupMem<TC, GRAD, CAP>& M,
+                                           bool count_long, const uint16_t* pairs, VolTable& V, double& emax,
+                                           double& mmax, bool& bad)
+{
+    constexpr int NK = (27 + G - 1) / G;   // neighbours per lane
+    constexpr int RQ = CAP;                // entries of a neighbour
+    constexpr bool IMPL = ListCode<TV>::kImplicit;
+    const int lane = static_cast<int>(threadIdx.x) & 63, l = lane & (G - 1);
+    const int64_t N = A.ncells;
+    const uint32_t N32 = static_cast<uint32_t>(N);
+    const uint32_t cc = static_cast<uint32_t>(run ? c : 0);
+
+    // ---- the box: positions l, l + G of stencil order
+    const int NY = A.ny, NZ = A.nz;
+    const int z0 = static_cast<int>(cc % static_cast<uint32_t>(NZ));
+    const int y0 = static_cast<int>((cc / static_cast<uint32_t>(NZ)) % static_cast<uint32_t>(NY));
+    const int x0 = static_cast<int>(cc / (static_cast<uint32_t>(NY) * static_cast<uint32_t>(NZ)));
+    const __amdgpu_buffer_rsrc_t rc = plane_rsrc(A.cnt_in, N32);
+    uint32_t nb[NK];
+    bool act[NK];
+    uint8_t code[NK];
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+        const int k = l + j * G;
+        const int ii = k / 9 - 1, jj = (k / 3) % 3 - 1, kk = k % 3 - 1;
+        act[j] = run && k < 27 && (ii == 0 || A.dnx) && (jj == 0 || A.dny) && (kk == 0 || A.dnz);
+        nb[j] = static_cast<uint32_t>((wrap1(x0 + (act[j] ? ii : 0), A.nx) * NY + wrap1(y0 + (act[j] ? jj : 0), NY)) * NZ +
+                                      wrap1(z0 + (act[j] ? kk : 0), NZ));
+        code[j] = buffer_load<uint8_t>(rc, act[j] ? nb[j] : kNoLoad);
+    }
+    const uint8_t code0 = buffer_load<uint8_t>(rc, run ? cc : kNoLoad);
+    const int n0 = ListCode<TV>::count(code0), imp0 = ListCode<TV>::implicit(code0);
+    int m[NK], mtop = n0;
+    bool multi = false;
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+        m[j] = ListCode<TV>::count(code[j]);
+        multi = multi || m[j] > 1;
+        mtop = max(mtop, m[j]);
+    }
+    // a neighbour's list longer than this form holds, or the own one
+    const bool wide = group_bits<G>(__ballot(multi)) != 0ull;
+    bool over = group_bits<G>(__ballot(mtop > CAP)) != 0ull;
+#pragma unroll
+    for (int k = 1; k < 64; k <<= 1) mtop = max(mtop, __shfl_xor(mtop, k));
+    const int qtop = min(__builtin_amdgcn_readfirstlane(mtop), RQ);
+
+    // ---- lists of the lane's neighbours, and entry l of the own list
+    uint32_t g[NK][RQ];
+    TV v[NK][RQ];
+    uint32_t left[NK];   // entries not in the merged list yet (bit q)
+#pragma unroll
+    for (int j = 0; j < NK; ++j) left[j] = 0u;
+#pragma unroll
+    for (int q = 0; q < RQ; ++q) {
+        if (q >= 2 && q >= qtop) {
+#pragma unroll
+            for (int j = 0; j < NK; ++j) { g[j][q] = 0u; v[j][q] = TV(0); }
+            continue;
+        }
+        // slot 0 of the cell in place of a slot it does not use: no branch between the loads
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+            const int64_t at = (q < m[j] ? static_cast<int64_t>(q) * N : 0) + nb[j];
+            g[j][q] = A.id_in[at];
+            v[j][q] = load_val<TV>(A.val_in, at);
+        }
+    }
+    double phi = 0.0;
+    uint32_t eid = 0u;
+    if (l < n0 && l < CAP) {
+        eid = A.id_in[static_cast<int64_t>(l) * N + cc];
+        if (!(IMPL && l == imp0)) phi = static_cast<double>(load_val<TV>(A.val_in, static_cast<int64_t>(l) * N + cc));
+    }
+#pragma unroll
+    for (int j = 0; j < NK; ++j)
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            // a lone implicit entry (FP32) has no stored value: it is 1
+            if (IMPL && q == 0 && m[j] == 1 && ListCode<TV>::implicit(code[j]) == 0) v[j][q] = TV(1);
+            if (q < m[j] && v[j][q] != TV(0)) left[j] |= 1u << q;
+        }
+    if (l < CAP) { M.phi[l] = phi; M.eid[l] = eid; }
+    __syncthreads();
+    if (IMPL) {
+        double others = 0.0;
+        for (int t = 0; t < CAP; ++t)
+            if (t < n0 && t != imp0) others += M.phi[t];
+        __syncthreads();
+        if (l < n0 && l == imp0) {
+            phi = 1.0 - others;
+            M.phi[l] = phi;
+        }
+    }
+
+    // ---- merged list: the own entries, then grains new to the box in stencil order. Row t of
+    // M.a: the value of entry t at every box position
+    int ne = over ? 0 : n0;
+    if (!wide || over) {
+#pragma unroll
+        for (int j = 0; j < NK; ++j) left[j] = 0u;
+    }
+    auto row = [&](int t, uint32_t gid, bool on) {
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+            TC a = TC(0);
+#pragma unroll
+            for (int q = 0; q < RQ; ++q)
+                if (((left[j] >> q) & 1u) && g[j][q] == gid && on) {
+                    a = static_cast<TC>(v[j][q]);
+                    left[j] &= ~(1u << q);
+                }
+            const int k = l + j * G;
+            if (on && k < 27) M.a[t][k] = a;
+        }
+    };
+    const int own_top = wave_max<G>(wide ? ne : 0);
+    for (int t = 0; t < own_top; ++t) row(t, M.eid[t], wide && t < ne);
+    while (true) {
+        uint32_t cand = 0u;
+        unsigned long long who = 0ull;
+#pragma unroll
+        for (int j = NK - 1; j >= 0; --j) {
+            const unsigned long long b = group_bits<G>(__ballot(left[j] != 0u));
+            if (b) {
+                who = b;
+                const int q = __ffs(static_cast<int>(left[j])) - 1;
+                cand = 0u;
+#pragma unroll
+                for (int r = 0; r < RQ; ++r) cand = r == q ? g[j][r] : cand;
+            }
+        }
+        if (!__any(who != 0ull)) break;
+        const int leader = who ? __ffsll(static_cast<long long>(who)) - 1 : 0;
+        const uint32_t gid = static_cast<uint32_t>(__shfl(static_cast<int>(cand), (lane & ~(G - 1)) + leader));
+        bool on = who != 0ull;
+        if (on && ne >= CAP) {
+            over = true;
+            on = false;
+#pragma unroll
+            for (int j = 0; j < NK; ++j) left[j] = 0u;
+        }
+        row(ne, gid, on);
+        if (on) {
+            if (l == ne) eid = gid;
+            ++ne;
+        }
+    }
+    if (l < CAP) M.eid[l] = eid;
+    const bool go = run && !over;            // the cell's result is written by this call
+    const bool work = go && wide;
+    if (work && ne > 6 && count_long && l == 0) atomicAdd(&A.work_count[3], 1u);
+    const int top = wave_max<G>(work ? ne : 0);
+    __syncthreads();
+
+    // ---- Laplacian (gradient) of entry l, in stencil order
+    TC lap = TC(0), gx = TC(0), gy = TC(0), gz = TC(0);
+    if (work && l < ne) {
+#pragma unroll
+        for (int k = 0; k < 27; ++k) {
+            const int ii = k / 9 - 1, jj = (k / 3) % 3 - 1, kk = k % 3 - 1;
+            const int nz = (ii != 0) + (jj != 0) + (kk != 0);
+            const TC a = M.a[l][k];
+            lap += static_cast<TC>(A.wl[nz]) * a;
+            if (GRAD && k != 13) {
+                const TC w = static_cast<TC>(A.wg[nz]);
+                if (ii) gx = gx + (ii < 0 ? -w : w) * a;
+                if (jj) gy = gy + (jj < 0 ? -w : w) * a;
+                if (kk) gz = gz + (kk < 0 ? -w : w) * a;
+            }
+        }
+    }
+    __syncthreads();  // M.p takes M.a's place
+    double vr = 0.0;
+    int ph = 0;
+    if (work && l < ne) {
+        ph = A.gphase[eid];
+        vr = A.gvr[eid];
+    }
+    const TC ev = static_cast<TC>(phi);
+    if (l < CAP) {
+        M.lap[l] = lap;
+        M.ev[l] = ev;
+        M.ph[l] = ph;
+        M.vr[l] = vr;
+        if (GRAD) { M.gr[GRAD ? l : 0][0] = gx; M.gr[GRAD ? l : 0][1] = gy; M.gr[GRAD ? l : 0][2] = gz; }
+    }
+    __syncthreads();
+
+    // ---- pair increments (compute_cell's formulas), pair p = b (b - 1) / 2 + a to lane p mod G
+    const int NP = A.nphases;
+    double localn = 0.0;
+    if (A.consider_nucleus) {
+        for (int t = 0; t < top; ++t) localn += t < ne ? M.vr[t] : 0.0;
+    } else {
+        localn = static_cast<double>(ne);
+    }
+    const double norm_1 = 1.0 / localn;
+    const bool uni = A.uniform != 0 && group_bits<G>(__ballot(work && l < ne && vr != 1.0)) == 0ull;
+    const TC P = static_cast<TC>(A.prefactor);
+    const int np = work ? ne * (ne - 1) / 2 : 0;
+    const int ptop = top * (top - 1) / 2;
+    if (__any(work && !uni)) {
+        for (int p0 = 0; p0 < ptop; p0 += G) {
+            const int p = p0 + l;
+            if (p < np && !uni) {
+                const int a = pairs[p] & 255, b = pairs[p] >> 8;
+                if (GRAD) {
+                    TC da[3], db[3];
+                    for (int d = 0; d < 3; ++d) { da[d] = M.gr[GRAD ? a : 0][d]; db[d] = M.gr[GRAD ? b : 0][d]; }
+                    const TC en = ip_pair_energy<TC>(A, M.ph[a] * NP + M.ph[b], M.eid[a], M.eid[b], M.ev[a], M.ev[b], da, db);
+                    M.p.sig[a][b] = en;
+                    M.p.sig[b][a] = en;
+                } else {
+                    M.p.sig[a][b] = static_cast<TC>(A.sigma[M.ph[a] * NP + M.ph[b]]);
+                    M.p.sig[b][a] = static_cast<TC>(A.sigma[M.ph[b] * NP + M.ph[a]]);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    for (int p0 = 0; p0 < ptop; p0 += G) {
+        const int p = p0 + l;
+        if (p < np) {
+            const int a = pairs[p] & 255, b = pairs[p] >> 8;
+            const int k = M.ph[a] * NP + M.ph[b];
+            TC d, mob;
+            if (uni) {
+                const TC s0 = static_cast<TC>(A.sigma0);
+                const TC mf = static_cast<TC>(A.mu0) * static_cast<TC>(norm_1);
+                d = s0 * ((M.lap[a] + P * M.ev[a]) - (M.lap[b] + P * M.ev[b]));
+                d *= mf;
+                mob = static_cast<TC>(A.mu0);
+                emax = smax(emax, static_cast<double>(s0));
+                mmax = smax(mmax, A.mu0);
+            } else {
+                const double scaled = sqrt(M.vr[a] * M.vr[b]);
+                const TC scale = static_cast<TC>(scaled);
+                const TC cf = TC(0.5) * (TC(1.0) + scale) * P;
+                d = M.p.sig[a][b] * ((M.lap[a] + cf * M.ev[a]) - (M.lap[b] + cf * M.ev[b]));
+                for (int g2 = 0; g2 < ne; ++g2) {
+                    if (g2 == a || g2 == b) continue;
+                    d += (M.p.sig[b][g2] - M.p.sig[a][g2]) * (M.lap[g2] + cf * M.ev[g2]);
+                    if (A.tj_model == 0) {
+                        if (A.tj_factor != 0.0 || scaled < 1.0) {
+                            const int pg = M.ph[g2];
+                            const TC e3 = static_cast<TC>(A.sigma[k]) + static_cast<TC>(A.sigma[M.ph[b] * NP + pg]) +
+                                          static_cast<TC>(A.sigma[M.ph[a] * NP + pg]);
+                            d += static_cast<TC>(smax(A.tj_factor, (1.0 - scaled))) * P * e3 *
+                                 (M.ev[a] * M.ev[g2] - M.ev[b] * M.ev[g2]);
+                        }
+                    } else if (A.tj_model == 1) {
+                        d += static_cast<TC>(A.tj_energy) * P * (M.ev[a] * M.ev[g2] - M.ev[b] * M.ev[g2]);
+                    }
+                }
+                mob = static_cast<TC>(A.mu[k]);
+                emax = smax(emax, static_cast<double>(M.p.sig[a][b]));
+                mmax = smax(mmax, static_cast<double>(mob));
+                if (DG && A.reg) {
+                    d = d * mob * static_cast<TC>(norm_1) * scale;
+                    if (A.reg_active) {
+                        d *= static_cast<TC>(A.reg_factor);
+                        if (A.curv != nullptr && n0 > 1 && b < n0) {
+                            const TC kappa = static_cast<TC>(A.curv[static_cast<int64_t>(p) * N + c]);
+                            d += kappa * mob * sqrt(M.ev[a] * M.ev[b]) * static_cast<TC>(A.dg_prefactor);
+                        }
+                    }
+                } else {
+                    d *= mob * static_cast<TC>(norm_1) * scale;
+                }
+            }
+            if (DG && n0 > 1 && A.dg_mode[k] == 1) {
+                const TC raw = dg_local<TC>(A, a, b, n0, c, k);
+                const TC weight = sqrt(M.ev[a] * M.ev[b]);
+                const TC allowed = static_cast<TC>(A.dg_allowed[k]);
+                const TC dgl = allowed * tanh(raw / allowed);
+                d += dgl * mob * weight * static_cast<TC>(A.dg_prefactor);
+            }
+            M.p.psi[a][b] = static_cast<double>(d);
+            M.p.psi[b][a] = -static_cast<double>(d);
+        }
+    }
+    __syncthreads();
+
+    // ---- limiter (FP64). A pair the reference drops from the increment list holds 0 here
+    const double dt = A.dt;
+    if (work && ne == 2 && l == 0) {
+        double d = M.p.psi[0][1];
+        const double va = d * dt;
+        const double old = phi;
+        if ((old == 0.0 && va < 0.0) || (old == 1.0 && va > 0.0)) {
+            d = 0.0;
+        } else {
+            const double nv = old + va;
+            double norm = 1.0;
+            if (nv < 0.0) norm *= -old / va;
+            else if (nv > 1.0) norm *= (1.0 - old) / va;
+            if (norm > DBL_EPSILON) d *= norm;
+            else d = 0.0;
+        }
+        M.p.psi[0][1] = d;
+        M.p.psi[1][0] = -d;
+    }
+    const bool many = work && ne > 2;
+    if (__any(many)) {
+        // zero the pairs that would push a field at 0 below or at 1 above, entry after entry
+        int done = -1;
+        while (true) {
+            bool stop = false;
+            if (many && l < ne && l > done) {
+                double dpsi = 0.0;
+                for (int u = 0; u < ne; ++u)
+                    if (u != l) dpsi += M.p.psi[l][u];
+                stop = (phi == 0.0 && dpsi < 0.0) || (phi == 1.0 && dpsi > 0.0);
+            }
+            const unsigned long long b = group_bits<G>(__ballot(stop));
+            if (!__any(stop)) break;
+            __syncthreads();
+            if (b) {
+                done = __ffsll(static_cast<long long>(b)) - 1;
+                if (l < ne && l != done) {
+                    M.p.psi[l][done] = 0.0;
+                    M.p.psi[done][l] = 0.0;
+                }
+            }
+            __syncthreads();
+        }
+        bool needed = many;
+        for (int iter = 1; iter <= 25 && __any(needed); ++iter) {
+            if (needed && l < ne) {
+                double pos = 0.0, neg = 0.0;
+                for (int u = 0; u < ne; ++u) {
+                    if (u == l) continue;
+                    const double x = M.p.psi[l][u];
+                    if (x < 0.0) neg += x;
+                    if (x > 0.0) pos += x;
+                }
+                double lim1 = 1.0, lim2 = 1.0;
+                const double npf = phi + (pos + neg) * dt;
+                if (npf < 0.0) lim2 = smin(lim2, -(phi + pos * dt) / (neg * dt));
+                if (npf > 1.0) lim1 = smin(lim1, (1.0 - (phi + neg * dt)) / (pos * dt));
+                M.lim1[l] = lim1;
+                M.lim2[l] = lim2;
+            }
+            __syncthreads();
+            bool again = false;
+            for (int p0 = 0; p0 < ptop; p0 += G) {
+                const int p = p0 + l;
+                if (needed && p < np) {
+                    const int a = pairs[p] & 255, b = pairs[p] >> 8;
+                    double x = M.p.psi[a][b];
+                    if (x < 0.0) {
+                        const double t = smin(M.lim2[a], M.lim1[b]);
+                        x *= t;
+                        if (t < 1.0) again = true;
+                    }
+                    if (x > 0.0) {
+                        const double t = smin(M.lim1[a], M.lim2[b]);
+                        x *= t;
+                        if (t < 1.0) again = true;
+                    }
+                    M.p.psi[a][b] = x;
+                    M.p.psi[b][a] = -x;
+                }
+            }
+            needed = needed && group_bits<G>(__ballot(again)) != 0ull;
+            __syncthreads();
+        }
+        // plausibility check of the limited increments (warning count)
+        if (many && l < ne) {
+            double tv = phi;
+            for (int u = 0; u < ne; ++u) {
+                if (u == l) continue;
+                const double x = M.p.psi[l][u];
+                if (x == 0.0 || fabs(x * dt) < DBL_EPSILON) continue;
+                tv += x * dt;
+            }
+            if (tv < -FLT_EPSILON || tv > 1.0 + FLT_EPSILON) atomicAdd(A.warnings, 1ull);
+        }
+    }
+    __syncthreads();
+
+    // ---- merge, then finalize (NodePF::finalize); a bulk cell keeps its list
+    bool keep = go && l < ne;
+    if (work && l < ne) {
+        for (int u = 0; u < ne; ++u) {
+            if (u == l) continue;
+            const double value = M.p.psi[l][u] * dt;
+            if (fabs(value) >= DBL_EPSILON) phi += value;
+        }
+        if (phi >= 1.0 - DBL_EPSILON) phi = 1.0;
+        if (phi <= 0.0 + DBL_EPSILON) { phi = 0.0; keep = false; }
+        M.phi[l] = phi;
+    }
+    unsigned long long kept = group_bits<G>(__ballot(keep));
+    const int ns = __popcll(kept);
+    __syncthreads();
+    if (work) {
+        double total = 0.0;
+        for (int t = 0; t < ne; ++t) total += M.phi[t];
+        if (ns > 1) {
+            const double norm = 1.0 / total;
+            if (keep) phi *= norm;
+        } else if (ns == 1) {
+            if (keep) phi = 1.0;
+        }
+        if (ns == 0 && l == 0) atomicOr(&A.status[kStatusEmpty], 1);
+    }
+    __syncthreads();
+
+    // ---- store (store_cell): FP32 lists hold their first largest entry implicitly
+    if (go && ns > A.slots) {
+        if (l == 0) {
+            atomicOr(&A.status[kStatusOverflow], 1);
+            atomicMin(A.first_overflow, static_cast<unsigned long long>(c));
+        }
+        keep = false;
+    } else if (go) {
+        const int w = __popcll(kept & ((1ull << l) - 1ull));
+        const TV sv = static_cast<TV>(phi);
+        int imp = -1;
+        if (IMPL) {
+            if (l < CAP) M.phi[l] = phi;
+            __builtin_amdgcn_wave_barrier();
+            double vmax = -1.0, others = 0.0;
+            for (int t = 0; t < ne; ++t)
+                if (((kept >> t) & 1ull) && M.phi[t] > vmax) { vmax = M.phi[t]; imp = t; }
+            for (int t = 0; t < ne; ++t)
+                if (((kept >> t) & 1ull) && t != imp) others += static_cast<double>(static_cast<TV>(M.phi[t]));
+            phi = l == imp ? 1.0 - others : static_cast<double>(sv);
+        }
+        if (keep) {
+            A.id_out[static_cast<int64_t>(w) * N + c] = static_cast<uint16_t>(eid);
+            if (!(IMPL && l == imp && ns == 1)) static_cast<TV*>(A.val_out)[static_cast<int64_t>(w) * N + c] = sv;
+        }
+        if (l == 0) {
+            const int wi = IMPL && imp >= 0 ? __popcll(kept & ((1ull << imp) - 1ull)) : 0;
+            A.cnt_out[c] = static_cast<uint8_t>(IMPL ? (ns | (wi << 4)) : ns);
+        }
+    }
+    if (keep) table_volume_add(V, eid, phi, A.vol_acc, bad);
+    return run && over;
+}
+
+// One wavefront per block; wavefront i of a domain takes the i-th part of its deferred cells (the
+// concatenated lists), neighbours in the list being neighbours in the grid.
+template <typename TV, typename TC, bool GRAD, bool DG>
+__global__ __launch_bounds__(64) void deferred_kernel(const StepArgs* __restrict__ batch, int32_t ndom)
+{
+    constexpr int G = kGroupLanes, C = 64 / G;
+    __shared__ union Arena {
+        GroupMem<TC, GRAD, kGroupCap> cell[C];
+        GroupMem<TC, GRAD, kWideSlots> one;
+    } mem;
+    __shared__ uint16_t pairs[kWideSlots * (kWideSlots - 1) / 2];
+    __shared__ VolTable V;
+    const unsigned per = gridDim.x / static_cast<unsigned>(ndom);
+    const unsigned dom = blockIdx.x / per, part = blockIdx.x - dom * per;
+    const StepArgs& A = batch[dom];
+    const unsigned n0 = A.work_count[0], n1 = A.work_count[1], n2 = A.work_count[2];
+    const unsigned n = n0 + n1 + n2;
+    if (n == 0u) return;
+    // whole rounds of C cells per wavefront
+    const unsigned rounds = (n + C - 1) / C, chunk = (rounds + per - 1) / per * C;
+    const unsigned begin = min(n, part * chunk), end = min(n, begin + chunk);
+    if (begin >= end) return;
+    const int lane = static_cast<int>(threadIdx.x);
+    for (int p = lane; p < kWideSlots * (kWideSlots - 1) / 2; p += 64) {
+        int b = 1;
+        while (b * (b + 1) / 2 <= p) ++b;
+        pairs[p] = static_cast<uint16_t>((p - b * (b - 1) / 2) | (b << 8));
+    }
+    if (lane < kVolSlots) V.key[lane] = -1;
+    for (int i = lane; i < kVolSlots * kLimbs; i += 64) (&V.acc[0][0])[i] = 0ull;
+    __syncthreads();
+    double emax = 0.0, mmax = 0.0;
+    bool bad = false;
+    auto cell_of = [&](unsigned i) -> int64_t {
+        if (i < n0) return A.work_list[i];
+        if (i < n0 + n1) return A.work_list[A.ncells + (i - n0)];
+        return A.work_list[2 * A.ncells + (i - n0 - n1)];
+    };
+    for (unsigned base = begin; base < end; base += C) {
+        const unsigned i = base + static_cast<unsigned>(lane / G);
+        const bool run = i < end;
+        const int64_t c = run ? cell_of(i) : 0;
+        const bool big = group_cell<TV, TC, GRAD, DG, G, kGroupCap>(A, run, c, mem.cell[lane / G], i < n0, pairs, V, emax,
+                                                                    mmax, bad);
+        unsigned long long todo = __ballot(big && (lane & (G - 1)) == 0);
+        __syncthreads();
+        while (todo) {
+            const int from = __ffsll(static_cast<long long>(todo)) - 1;
+            todo &= todo - 1ull;
+            const int64_t cb = static_cast<int64_t>(__shfl(static_cast<int>(c), from));
+            const bool first = base + static_cast<unsigned>(from / G) < n0;
+            if (group_cell<TV, TC, GRAD, DG, 64, kWideSlots>(A, true, cb, mem.one, first, pairs, V, emax, mmax, bad) &&
+                lane == 0) {
+                atomicOr(&A.status[kStatusOverflow], 1);
+                atomicMin(A.first_overflow, static_cast<unsigned long long>(cb));
+            }
+            __syncthreads();
+        }
+    }
+    note_maxima(A.obs, emax, mmax);
+    if (__any(bad) && lane == 0) atomicOr(&A.status[kStatusVolumeRange], 1);
+    for (int i = lane; i < kVolSlots * kLimbs; i += 64) {
+        const int s = i / kLimbs;
+        const unsigned long long x = V.acc[s][i - s * kLimbs];
+        if (x) atomicAdd(&A.vol_acc[static_cast<int64_t>(V.key[s]) * kLimbs + (i - s * kLimbs)], x);
+    }
+}
+
+}  // namespace
+
+}  // namespace mpf

@@ -7,8 +7,7 @@ namespace mpf {
 
 constexpr int kMaxSlots = 16;                        // largest per-cell list capacity of the stored state
 constexpr int kBlock = 256;                          // threads per block of the step kernels
-constexpr int kWideBlock = 64;                       // threads per block of the deferred-cell kernel
-constexpr int kWideGrid = 4096;                      // blocks of the deferred-cell kernels (grid-stride)
+constexpr int kWideGrid = 4096;                      // blocks (wavefronts) of the deferred-cell kernel
 constexpr int kLimbs = 4;                            // 32-bit limbs of the exact per-grain volume sums
 
 // Device status words (one int each).
@@ -74,10 +73,11 @@ struct StepArgs {
     // largest interface energy and mobility of the pairs this step's IP.Set evaluates (FP64 bit
     // patterns of non-negative values, atomicMax): InterfaceProperties maxEnergies/maxMobilities
     unsigned long long* obs;
-    uint32_t* work_list;         // deferred cells: four lists of ncells each (mid kernel levels 0-2; wide kernel)
-    unsigned* work_count;        // [4] lengths of the four lists
+    uint32_t* work_list;         // deferred cells: three lists of ncells each, by merged length where it is
+                                 // known (up to 6 or unknown; 7-8; more)
+    unsigned* work_count;        // [4] their lengths, and the cells of list 0 that have more than 6 entries
     // launch shape (chosen by mpf_autotune): XCD-contiguous block order of the step kernel, and
-    // the number of blocks of the grid-stride deferred-cell kernels
+    // the number of blocks of the deferred-cell kernel
     int32_t xcd_order;
     int32_t deferred_grid;
     // LDS-tiled step kernel (mpf_tile.hip): tile of tile_y x tile_z cells of the (y, z) plane
@@ -180,7 +180,7 @@ int launch_curvature(const CurvArgs& a, bool average, void* stream);
 // grain kernels run over one or several domains of the same kernel variant in one launch: `args`
 // (device memory) holds one argument block per domain and `first` (device, ndom + 1 entries) the
 // prefix sums of the domains' block counts (the step kernel takes a single domain's arguments by
-// value in `one` when ndom is 1, and ignores `args` then); the deferred-cell kernels give every domain
+// value in `one` when ndom is 1, and ignores `args` then); the deferred-cell kernel gives every domain
 // `per_domain` blocks. `full`: orientation-dependent energies and/or constant driving force;
 // `uni`: the equal-energy form.
 int launch_step(const StepArgs& one, const StepArgs* args, const uint32_t* first, int ndom, unsigned blocks, bool fp32,

@@ -13,8 +13,8 @@
 //
 // Work per cell is dominated by the merged-list length n (2-4 in grain growth). The main kernel
 // merges in registers with capacity 4 and compiles the pair/limiter/finalize part separately for
-// n = 2, 3, 4, so a wavefront only executes the sizes its cells have. Cells with longer lists go
-// to a work list for a second kernel (n = 5, 6 in registers) and from there to a third (up to 16).
+// n = 2, 3, 4, so a wavefront only executes the sizes its cells have. Cells with longer lists (up
+// to 16) go to a work list for the deferred-cell kernel (mpf_deferred.h).
 // The neighbour lists are read with batched loads (all count bytes of the box, then the first two
 // entries of each plane of nine neighbours), so a wavefront waits on a few memory round trips per
 // cell rather than one per neighbour entry.
@@ -137,7 +137,7 @@ __global__ void grains_kernel(const GrainArgs* __restrict__ batch, const uint32_
     const int g = static_cast<int>(blockIdx.x - first[dom]) * blockDim.x + threadIdx.x;
     if (g == 0) {
         G.stats[0] += G.work_count[0];
-        G.stats[1] += G.work_count[1] + G.work_count[2];
+        G.stats[1] += G.work_count[1] + G.work_count[2] + G.work_count[3];
         G.work_count[0] = 0u;
         G.work_count[1] = 0u;
         G.work_count[2] = 0u;

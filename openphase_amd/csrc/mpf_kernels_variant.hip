@@ -1,8 +1,9 @@
-// One variant of the per-cell step and deferred-cell kernels (mpf_step_kernels.h), compiled once
+// One variant of the per-cell step kernel (mpf_step_kernels.h) and the deferred-cell kernel (mpf_deferred.h), compiled once
 // per precision and variant with MPF_VARIANT_FP32 (0 FP64, 1 FP32) and MPF_VARIANT_FULL (0 plain
 // isotropic, 1 orientation-dependent energies and driving force), so the four variants build in
 // parallel. The launchers sit in namespace mpf::v{64,32}_{plain,full} (mpf_device.h).
 #include "mpf_step_kernels.h"
+#include "mpf_deferred.h"
 
 #if MPF_VARIANT_FP32
 #define MPF_TV float
@@ -41,12 +42,9 @@ int launch_step(const StepArgs& one, const StepArgs* args, const uint32_t* first
 int launch_deferred(const StepArgs* args, int ndom, int per_domain, void* stream)
 {
     constexpr bool F = MPF_VARIANT_FULL != 0;
-    const dim3 grid(static_cast<unsigned>(per_domain) * static_cast<unsigned>(ndom));
-    const dim3 grid2(2u * static_cast<unsigned>(per_domain) * static_cast<unsigned>(ndom));
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL((mid_kernel<MPF_TV, MPF_TV, F, F, 0>), grid, dim3(kWideBlock), 0, s, args, ndom);
-    hipLaunchKernelGGL((mid_tail_kernel<MPF_TV, MPF_TV, F, F>), grid2, dim3(kWideBlock), 0, s, args, ndom);
-    hipLaunchKernelGGL((wide_kernel<MPF_TV, MPF_TV, F, F>), grid, dim3(kWideBlock), 0, s, args, ndom);
+    hipLaunchKernelGGL((deferred_kernel<MPF_TV, MPF_TV, F, F>),
+                       dim3(static_cast<unsigned>(per_domain) * static_cast<unsigned>(ndom)), dim3(64), 0,
+                       static_cast<hipStream_t>(stream), args, ndom);
     return static_cast<int>(hipGetLastError());
 }
 

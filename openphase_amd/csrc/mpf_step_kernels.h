@@ -1,4 +1,4 @@
-// Step and deferred-cell kernels of the per-cell path (templates), instantiated per precision and
+// Step kernel of the per-cell path (template), instantiated per precision and
 // variant by mpf_kernels_variant.hip. See mpf_kernels.hip for what the step computes.
 #pragma once
 
@@ -40,7 +40,7 @@ __device__ __forceinline__ void wave_volume_add_split(bool act, uint32_t g, doub
 // box: bulk cells (one entry, no multi-entry neighbour) keep their list and are copied through;
 // wide cells are compacted in thread order into LDS. Phase 2 runs full wavefronts of wide cells
 // through merge, pair increments, limiter, merge and finalize, so bulk lanes no longer ride along
-// with interface lanes. Cells needing more than kMainSlots entries go to the mid kernel's list.
+// with interface lanes. Cells needing more than kMainSlots entries go to the deferred-cell list.
 constexpr int kStepWaves = kBlock / 64;
 
 template <typename TV, typename TC, bool GRAD, bool DG, bool UNI>
@@ -127,9 +127,9 @@ __device__ __forceinline__ void step_block(const StepArgs& A, int64_t base, uint
         load_own<K, TV, TC, GRAD>(A, cw, box_code(codes, 13), L);
         int r = merge_neighbours<K, TV, TC, GRAD, true>(A, make_box(A, cw), codes, L);
         if (r == kCellWide) {
-            // merged lists of 2-4 entries here; longer ones (few cells) go to the mid kernel
+            // merged lists of 2-4 entries here; longer ones (few cells) are deferred
             // UNI: the equal-energy form only; cells next to a grain below its reference volume
-            // (VolumeRatio < 1) go to the mid kernel
+            // (VolumeRatio < 1) are deferred
             constexpr int PATH = UNI ? 1 : 2;
             bool done = false;
             switch (L.ne) {
@@ -178,130 +178,6 @@ __global__ __launch_bounds__(kBlock, (GRAD || DG) ? 3 : 6) void step_kernel(cons
         const int dom = batch_domain(first, ndom, gb);
         step_block<TV, TC, GRAD, DG, UNI>(batch[dom], static_cast<int64_t>(gb - first[dom]) * kBlock, s_codes, s_list,
                                           s_wide);
-    }
-}
-
-// Cells the main kernel deferred, with register-resident lists. LEVEL 0 (list 0: merged lists of
-// 5-6 entries, more than 4 own entries, or 2-4 entries next to a grain below its reference
-// volume) computes 2-6 entries with capacity 8 and sends 7-8 entries to list 1 and longer lists
-// (capacity 8 exceeded) to list 2; LEVEL 1 computes 7 and 8 entries, LEVEL 2 (capacity 12) 9 and
-// 10; both send anything else to list 3, the 16-entry kernel's. Lists 1 and 2 are independent, so
-// one launch runs both levels (mid_tail_kernel) and their few long cells overlap. Splitting the
-// sizes keeps the register count of the common level low and the few long lists off the
-// private-memory path.
-template <typename TV, typename TC, bool GRAD, bool DG, int LEVEL>
-__device__ __forceinline__ void mid_level(const StepArgs& A, unsigned lblock, unsigned per)
-{
-    constexpr int K = LEVEL < 2 ? 8 : 12;
-    const unsigned n = A.work_count[LEVEL];
-    const uint32_t* list = A.work_list + LEVEL * A.ncells;
-    const unsigned stride = per * kWideBlock;
-    for (unsigned base = lblock * kWideBlock; base < n; base += stride) {
-        const unsigned i = base + threadIdx.x;
-        const bool valid = i < n;
-        CellList<K, TC, GRAD> L;
-        bool empty = false, bad_volume = false;
-#pragma unroll
-        for (int t = 0; t < K; ++t) { L.keep[t] = false; L.eid[t] = 0u; L.phi[t] = 0.0; }
-        L.emax = 0.0;
-        L.mmax = 0.0;
-        if (valid) {
-            const int64_t c = list[i];
-            const int r = gather_cell<K, TV, TC, GRAD>(A, c, L);
-            int dest = -1;  // work list the cell moves on to
-            if (r == kCellWide) {
-                if (LEVEL == 0) {
-                    switch (L.ne) {
-                    case 2: compute_cell<2, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    case 3: compute_cell<3, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    case 4: compute_cell<4, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    case 5: compute_cell<5, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    case 6: compute_cell<6, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    default: dest = 1; break;
-                    }
-                } else if (LEVEL == 1) {
-                    switch (L.ne) {
-                    case 7: compute_cell<7, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    case 8: compute_cell<8, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    default: dest = 3; break;
-                    }
-                } else {
-                    switch (L.ne) {
-                    case 9: compute_cell<9, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    case 10: compute_cell<10, true, K, TC, GRAD, DG>(A, L, empty, c); break;
-                    default: dest = 3; break;
-                    }
-                }
-            } else if (r == kCellDeferred) {
-                dest = LEVEL == 0 ? 2 : 3;  // more entries than this level's capacity
-            }
-            if (dest >= 0) {
-#pragma unroll
-                for (int t = 0; t < K; ++t) L.keep[t] = false;
-                const unsigned slot = atomicAdd(&A.work_count[dest], 1u);
-                A.work_list[dest * A.ncells + slot] = static_cast<uint32_t>(c);
-            } else if (!store_cell<K, TV, TC, GRAD>(A, c, L)) {
-                report_overflow<K, TC, GRAD>(A, c, L);
-            }
-            if (empty) atomicOr(&A.status[kStatusEmpty], 1);
-        }
-        note_maxima(A.obs, L.emax, L.mmax);
-#pragma unroll
-        for (int t = 0; t < K; ++t) wave_volume_add<true>(L.keep[t], L.eid[t], L.phi[t], A.vol_acc, bad_volume);
-        if (bad_volume) atomicOr(&A.status[kStatusVolumeRange], 1);
-    }
-}
-
-// gridDim.x / ndom blocks per domain, each domain's list walked grid-stride by its blocks. The
-// plain variants run at 3 wavefronts per SIMD (168 VGPRs, no spill; level 0 at 256^3: 0.60 ms vs
-// 0.71 ms at the unconstrained 219 VGPRs and 2 wavefronts).
-template <typename TV, typename TC, bool GRAD, bool DG, int LEVEL>
-__global__ __launch_bounds__(kWideBlock, (GRAD || DG) ? 1 : 3) void mid_kernel(const StepArgs* __restrict__ batch, int32_t ndom)
-{
-    const unsigned per = gridDim.x / static_cast<unsigned>(ndom);
-    const unsigned dom = blockIdx.x / per, lblock = blockIdx.x - dom * per;
-    mid_level<TV, TC, GRAD, DG, LEVEL>(batch[dom], lblock, per);
-}
-
-// Levels 1 and 2 in one launch: the first half of each domain's blocks walks list 1, the second
-// half list 2.
-template <typename TV, typename TC, bool GRAD, bool DG>
-__global__ __launch_bounds__(kWideBlock) void mid_tail_kernel(const StepArgs* __restrict__ batch, int32_t ndom)
-{
-    const unsigned per = gridDim.x / static_cast<unsigned>(ndom);
-    const unsigned dom = blockIdx.x / per, lblock = blockIdx.x - dom * per, half = per / 2;
-    if (lblock < half) mid_level<TV, TC, GRAD, DG, 1>(batch[dom], lblock, half);
-    else mid_level<TV, TC, GRAD, DG, 2>(batch[dom], lblock - half, per - half);
-}
-
-// Cells whose merged list is longer than 8 entries (up to 16, held in private memory).
-template <typename TV, typename TC, bool GRAD, bool DG>
-__global__ __launch_bounds__(kWideBlock) void wide_kernel(const StepArgs* __restrict__ batch, int32_t ndom)
-{
-    constexpr int K = kWideSlots;
-    const unsigned per = gridDim.x / static_cast<unsigned>(ndom);
-    const unsigned dom = blockIdx.x / per, lblock = blockIdx.x - dom * per;
-    const StepArgs& A = batch[dom];
-    const unsigned n = A.work_count[3];
-    const unsigned stride = per * kWideBlock;
-    for (unsigned base = lblock * kWideBlock; base < n; base += stride) {
-        const unsigned i = base + threadIdx.x;
-        const bool valid = i < n;
-        CellList<K, TC, GRAD> L;
-        bool empty = false, bad_volume = false;
-        for (int t = 0; t < K; ++t) { L.keep[t] = false; L.eid[t] = 0u; L.phi[t] = 0.0; }
-        L.emax = 0.0;
-        L.mmax = 0.0;
-        if (valid) {
-            const int64_t c = A.work_list[3 * A.ncells + i];
-            const int r = gather_cell<K, TV, TC, GRAD>(A, c, L);
-            if (r == kCellWide) compute_cell<K, false, K, TC, GRAD, DG>(A, L, empty, c);
-            if (r == kCellDeferred || !store_cell<K, TV, TC, GRAD>(A, c, L)) report_overflow<K, TC, GRAD>(A, c, L);
-            if (empty) atomicOr(&A.status[kStatusEmpty], 1);
-        }
-        note_maxima(A.obs, L.emax, L.mmax);
-        for (int t = 0; t < K; ++t) wave_volume_add<true>(L.keep[t], L.eid[t], L.phi[t], A.vol_acc, bad_volume);
-        if (bad_volume) atomicOr(&A.status[kStatusVolumeRange], 1);
     }
 }
 

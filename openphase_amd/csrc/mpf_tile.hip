@@ -18,7 +18,7 @@
 //
 // Cells the tile cannot hold - a neighbourhood with a list of more than three entries or a grain
 // that did not fit the 32 local ids, more than four merged entries, fewer than two - go to the
-// deferred-cell work list of the existing kernels, which handle any list.
+// deferred-cell work list, whose kernel handles any list.
 //
 // Grain volumes (PhaseField::CalculateGrainsVolume, src/PhaseField.cpp:812-951) accumulate per
 // local id in LDS as exact 128-bit fixed-point integers (entries of exactly 1 as counts) and go to
@@ -148,7 +148,7 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
     __shared__ unsigned long long s_acc[kLocal][kCopies][kLimbs];
     __shared__ uint16_t s_list[kBlock];
     __shared__ uint32_t s_nwide[kTileWaves];
-    // cells of a plane for the deferred-cell kernels, by plane parity: appended in LDS, moved to
+    // cells of a plane for the deferred-cell kernel, by plane parity: appended in LDS, moved to
     // the global work list by wavefront 0 after the plane (one global atomic per plane)
     // entries: tile-local cell index (y * TZ + z) | work list << 8
     __shared__ uint16_t s_defer[2][kBlock];
@@ -403,7 +403,7 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
             const bool go = tid < nwide && ne <= K && ne >= 2;
             if (tid < nwide && !go) {
                 // the deferred-cell lists by merged length: 5-6 (and fewer than 2) entries, 7-8, 9 and
-                // more (levels 0, 1 and 2 of the deferred-cell kernels; lists 1 and 2 run after list 0)
+                // more
                 const int dest = ne <= 6 ? 0 : (ne <= 8 ? 1 : 2);
                 s_defer[par][atomicAdd(&s_ndefer[par], 1)] = static_cast<uint16_t>(local | (dest << 8));
             }

@@ -1,0 +1,82 @@
+"""The deferred-cell kernel on every list length it takes: random lists drawn from a small pool of
+grains give merged lists of up to the pool's size (2 to 16), against the CPU oracle."""
+import numpy as np
+import pytest
+
+from openphase_amd import _capi
+from openphase_amd.engine import Engine, StepConfig
+from openphase_amd.microstructure import Lists, random_rotations
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _random_lists(shape, pool, longest, seed):
+    """Cells of 1 to `longest` entries in random order with values summing to 1; a third are bulk."""
+    rng = np.random.default_rng(seed)
+    n = int(np.prod(shape))
+    count = np.where(rng.random(n) < 1 / 3, 1, rng.integers(1, longest + 1, n)).astype(np.int32)
+    index = np.concatenate([rng.permutation(pool)[:c] for c in count]).astype(np.int32)
+    value = np.concatenate([rng.dirichlet(np.ones(c)) for c in count])
+    return Lists(shape, count, index, value)
+
+
+def _config(model, dims, precision=0):
+    kw = dict(slots=16 if precision == 0 else 15, precision=precision, nucleus_volume_factor=1e-3)
+    if model != "iso":
+        kw.update(nphases=2, sigma=np.array([[0.24, 0.3], [0.3, 0.2]]), mu=np.array([[4e-9, 3e-9], [3e-9, 4e-9]]))
+    if model == "tj":
+        kw.update(tj_model=_capi.MPF_TJ_VALUE, tj_energy=0.1)
+    if model == "cubic":
+        kw.update(energy_model=np.full((2, 2), _capi.MPF_ENERGY_CUBIC, np.int32), epsilon=np.full((2, 2), 0.05),
+                  dg_mode=np.array([[0, 1], [1, 0]], np.int32), dg_value=np.array([[0.0, 1e5], [-1e5, 0.0]]))
+    return StepConfig(*dims, **kw)
+
+
+def _step(make, cfg, lists, pool, dt):
+    _, rot = random_rotations(pool, seed=3)
+    e = make(cfg)
+    e.set_grains(np.arange(pool, dtype=np.int32) % cfg.nphases, rot)
+    e.upload(lists)
+    e.finalize_initialization()
+    e.step(dt, 1)
+    out = e.download(), e.limiter_warnings()
+    e.close()
+    return out
+
+
+def _dense(lists, pool):
+    out = np.zeros((lists.ncells, pool))
+    out[np.repeat(np.arange(lists.ncells), lists.count), lists.index] = lists.value
+    return out
+
+
+@pytest.mark.parametrize("model", ["iso", "two", "tj", "cubic"])
+@pytest.mark.parametrize("dims,pool,longest", [((9, 7, 0), 2, 2), ((9, 7, 0), 7, 3), ((7, 6, 5), 5, 5), ((7, 6, 5), 8, 8),
+                                               ((7, 6, 5), 9, 4), ((5, 6, 7), 16, 9)])
+def test_lists_of_every_length(model, dims, pool, longest):
+    cfg = _config(model, dims)
+    lists = _random_lists(cfg.shape, pool, longest, seed=11 * pool + longest)
+    dt = 0.5 * cfg.max_time_step()
+    print(f"{model} {dims} pool {pool} longest {longest}", flush=True)
+    got, warn = _step(Engine, cfg, lists, pool, dt)
+    exp, warn_exp = _step(O.Oracle, cfg, lists, pool, dt)
+    assert np.array_equal(got.count, exp.count) and np.array_equal(got.index, exp.index)
+    if model == "cubic":
+        # the pair energy's fourth power and tanh differ in the last bit (1e-12 bounds a step's values)
+        assert np.abs(got.value - exp.value).max() <= 1e-12
+    else:
+        assert np.array_equal(got.value, exp.value)
+        assert warn == warn_exp
+
+
+@pytest.mark.parametrize("pool,longest", [(3, 3), (8, 5), (15, 9)])
+def test_single_precision_lists(pool, longest):
+    cfg = _config("two", (7, 6, 5), precision=1)
+    lists = _random_lists(cfg.shape, pool, longest, seed=5 * pool + longest)
+    dt = 0.5 * cfg.max_time_step()
+    print(f"fp32 pool {pool} longest {longest}", flush=True)
+    got, _ = _step(Engine, cfg, lists, pool, dt)
+    exp, _ = _step(O.Oracle, _config("two", (7, 6, 5)), lists, pool, dt)
+    # one step in FP32: increments of order 1 with 24-bit terms that cancel to a few per cent
+    assert np.abs(_dense(got, pool) - _dense(exp, pool)).max() <= 1e-5
