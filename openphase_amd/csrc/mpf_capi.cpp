@@ -43,6 +43,16 @@ template <typename T> void h2d(hipError_t& e, T* dst, const T* src, size_t n)
 
 }  // namespace
 
+// Averaging sphere of a context: offsets (3 each), their distance weights, and the staged tile.
+struct mpf_sphere {
+    std::vector<int32_t> off, tile_off;
+    std::vector<double> w;
+    int tile[3] = {0, 0, 0}, reach[3] = {0, 0, 0};
+    int32_t* d_off = nullptr;
+    int32_t* d_tile_off = nullptr;
+    double* d_w = nullptr;
+};
+
 struct mpf_ctx {
     mpf_grid grid{};
     int nx = 1, ny = 1, nz = 1, dnx = 0, dny = 0, dnz = 0, active = 0;
@@ -63,24 +73,18 @@ struct mpf_ctx {
     bool dg_avg = false;
     int avg_range = 0, avg_weights = 0;
     double avg_threshold = 0.0;
-    std::vector<int32_t> avg_off;    // sphere offsets (3 each) and their distance weights
-    std::vector<double> avg_off_w;
+    mpf_sphere avg_sphere;
     double* d_avg_tmp = nullptr;
     double* d_avg = nullptr;
-    int32_t* d_avg_off = nullptr;
-    double* d_avg_off_w = nullptr;
     // interface regularization (InterfaceRegularization): raw, tmp and averaged curvature per pair
     // of own entries, and the averaging sphere
     bool reg = false, reg_active = false, reg_average = true;
     double curvature_factor = 1.0, reg_threshold = 0.0;
     int reg_range = 0;
-    std::vector<int32_t> reg_off;
-    std::vector<double> reg_off_w;
+    mpf_sphere reg_sphere;
     double* d_curv_raw = nullptr;
     double* d_curv_tmp = nullptr;
     double* d_curv = nullptr;
-    int32_t* d_reg_off = nullptr;
-    double* d_reg_off_w = nullptr;
     // per-step terms (mpf_set_step_terms): the driving force acts / is averaged in the next steps
     bool dg_on = true, avg_on = true;
     int32_t* d_dgmode_off = nullptr;  // all-zero mode table: no pair takes the driving force
@@ -358,15 +362,24 @@ mpf_status sync_args(mpf_ctx* c, double dt, hipStream_t stream)
     return c->hip(e, "argument upload");
 }
 
-mpf::AvgArgs avg_args(const mpf_ctx* c, const mpf::StepArgs& s)
+mpf::SphereArgs sphere_args(const mpf_sphere& p, const mpf::StepArgs& s)
 {
-    mpf::AvgArgs a{};
+    mpf::SphereArgs a{};
     a.s = s;
+    a.off = p.d_off;
+    a.off_w = p.d_w;
+    a.noff = static_cast<int32_t>(p.w.size());
+    a.tx = p.tile[0]; a.ty = p.tile[1]; a.tz = p.tile[2];
+    a.rx = p.reach[0]; a.ry = p.reach[1]; a.rz = p.reach[2];
+    a.tile_off = p.d_tile_off;
+    return a;
+}
+
+mpf::SphereArgs avg_args(const mpf_ctx* c, const mpf::StepArgs& s)
+{
+    mpf::SphereArgs a = sphere_args(c->avg_sphere, s);
     a.tmp = c->d_avg_tmp;
     a.avg = c->d_avg;
-    a.off = c->d_avg_off;
-    a.off_w = c->d_avg_off_w;
-    a.noff = static_cast<int32_t>(c->avg_off_w.size());
     a.weights = c->avg_weights;
     a.threshold = c->avg_threshold;
     return a;
@@ -376,13 +389,11 @@ mpf::CurvArgs curv_args(const mpf_ctx* c, const mpf::StepArgs& s)
 {
     mpf::CurvArgs a{};
     a.s = s;
-    a.raw = c->d_curv_raw;
-    a.tmp = c->d_curv_tmp;
-    a.avg = c->d_curv;
-    a.off = c->d_reg_off;
-    a.off_w = c->d_reg_off_w;
-    a.noff = static_cast<int32_t>(c->reg_off_w.size());
-    a.threshold = std::sqrt(c->reg_threshold * (1.0 - c->reg_threshold));
+    a.sphere = sphere_args(c->reg_sphere, s);
+    a.sphere.raw = c->d_curv_raw;
+    a.sphere.tmp = c->d_curv_tmp;
+    a.sphere.avg = c->d_curv;
+    a.sphere.threshold = std::sqrt(c->reg_threshold * (1.0 - c->reg_threshold));
     a.factor = c->curvature_factor - c->regularization;
     a.prefactor2 = c->grid.iwidth * c->grid.dx / kPi;
     a.grad = c->grad ? 1 : 0;
@@ -398,7 +409,7 @@ mpf_status launch_step_part(mpf_ctx* c, hipStream_t stream)
     }
     if (c->reg_active && c->reg_average) {
         // the curvature only enters through its average: unaveraged, its merge weight is 0
-        mpf_status st = c->hip(static_cast<hipError_t>(mpf::launch_curvature(curv_args(c, c->h_args[c->cur]), true, stream)),
+        mpf_status st = c->hip(static_cast<hipError_t>(mpf::launch_curvature(curv_args(c, c->h_args[c->cur]), stream)),
                                "interface regularization kernels");
         if (st) return st;
     }
@@ -424,6 +435,60 @@ mpf_status enqueue_step(mpf_ctx* c, double dt, hipStream_t stream)
     if (!st) st = launch_rest_part(c, stream);
     if (!st) c->cur = 1 - c->cur;
     return st;
+}
+
+// The sphere of radius `range`: the loop bounds and distance weights of CollectAverage /
+// DistributeAverage (src/DrivingForce.cpp:295-324, src/InterfaceRegularization.cpp:198-213), and the
+// tile the averaging kernels stage with it: 8 x 8 x 8 cells in 3D (4 x 8 x 8 where that lets a second
+// block onto a CU), 16 x 32 in 2D, 256 in 1D; none when that does not fit LDS.
+void make_sphere(const mpf_ctx* c, int range, mpf_sphere* p)
+{
+    const int n[3] = {c->nx, c->ny, c->nz}, d[3] = {c->dnx, c->dny, c->dnz};
+    int r[3];
+    for (int q = 0; q < 3; ++q) r[q] = std::min(range, n[q] - 1) * d[q];
+    for (int ii = -r[0]; ii <= r[0]; ii++)
+        for (int jj = -r[1]; jj <= r[1]; jj++)
+            for (int kk = -r[2]; kk <= r[2]; kk++) {
+                const double wd = range - std::sqrt(static_cast<double>(ii * ii + jj * jj + kk * kk));
+                if (!(wd > 0.0)) continue;
+                p->off.insert(p->off.end(), {ii, jj, kk});
+                p->w.push_back(wd);
+            }
+    for (size_t t = 0; t < p->off.size(); ++t) p->reach[t % 3] = std::max(p->reach[t % 3], std::abs(p->off[t]));
+    const int edge = c->active == 3 ? 8 : (c->active == 2 ? 16 : 256);
+    int last = -1;
+    for (int q = 0; q < 3; ++q) {
+        p->tile[q] = d[q] ? std::min(edge, n[q]) : 1;
+        if (d[q]) last = q;
+    }
+    if (c->active == 2) p->tile[last] = std::min(32, n[last]);
+    auto box = [&](int q) { return p->tile[q] + 2 * p->reach[q]; };
+    auto bytes = [&]() { return static_cast<int64_t>(box(0)) * box(1) * (box(2) * mpf::kSphereCellBytes + 4); };
+    if (c->active == 3 && bytes() > 78 * 1024) p->tile[0] = std::min(4, n[0]);
+    if (p->w.size() > mpf::kSphereOffsets || bytes() > mpf::kSphereLds || box(2) > mpf::kSphereCells) {
+        p->tile[0] = p->tile[1] = p->tile[2] = 0;
+        return;
+    }
+    for (size_t t = 0; t < p->off.size(); t += 3)
+        p->tile_off.push_back((p->off[t] * box(1) + p->off[t + 1]) * box(2) + p->off[t + 2]);
+}
+
+mpf_status upload_sphere(mpf_ctx* c, mpf_sphere* p)
+{
+    if (c->hip(dalloc(&p->d_off, p->off.size()), "averaging sphere") ||
+        c->hip(dalloc(&p->d_tile_off, p->tile_off.size()), "averaging sphere") ||
+        c->hip(dalloc(&p->d_w, p->w.size()), "averaging sphere"))
+        return MPF_ERR_NOMEM;
+    hipError_t e = p->tile[0] ? static_cast<hipError_t>(mpf::sphere_lds_limit()) : hipSuccess;
+    h2d(e, p->d_off, p->off.data(), p->off.size());
+    h2d(e, p->d_tile_off, p->tile_off.data(), p->tile_off.size());
+    h2d(e, p->d_w, p->w.data(), p->w.size());
+    return c->hip(e, "averaging sphere");
+}
+
+void free_sphere(mpf_sphere* p)
+{
+    dfree(p->d_off); dfree(p->d_tile_off); dfree(p->d_w);
 }
 
 mpf_status read_status(mpf_ctx* c)
@@ -521,17 +586,7 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
         if ((c->dnx && c->nx < c->reg_range) || (c->dny && c->ny < c->reg_range) || (c->dnz && c->nz < c->reg_range))
             return bail(MPF_ERR_UNSUPPORTED, "interface regularization needs every active axis >= Range cells");
         // CollectAverageSR / DistributeAverageSR loop bounds and distance weights (:198-213)
-        const int xr = std::min(c->reg_range, c->nx - 1) * c->dnx;
-        const int yr = std::min(c->reg_range, c->ny - 1) * c->dny;
-        const int zr = std::min(c->reg_range, c->nz - 1) * c->dnz;
-        for (int ii = -xr; ii <= xr; ii++)
-            for (int jj = -yr; jj <= yr; jj++)
-                for (int kk = -zr; kk <= zr; kk++) {
-                    const double wd = c->reg_range - std::sqrt(static_cast<double>(ii * ii + jj * jj + kk * kk));
-                    if (!(wd > 0.0)) continue;
-                    c->reg_off.insert(c->reg_off.end(), {ii, jj, kk});
-                    c->reg_off_w.push_back(wd);
-                }
+        make_sphere(c, c->reg_range, &c->reg_sphere);
     }
 
     const double eta = grid->iwidth * grid->dx;
@@ -570,17 +625,7 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
         if ((c->dnx && c->nx < c->avg_range) || (c->dny && c->ny < c->avg_range) || (c->dnz && c->nz < c->avg_range))
             return bail(MPF_ERR_UNSUPPORTED, "driving-force averaging needs every active axis >= Range cells");
         // CollectAverage / DistributeAverage loop bounds and distance weights (src/DrivingForce.cpp:295-324)
-        const int xr = std::min(c->avg_range, c->nx - 1) * c->dnx;
-        const int yr = std::min(c->avg_range, c->ny - 1) * c->dny;
-        const int zr = std::min(c->avg_range, c->nz - 1) * c->dnz;
-        for (int ii = -xr; ii <= xr; ii++)
-            for (int jj = -yr; jj <= yr; jj++)
-                for (int kk = -zr; kk <= zr; kk++) {
-                    const double wd = c->avg_range - std::sqrt(static_cast<double>(ii * ii + jj * jj + kk * kk));
-                    if (!(wd > 0.0)) continue;
-                    c->avg_off.insert(c->avg_off.end(), {ii, jj, kk});
-                    c->avg_off_w.push_back(wd);
-                }
+        make_sphere(c, c->avg_range, &c->avg_sphere);
     }
 
     // Stencil weights by number of non-zero offset components: Laplacian / dx^2, gradient / dx
@@ -624,17 +669,15 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
         const size_t pairs = static_cast<size_t>(c->slots) * (c->slots - 1) / 2;
         if (c->hip(dalloc(&c->d_curv_raw, pairs * N), "regularization arrays") ||
             c->hip(dalloc(&c->d_curv_tmp, pairs * N), "regularization arrays") ||
-            c->hip(dalloc(&c->d_curv, pairs * N), "regularization arrays") ||
-            c->hip(dalloc(&c->d_reg_off, c->reg_off.size()), "regularization arrays") ||
-            c->hip(dalloc(&c->d_reg_off_w, c->reg_off_w.size()), "regularization arrays"))
+            c->hip(dalloc(&c->d_curv, pairs * N), "regularization arrays"))
             return bail(MPF_ERR_NOMEM, c->err.c_str());
+        if ((s = upload_sphere(c, &c->reg_sphere))) return bail(s, c->err.c_str());
     }
     if (c->dg_avg) {
         const size_t pairs = static_cast<size_t>(c->slots) * (c->slots - 1) / 2;
-        if (c->hip(dalloc(&c->d_avg_tmp, pairs * N), "averaging arrays") || c->hip(dalloc(&c->d_avg, pairs * N), "averaging arrays") ||
-            c->hip(dalloc(&c->d_avg_off, c->avg_off.size()), "averaging arrays") ||
-            c->hip(dalloc(&c->d_avg_off_w, c->avg_off_w.size()), "averaging arrays"))
+        if (c->hip(dalloc(&c->d_avg_tmp, pairs * N), "averaging arrays") || c->hip(dalloc(&c->d_avg, pairs * N), "averaging arrays"))
             return bail(MPF_ERR_NOMEM, c->err.c_str());
+        if ((s = upload_sphere(c, &c->avg_sphere))) return bail(s, c->err.c_str());
     }
     hipError_t e = hipSuccess;
     h2d(e, c->d_sigma, c->sigma.data(), np2);
@@ -647,14 +690,6 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
     h2d(e, c->d_dgmode_off, no_mode.data(), np2);
     h2d(e, c->d_dgval, c->dgval.data(), np2);
     h2d(e, c->d_dgallowed, c->dgallowed.data(), np2);
-    if (c->reg_active && c->reg_average) {
-        h2d(e, c->d_reg_off, c->reg_off.data(), c->reg_off.size());
-        h2d(e, c->d_reg_off_w, c->reg_off_w.data(), c->reg_off_w.size());
-    }
-    if (c->dg_avg) {
-        h2d(e, c->d_avg_off, c->avg_off.data(), c->avg_off.size());
-        h2d(e, c->d_avg_off_w, c->avg_off_w.data(), c->avg_off_w.size());
-    }
     const int32_t zeros[mpf::kStatusWords] = {0, 0, 0, 0};
     const unsigned long long none = ~0ull, zero = 0ull;
     h2d(e, c->d_status, zeros, mpf::kStatusWords);
@@ -1155,8 +1190,8 @@ void mpf_destroy(mpf_ctx* c)
     dfree(c->d_energy); dfree(c->d_fractions);
     dfree(c->d_status); dfree(c->d_first_overflow); dfree(c->d_warnings);
     dfree(c->d_work_list); dfree(c->d_work_count); dfree(c->d_stats); dfree(c->d_obs);
-    dfree(c->d_avg_tmp); dfree(c->d_avg); dfree(c->d_avg_off); dfree(c->d_avg_off_w);
-    dfree(c->d_curv_raw); dfree(c->d_curv_tmp); dfree(c->d_curv); dfree(c->d_reg_off); dfree(c->d_reg_off_w);
+    dfree(c->d_avg_tmp); dfree(c->d_avg); free_sphere(&c->avg_sphere);
+    dfree(c->d_curv_raw); dfree(c->d_curv_tmp); dfree(c->d_curv); free_sphere(&c->reg_sphere);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
 }

@@ -140,10 +140,11 @@ int launch_tile(const StepArgs& a, unsigned blocks, bool fp32, bool full, bool u
 int launch_tile_batch(const StepArgs* args, const uint32_t* first, int ndom, unsigned blocks, bool fp32, bool full,
                       bool uni, void* stream);
 
-// Driving-force averaging (mpf_dgavg.hip): CollectAverage into `tmp`, DistributeAverage into
-// `avg` (= s.dg_avg), both [pairs][ncells] with pair a < b of the own entries at b(b-1)/2 + a.
-struct AvgArgs {
+// Averaging over the interface (mpf_dgavg.hip): CollectAverage into `tmp`, DistributeAverage into
+// `avg`, both [pairs][ncells] with pair a < b of the own entries at b(b-1)/2 + a.
+struct SphereArgs {
     StepArgs s;                  // state of the step start (cnt_in, id_in, val_in), grains, tables
+    double* raw;                 // raw curvature (null: the driving force, raw = phase-pair value)
     double* tmp;
     double* avg;
     // offsets of the averaging sphere in the reference's loop order (x outer, z inner; each axis
@@ -152,29 +153,34 @@ struct AvgArgs {
     const int32_t* off;
     const double* off_w;
     int32_t noff;
-    int32_t weights;             // 0 PHASEFIELDS, 1 RANGE, 2 COUNTER
+    int32_t weights;             // driving force: 0 PHASEFIELDS, 1 RANGE, 2 COUNTER
     double threshold;            // sqrt(PhiThreshold * (1 - PhiThreshold))
+    // staged tile: its cells, the sphere's reach per axis, and the offsets as distances in the
+    // staged box; tx = 0: a wavefront at a time instead
+    int32_t tx, ty, tz;
+    int32_t rx, ry, rz;
+    const int32_t* tile_off;
 };
 constexpr int kAvgBlock = 256;
-int launch_dg_average(const AvgArgs& a, bool fp32, void* stream);
+constexpr int kSphereOffsets = 256;      // offsets up to which tiles are staged
+constexpr int kSphereCells = 512;        // cells of a staged tile at most
+constexpr int kSphereCellBytes = 25;     // LDS per staged cell
+constexpr int kSphereLds = 150 * 1024;   // LDS of a staged tile at most
+int sphere_lds_limit();                  // to be called before the first launch with tx > 0
+// Averaged driving force (avg = s.dg_avg).
+int launch_dg_average(const SphereArgs& a, bool fp32, void* stream);
 
 // Interface regularization (mpf_dgavg.hip), FP64 state: the raw curvature of every own pair of
-// the interface cells into `raw`, then InterfaceRegularization's CollectAverage into `tmp` and
-// DistributeAverage into `avg` (= s.curv), all [pairs][ncells] like AvgArgs.
+// the interface cells into sphere.raw, then InterfaceRegularization's CollectAverage and
+// DistributeAverage (sphere.avg = s.curv).
 struct CurvArgs {
     StepArgs s;                  // state of the step start, grains, tables
-    double* raw;
-    double* tmp;
-    double* avg;
-    const int32_t* off;          // sphere offsets within Range (3 ints each), x outer, z inner
-    const double* off_w;         // Range - |offset|
-    int32_t noff;
-    double threshold;            // sqrt(PhiThreshold * (1 - PhiThreshold))
+    SphereArgs sphere;
     double factor;               // CurvatureFactor - RegularizationFactor
     double prefactor2;           // Eta / Pi
     int32_t grad;                // orientation-dependent energies present (gradients needed)
 };
-int launch_curvature(const CurvArgs& a, bool average, void* stream);
+int launch_curvature(const CurvArgs& a, void* stream);
 
 // Host-side launchers (mpf_kernels.hip); return a hipError_t value. The step, deferred-cell and
 // grain kernels run over one or several domains of the same kernel variant in one launch: `args`

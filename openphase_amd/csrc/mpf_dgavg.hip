@@ -7,10 +7,9 @@
 // raw by its weighted mean over the sphere of radius Range (tmp); DistributeAverage (:381-478)
 // averages tmp again (average), which MergePhaseFieldIncrementsSR then limits and merges. Here no
 // Force storage exists: an entry's raw value and weight follow from the node's own list (grains,
-// values) and the phase-pair table, so both passes read the step-start state directly. A
-// wavefront takes one interface cell at a time and, per own pair, the sphere's offsets x outer,
-// z inner (the reference's loop order; every sum is formed in that order); a neighbour contributes
-// when it is an interface cell holding both grains. tmp and the averaged value are stored per pair of own
+// values) and the phase-pair table, so both passes read the step-start state directly, the sphere's
+// offsets x outer, z inner (the reference's loop order; every sum is formed in that order); a
+// neighbour contributes when it is an interface cell holding both grains. tmp and the averaged value are stored per pair of own
 // entries (a < b at plane b(b-1)/2 + a) for the step kernel, which reads them in place of the
 // phase-pair value.
 //
@@ -22,6 +21,7 @@
 
 #include "mpf_device.h"
 #include "mpf_lists.h"
+#include "mpf_step_ops.h"
 
 namespace mpf {
 
@@ -84,14 +84,14 @@ __device__ __forceinline__ double lane_value(double x, int l)
 constexpr int kAvgCells = 64;                 // cells per block
 constexpr int kAvgWaves = kAvgBlock / 64;     // wavefronts per block
 
-// SECOND = false: CollectAverage into tmp; true: DistributeAverage into avg. A block takes 64
-// consecutive cells and compacts their interface cells in LDS; its wavefronts take them in turn.
+// SECOND = false: CollectAverage into tmp; true: DistributeAverage into avg, for spheres too large
+// for staged tiles (sphere_tile_kernel). A block takes 64 consecutive cells and compacts their interface cells in LDS; its wavefronts take them in turn.
 // For one cell and pair the 64 lanes evaluate 64 sphere offsets at once (the neighbour's weight
 // and raw or tmp value), then every lane adds the terms of the lanes that count in lane order,
 // chunk after chunk: the sums are formed in the reference's offset order, and a wavefront waits
 // on a few memory round trips per chunk instead of one chain per offset.
 template <typename TV, bool SECOND>
-__global__ __launch_bounds__(kAvgBlock) void dg_average_kernel(const AvgArgs P)
+__global__ __launch_bounds__(kAvgBlock) void dg_average_kernel(const SphereArgs P)
 {
     __shared__ uint16_t s_list[kAvgCells];
     __shared__ int s_count;
@@ -249,7 +249,7 @@ __device__ __forceinline__ bool raw_cell(const CurvArgs& P, int64_t c)
             }
             double kappa = d * P.prefactor2 * scale * norm_1 / sqrt(L.phi[a] * L.phi[b]);
             kappa *= P.factor;
-            P.raw[static_cast<int64_t>(pair_plane(a, b)) * N + c] = kappa;
+            P.sphere.raw[static_cast<int64_t>(pair_plane(a, b)) * N + c] = kappa;
         }
     return true;
 }
@@ -291,7 +291,7 @@ __global__ __launch_bounds__(kCurvBlock) void curvature_raw_kernel(const CurvArg
 // the entries below those bounds keep 0. Lane-parallel over the sphere, summed in offset order as
 // dg_average_kernel does.
 template <bool SECOND>
-__global__ __launch_bounds__(kAvgBlock) void curvature_average_kernel(const CurvArgs P)
+__global__ __launch_bounds__(kAvgBlock) void curvature_average_kernel(const SphereArgs P)
 {
     __shared__ uint16_t s_list[kAvgCells];
     __shared__ int s_count;
@@ -364,33 +364,277 @@ __global__ __launch_bounds__(kAvgBlock) void curvature_average_kernel(const Curv
     }
 }
 
+// ---- both averagings on staged tiles
+
+constexpr int kSphereBlock = kSphereCells;     // threads of a block
+
+struct __align__(16) PairCell {
+    double w, v;   // weight and value of the staged pair at a cell (absent: 0, 0)
+};
+static_assert(sizeof(PairCell) + sizeof(unsigned long long) + 1 == kSphereCellBytes, "LDS of a staged cell");
+
+// Grain of entry t of cell c, `rec` holding its first four.
+__device__ __forceinline__ uint32_t listed_grain(const StepArgs& A, unsigned long long rec, int64_t c, int t)
+{
+    return t < 4 ? static_cast<uint32_t>(rec >> (16 * t)) & 0xFFFFu : A.id_in[static_cast<int64_t>(t) * A.ncells + c];
+}
+
+// SECOND = false: CollectAverage into tmp; true: DistributeAverage into avg, of the driving force or
+// (CURV) of the curvature: the sums of dg_average_kernel and curvature_average_kernel, on tiles.
+//
+// A block stages the lists' grains of its tile plus the sphere's reach in LDS, and then takes the
+// pairs of grains its cells hold one after another (ascending): the pair's weight and value at every
+// staged cell go to LDS (0 where it is absent: such a term never counts), and every lane sums the
+// sphere around one of the tile's cells that hold the pair, x outer, z inner as the reference does,
+// from LDS at fixed distances. Values are staged in the orientation (lower grain, higher grain); a
+// sum in the other orientation is its exact negative. So a pair is looked up once per staged cell
+// and not once per cell and offset, and a wavefront holds 64 cells' sums instead of one. What
+// bounds it is the chain of the sums (an LDS read and about 11 instructions per offset) of the
+// pairs that only a few of the tile's cells hold. Collect / Distribute of the curvature, 93
+// offsets, 160^3: 7.66 / 5.70 ms a wavefront at a time, 1.68 / 1.54 ms on tiles. The driving force
+// with 485 offsets, 96^3: 0.64 / 1.88 ms a wavefront at a time, 0.61 / 2.70 ms on tiles: so tiles
+// are staged up to kSphereOffsets offsets.
+template <typename TV, bool CURV, bool SECOND>
+__global__ __launch_bounds__(kSphereBlock) void sphere_tile_kernel(const SphereArgs P)
+{
+    extern __shared__ __align__(16) unsigned char s_dyn[];
+    __shared__ uint32_t s_item[kSphereBlock];
+    __shared__ uint32_t s_key, s_items;
+    const StepArgs& A = P.s;
+    const int64_t N = A.ncells;
+    const int NP = A.nphases;
+    const int tid = static_cast<int>(threadIdx.x);
+    const int HY = P.ty + 2 * P.ry, HZ = P.tz + 2 * P.rz, H = (P.tx + 2 * P.rx) * HY * HZ;
+    PairCell* s_pair = reinterpret_cast<PairCell*>(s_dyn);
+    unsigned long long* s_rec = reinterpret_cast<unsigned long long*>(s_pair + H);
+    uint32_t* s_row = reinterpret_cast<uint32_t*>(s_rec + H);   // first cell of a staged row of z
+    uint8_t* s_code = reinterpret_cast<uint8_t*>(s_row + H / HZ);
+    const unsigned b = A.xcd_order ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const unsigned ntz = static_cast<unsigned>((A.nz + P.tz - 1) / P.tz), nty = static_cast<unsigned>((A.ny + P.ty - 1) / P.ty);
+    const int z0 = static_cast<int>(b % ntz) * P.tz, y0 = static_cast<int>((b / ntz) % nty) * P.ty,
+              x0 = static_cast<int>(b / (ntz * nty)) * P.tx;
+    for (int r = tid; r < H / HZ; r += kSphereBlock) {
+        const int x = (x0 - P.rx + r / HY + A.nx) % A.nx, y = (y0 - P.ry + r % HY + A.ny) % A.ny;
+        s_row[r] = static_cast<uint32_t>((x * A.ny + y) * A.nz);
+    }
+    __syncthreads();
+    // a thread stages the cells of one z in every step-th row
+    const int step = kSphereBlock / HZ, row0 = tid / HZ < step ? tid / HZ : H / HZ, hz = tid % HZ;
+    const uint32_t zg = static_cast<uint32_t>((z0 - P.rz + hz + A.nz) % A.nz);
+    for (int r = row0; r < H / HZ; r += step) {
+        const int64_t c = s_row[r] + zg;
+        const uint8_t code = A.cnt_in[c];
+        const int n = ListCode<TV>::count(code);
+        unsigned long long rec = 0ull;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            if (s < n) rec |= static_cast<unsigned long long>(A.id_in[static_cast<int64_t>(s) * N + c]) << (16 * s);
+        s_rec[r * HZ + hz] = rec;
+        s_code[r * HZ + hz] = code;
+    }
+    // the thread's own cell
+    const int lx = tid / (P.ty * P.tz), ly = (tid / P.tz) % P.ty, lz = tid % P.tz;
+    const bool own = lx < P.tx && x0 + lx < A.nx && y0 + ly < A.ny && z0 + lz < A.nz;
+    const int hown = own ? ((lx + P.rx) * HY + ly + P.ry) * HZ + lz + P.rz : 0;
+    const int64_t cown = own ? (static_cast<int64_t>(x0 + lx) * A.ny + y0 + ly) * A.nz + z0 + lz : 0;
+    __syncthreads();
+    const int nown = own ? ListCode<TV>::count(s_code[hown]) : 0;
+    const unsigned long long rown = s_rec[hown];
+    // key of the own pair (d, e): its grains, lower first, ~0 for a driving force's pair of phases
+    // without one (no Force entry); those of the first four entries are kept
+    auto own_key = [&](int d, int e) -> uint32_t {
+        const uint32_t gd = listed_grain(A, rown, cown, d), ge = listed_grain(A, rown, cown, e);
+        if (!CURV && A.dg_mode[A.gphase[gd] * NP + A.gphase[ge]] != 1) return ~0u;
+        return min(gd, ge) << 16 | max(gd, ge);
+    };
+    uint32_t key4[6];
+#pragma unroll
+    for (int e = 1; e < 4; ++e)
+#pragma unroll
+        for (int d = 0; d < e; ++d) key4[pair_plane(d, e)] = e < nown ? own_key(d, e) : ~0u;
+    uint32_t last = 0u;  // keys (lower grain << 16 | higher grain) are not 0
+    while (true) {
+        if (tid == 0) {
+            s_key = ~0u;
+            s_items = 0u;
+        }
+        __syncthreads();
+        uint32_t next = ~0u;
+#pragma unroll
+        for (int p = 0; p < 6; ++p) next = key4[p] > last ? min(next, key4[p]) : next;
+        for (int e = 4; e < nown; ++e)
+            for (int d = 0; d < e; ++d) {
+                const uint32_t k = own_key(d, e);
+                next = k > last ? min(next, k) : next;
+            }
+#pragma unroll
+        for (int k = 32; k >= 1; k >>= 1) next = min(next, static_cast<uint32_t>(__shfl_xor(static_cast<int>(next), k)));
+        if ((tid & 63) == 0 && next != ~0u) atomicMin(&s_key, next);
+        __syncthreads();
+        const uint32_t key = s_key;
+        if (key == ~0u) break;
+        last = key;
+        const uint32_t glo = key >> 16, ghi = key & 0xFFFFu;
+        const int plo = A.gphase[glo], phi = A.gphase[ghi];
+        double cut = P.threshold;
+        if (!CURV) cut *= A.gvr[glo] * A.gvr[ghi];
+        // the tile's cells that hold the pair; those whose weight is too small keep a fresh entry's 0
+        int plane = -1, ia = 0, ib = 0;
+#pragma unroll
+        for (int e = 1; e < 4; ++e)
+#pragma unroll
+            for (int d = 0; d < e; ++d)
+                if (key4[pair_plane(d, e)] == key) { plane = pair_plane(d, e); ia = d; ib = e; }
+        for (int e = 4; e < nown && plane < 0; ++e)
+            for (int d = 0; d < e; ++d)
+                if (own_key(d, e) == key) { plane = pair_plane(d, e); ia = d; ib = e; }
+        if (plane >= 0) {
+            const uint8_t code = s_code[hown];
+            const double w = sqrt(entry_value<TV>(A, cown, code, ia) * entry_value<TV>(A, cown, code, ib));
+            const bool back = listed_grain(A, rown, cown, ia) != glo;
+            if (CURV ? (SECOND ? w > DBL_EPSILON : w > P.threshold) : (SECOND ? w > 0.0 : w > cut))
+                s_item[atomicAdd(&s_items, 1u)] = static_cast<uint32_t>(tid) | static_cast<uint32_t>(plane) << 16 | (back ? 1u << 31 : 0u);
+            else
+                (SECOND ? P.avg : P.tmp)[static_cast<int64_t>(plane) * N + cown] = 0.0;
+        }
+        __syncthreads();
+        const uint32_t items = s_items;
+        if (items) {
+            const double* __restrict__ src = SECOND ? P.tmp : P.raw;
+            const double fwd = CURV ? 0.0 : A.dg_value[plo * NP + phi], rev = CURV ? 0.0 : -A.dg_value[phi * NP + plo];
+            for (int r = row0; r < H / HZ; r += step) {
+                const int h = r * HZ + hz;
+                const uint8_t code = s_code[h];
+                const int n = ListCode<TV>::count(code);
+                const unsigned long long rec = s_rec[h];
+                PairCell p{0.0, 0.0};
+                if (n > 1) {
+                    int ja = -1, jb = -1;
+#pragma unroll
+                    for (int s = 0; s < 4; ++s) {
+                        const uint32_t g = static_cast<uint32_t>(rec >> (16 * s)) & 0xFFFFu;
+                        ja = s < n && g == glo ? s : ja;
+                        jb = s < n && g == ghi ? s : jb;
+                    }
+                    const int64_t c = s_row[r] + zg;
+                    if (n > 4 && (ja < 0 || jb < 0)) {
+                        for (int s = 4; s < n; ++s) {
+                            const uint32_t g = A.id_in[static_cast<int64_t>(s) * N + c];
+                            ja = g == glo ? s : ja;
+                            jb = g == ghi ? s : jb;
+                        }
+                    }
+                    if (ja >= 0 && jb >= 0) {
+                        if (SECOND || CURV) p.v = src[static_cast<int64_t>(pair_plane(min(ja, jb), max(ja, jb))) * N + c];
+                        p.w = sqrt(entry_value<TV>(A, c, code, ja) * entry_value<TV>(A, c, code, jb));
+                        if (SECOND || CURV) p.v = ja < jb ? p.v : -p.v;
+                        else p.v = ja < jb ? fwd : rev;
+                    }
+                }
+                s_pair[h] = p;
+            }
+        }
+        __syncthreads();
+        for (uint32_t i = static_cast<uint32_t>(tid); i < items; i += kSphereBlock) {
+            const int t0 = static_cast<int>(s_item[i] & 0xFFFFu);
+            const int plane = static_cast<int>((s_item[i] >> 16) & 0x7FFFu);
+            const bool back = (s_item[i] >> 31) != 0u;
+            const int cx = t0 / (P.ty * P.tz), cy = (t0 / P.tz) % P.ty, cz = t0 % P.tz;
+            const int64_t here = static_cast<int64_t>(plane) * N + (static_cast<int64_t>(x0 + cx) * A.ny + y0 + cy) * A.nz + z0 + cz;
+            const PairCell* at = s_pair + ((cx + P.rx) * HY + cy + P.ry) * HZ + cz + P.rz;
+            double value = 0.0, sum = 0.0;
+            int counter = 0;
+#pragma unroll 8
+            for (int t = 0; t < P.noff; ++t) {
+                const PairCell p = at[P.tile_off[t]];
+                // terms that do not count add +0, which leaves the sums as they are (never -0)
+                if (CURV && SECOND) {
+                    const bool ok = p.w > P.threshold;
+                    value += ok ? p.v : 0.0;
+                    counter += ok ? 1 : 0;
+                } else {
+                    const double wt = CURV ? p.w * P.off_w[t] : (P.weights == 0 ? p.w : (P.weights == 1 ? P.off_w[t] : 1.0));
+                    const bool ok = CURV ? wt > DBL_EPSILON : (SECOND ? p.w > cut : p.w > 0.0);
+                    value += ok ? wt * p.v : 0.0;
+                    sum += ok ? wt : 0.0;
+                }
+            }
+            if (back) value = -value;
+            double result;
+            if (CURV) {
+                if (SECOND) result = counter != 0 ? value / static_cast<double>(counter) : P.tmp[here];
+                else result = sum > DBL_EPSILON ? value / sum : 0.0;
+            } else {
+                // COUNTER weights are 1: their sum is the count
+                if (sum > 0.0) result = value / sum;
+                else result = SECOND ? P.tmp[here] : A.dg_value[back ? phi * NP + plo : plo * NP + phi];
+            }
+            (SECOND ? P.avg : P.tmp)[here] = result;
+        }
+    }
+}
+
 }  // namespace
 
-int launch_curvature(const CurvArgs& a, bool average, void* stream)
+// LDS of a staged tile: pair field, grains and count byte per cell, first cell per row.
+static size_t sphere_lds(const SphereArgs& a)
+{
+    const size_t rows = static_cast<size_t>(a.tx + 2 * a.rx) * (a.ty + 2 * a.ry);
+    return rows * ((a.tz + 2 * a.rz) * kSphereCellBytes + sizeof(uint32_t));
+}
+
+template <typename TV, bool CURV>
+static void launch_sphere(const SphereArgs& a, hipStream_t s)
+{
+    if (a.tx) {
+        const size_t lds = sphere_lds(a);
+        const int64_t blocks = static_cast<int64_t>((a.s.nx + a.tx - 1) / a.tx) * ((a.s.ny + a.ty - 1) / a.ty) * ((a.s.nz + a.tz - 1) / a.tz);
+        const dim3 grid(static_cast<unsigned>(blocks));
+        hipLaunchKernelGGL((sphere_tile_kernel<TV, CURV, false>), grid, dim3(kSphereBlock), lds, s, a);
+        hipLaunchKernelGGL((sphere_tile_kernel<TV, CURV, true>), grid, dim3(kSphereBlock), lds, s, a);
+    } else {
+        const dim3 grid(static_cast<unsigned>((a.s.ncells + kAvgCells - 1) / kAvgCells));
+        if constexpr (CURV) {
+            hipLaunchKernelGGL((curvature_average_kernel<false>), grid, dim3(kAvgBlock), 0, s, a);
+            hipLaunchKernelGGL((curvature_average_kernel<true>), grid, dim3(kAvgBlock), 0, s, a);
+        } else {
+            hipLaunchKernelGGL((dg_average_kernel<TV, false>), grid, dim3(kAvgBlock), 0, s, a);
+            hipLaunchKernelGGL((dg_average_kernel<TV, true>), grid, dim3(kAvgBlock), 0, s, a);
+        }
+    }
+}
+
+int sphere_lds_limit()
+{
+    // more than 64 KiB of dynamic LDS has to be asked for, once per kernel
+    const void* kernels[] = {reinterpret_cast<const void*>(&sphere_tile_kernel<double, true, false>),
+                             reinterpret_cast<const void*>(&sphere_tile_kernel<double, true, true>),
+                             reinterpret_cast<const void*>(&sphere_tile_kernel<double, false, false>),
+                             reinterpret_cast<const void*>(&sphere_tile_kernel<double, false, true>),
+                             reinterpret_cast<const void*>(&sphere_tile_kernel<float, false, false>),
+                             reinterpret_cast<const void*>(&sphere_tile_kernel<float, false, true>)};
+    for (const void* k : kernels) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kSphereLds);
+        if (e != hipSuccess) return static_cast<int>(e);
+    }
+    return 0;
+}
+
+int launch_curvature(const CurvArgs& a, void* stream)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 raw_grid(static_cast<unsigned>((a.s.ncells + kRawCells - 1) / kRawCells));
     if (a.grad) hipLaunchKernelGGL((curvature_raw_kernel<true>), raw_grid, dim3(kCurvBlock), 0, s, a);
     else hipLaunchKernelGGL((curvature_raw_kernel<false>), raw_grid, dim3(kCurvBlock), 0, s, a);
-    if (average) {
-        const dim3 grid(static_cast<unsigned>((a.s.ncells + kAvgCells - 1) / kAvgCells));
-        hipLaunchKernelGGL((curvature_average_kernel<false>), grid, dim3(kAvgBlock), 0, s, a);
-        hipLaunchKernelGGL((curvature_average_kernel<true>), grid, dim3(kAvgBlock), 0, s, a);
-    }
+    launch_sphere<double, true>(a.sphere, s);
     return static_cast<int>(hipGetLastError());
 }
 
-int launch_dg_average(const AvgArgs& a, bool fp32, void* stream)
+int launch_dg_average(const SphereArgs& a, bool fp32, void* stream)
 {
-    const dim3 grid(static_cast<unsigned>((a.s.ncells + kAvgCells - 1) / kAvgCells));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (fp32) {
-        hipLaunchKernelGGL((dg_average_kernel<float, false>), grid, dim3(kAvgBlock), 0, s, a);
-        hipLaunchKernelGGL((dg_average_kernel<float, true>), grid, dim3(kAvgBlock), 0, s, a);
-    } else {
-        hipLaunchKernelGGL((dg_average_kernel<double, false>), grid, dim3(kAvgBlock), 0, s, a);
-        hipLaunchKernelGGL((dg_average_kernel<double, true>), grid, dim3(kAvgBlock), 0, s, a);
-    }
+    if (fp32) launch_sphere<float, false>(a, s);
+    else launch_sphere<double, false>(a, s);
     return static_cast<int>(hipGetLastError());
 }
 

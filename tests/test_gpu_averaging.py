@@ -1,0 +1,43 @@
+"""Averaging over the interface (driving force, curvature) on staged tiles and, for spheres that do not
+fit LDS, per wavefront: ragged grids, every reach, lists of up to six entries, against the oracle."""
+import numpy as np
+import pytest
+
+from openphase_amd.engine import Engine, StepConfig
+import oracle as O
+from test_gpu_deferred import _random_lists, _step
+
+pytestmark = pytest.mark.gpu
+
+# a step's values: the limiter's tanh differs in the last bit between device and host
+TOL = 1e-12
+
+
+def _compare(cfg, pool, longest, seed):
+    lists = _random_lists(cfg.shape, pool, longest, seed)
+    dt = 0.3 * cfg.max_time_step()
+    got, _ = _step(Engine, cfg, lists, pool, dt)
+    exp, _ = _step(O.Oracle, cfg, lists, pool, dt)
+    assert np.array_equal(got.count, exp.count) and np.array_equal(got.index, exp.index)
+    assert np.abs(got.value - exp.value).max() <= TOL
+
+
+# Range 9 in 3D does not fit LDS, Range 6 leaves one block per CU, Range 5 takes the smaller tile
+@pytest.mark.parametrize("dims,reach", [((33, 19, 0), 3), ((12, 50, 0), 5), ((9, 8, 10), 3), ((13, 9, 10), 5), ((12, 9, 11), 6),
+                                        ((9, 10, 11), 9), ((40, 0, 0), 4)])
+@pytest.mark.parametrize("weights", [0, 1, 2])
+def test_driving_force(dims, reach, weights):
+    cfg = StepConfig(*dims, nphases=2, sigma=np.full((2, 2), 0.24), mu=np.full((2, 2), 4e-9), slots=16,
+                     nucleus_volume_factor=1e-3, dg_mode=np.array([[0, 1], [1, 0]], np.int32),
+                     dg_value=np.array([[0.0, 1e5], [-7e4, 0.0]]), dg_average=True, dg_range=reach, dg_threshold=0.05,
+                     dg_weights=weights)
+    print(f"driving force {dims} range {reach} weights {weights}", flush=True)
+    _compare(cfg, 7, 6, seed=17 * reach + weights)
+
+
+@pytest.mark.parametrize("dims,reach", [((33, 19, 0), 2), ((12, 50, 0), 6), ((9, 8, 10), 3), ((13, 9, 10), 4), ((9, 10, 11), 9)])
+def test_curvature(dims, reach):
+    cfg = StepConfig(*dims, slots=16, nucleus_volume_factor=1e-3, regularization=True, regularization_factor=1.5,
+                     curvature_factor=0.7, reg_range=reach, reg_threshold=0.02)
+    print(f"curvature {dims} range {reach}", flush=True)
+    _compare(cfg, 7, 6, seed=23 * reach)
