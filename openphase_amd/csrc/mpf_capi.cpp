@@ -1041,6 +1041,10 @@ mpf_status mpf_interface_energy(mpf_ctx* c, int32_t ip_state, double* sum)
     const double eta = c->grid.iwidth * c->grid.dx;
     a.eta = eta;
     a.pref = eta * eta / (kPi * kPi);
+    a.full = c->grad ? 1 : 0;
+    for (int p = 0; p < c->nphases; ++p)
+        for (int q = 0; q < p; ++q)
+            if (c->sigma[static_cast<size_t>(p) * c->nphases + q] != c->sigma[static_cast<size_t>(q) * c->nphases + p]) a.full = 1;
     a.partial = c->d_energy;
     a.status = c->d_status + 3;
     const int32_t zero = 0;

@@ -4,11 +4,9 @@
 //
 // A group of lanes takes one cell: 16 lanes, four cells per wavefront. What bounds such a cell is
 // latency - one chain of dependent loads, list searches and divisions - so its work is spread over
-// the group instead of run by one lane: every lane fetches the lists of its two neighbours of the
-// 3^d box (two round trips for the whole cell), the merged list (PhaseField::CalculateDerivativesSR,
-// src/PhaseField.cpp:566-615) is formed with one ballot per appended grain, and then lane t holds
-// entry t (Laplacian, limiter bounds, merge, finalize) and the pair increments are dealt to the
-// lanes. Sums that the reference forms in an order are formed by one lane in that order (stencil
+// the group instead of run by one lane: the merged list is formed by the group (group_gather), lane t
+// holds entry t (Laplacian, limiter bounds, merge, finalize) and the pair increments are dealt to
+// the lanes. Sums that the reference forms in an order are formed by one lane in that order (stencil
 // order, list order, pair order), so every value equals the one-lane form bit for bit.
 //
 // Lists are held in LDS with run-time lengths, so one kernel takes every length: a cell of more
@@ -24,6 +22,7 @@
 #include <stdint.h>
 
 #include "mpf_device.h"
+#include "mpf_group.h"
 #include "mpf_lists.h"
 #include "mpf_step_ops.h"
 
@@ -31,28 +30,7 @@ namespace mpf {
 
 namespace {
 
-constexpr int kGroupLanes = 16;  // lanes per cell
-constexpr int kGroupCap = 8;     // merged entries a group has room for
 constexpr int kVolSlots = 32;    // grains of the wavefront's volume table
-
-// One cell's list and tables in LDS.
-template <typename TC, bool GRAD, int CAP> struct GroupMem {
-    union {
-        TC a[CAP][27];                 // value of merged entry t at box position k
-        struct {
-            double psi[CAP][CAP + 1];  // increment of (t, u), antisymmetric
-            TC sig[CAP][CAP + 1];      // interface energy of (t, u)
-        } p;
-    };
-    TC gr[GRAD ? CAP : 1][3];
-    double phi[CAP];
-    TC lap[CAP];
-    TC ev[CAP];                        // value in the stencil arithmetic
-    double lim1[CAP], lim2[CAP];
-    double vr[CAP];
-    int ph[CAP];
-    uint32_t eid[CAP];
-};
 
 struct VolTable {
     int32_t key[kVolSlots];
@@ -83,22 +61,6 @@ __device__ __forceinline__ void table_volume_add(VolTable& V, uint32_t g, double
         if (l[i]) atomicAdd(&dst[i], l[i]);
 }
 
-// Largest n over the wavefront's groups of G lanes (n uniform within a group), in a scalar.
-template <int G> __device__ __forceinline__ int wave_max(int n)
-{
-#pragma unroll
-    for (int k = G; k < 64; k <<= 1) n = max(n, __shfl_xor(n, k));
-    return __builtin_amdgcn_readfirstlane(n);
-}
-
-// The ballot's bits of this lane's group, shifted to bit 0.
-template <int G> __device__ __forceinline__ unsigned long long group_bits(unsigned long long m)
-{
-    if (G == 64) return m;
-    const int lane = static_cast<int>(threadIdx.x) & 63;
-    return (m >> (lane & ~(G - 1))) & ((1ull << (G & 63)) - 1ull);
-}
-
 // The step of cell c (when `run`) by the G lanes of this lane's group. Returns true (uniform in
 // the group) when the cell needs more than CAP entries: nothing was written then. All lanes of the
 // wavefront call it together; loops run to the longest list of its groups.
@@ -107,175 +69,17 @@ __device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t 
                                            bool count_long, const uint16_t* pairs, VolTable& V, double& emax,
                                            double& mmax, bool& bad)
 {
-    constexpr int NK = (27 + G - 1) / G;   // neighbours per lane
-    constexpr int RQ = CAP;                // entries of a neighbour
     constexpr bool IMPL = ListCode<TV>::kImplicit;
     const int lane = static_cast<int>(threadIdx.x) & 63, l = lane & (G - 1);
     const int64_t N = A.ncells;
-    const uint32_t N32 = static_cast<uint32_t>(N);
-    const uint32_t cc = static_cast<uint32_t>(run ? c : 0);
-
-    // ---- the box: positions l, l + G of stencil order
-    const int NY = A.ny, NZ = A.nz;
-    const int z0 = static_cast<int>(cc % static_cast<uint32_t>(NZ));
-    const int y0 = static_cast<int>((cc / static_cast<uint32_t>(NZ)) % static_cast<uint32_t>(NY));
-    const int x0 = static_cast<int>(cc / (static_cast<uint32_t>(NY) * static_cast<uint32_t>(NZ)));
-    const __amdgpu_buffer_rsrc_t rc = plane_rsrc(A.cnt_in, N32);
-    uint32_t nb[NK];
-    bool act[NK];
-    uint8_t code[NK];
-#pragma unroll
-    for (int j = 0; j < NK; ++j) {
-        const int k = l + j * G;
-        const int ii = k / 9 - 1, jj = (k / 3) % 3 - 1, kk = k % 3 - 1;
-        act[j] = run && k < 27 && (ii == 0 || A.dnx) && (jj == 0 || A.dny) && (kk == 0 || A.dnz);
-        nb[j] = static_cast<uint32_t>((wrap1(x0 + (act[j] ? ii : 0), A.nx) * NY + wrap1(y0 + (act[j] ? jj : 0), NY)) * NZ +
-                                      wrap1(z0 + (act[j] ? kk : 0), NZ));
-        code[j] = buffer_load<uint8_t>(rc, act[j] ? nb[j] : kNoLoad);
-    }
-    const uint8_t code0 = buffer_load<uint8_t>(rc, run ? cc : kNoLoad);
-    const int n0 = ListCode<TV>::count(code0), imp0 = ListCode<TV>::implicit(code0);
-    int m[NK], mtop = n0;
-    bool multi = false;
-#pragma unroll
-    for (int j = 0; j < NK; ++j) {
-        m[j] = ListCode<TV>::count(code[j]);
-        multi = multi || m[j] > 1;
-        mtop = max(mtop, m[j]);
-    }
-    // a neighbour's list longer than this form holds, or the own one
-    const bool wide = group_bits<G>(__ballot(multi)) != 0ull;
-    bool over = group_bits<G>(__ballot(mtop > CAP)) != 0ull;
-#pragma unroll
-    for (int k = 1; k < 64; k <<= 1) mtop = max(mtop, __shfl_xor(mtop, k));
-    const int qtop = min(__builtin_amdgcn_readfirstlane(mtop), RQ);
-
-    // ---- lists of the lane's neighbours, and entry l of the own list
-    uint32_t g[NK][RQ];
-    TV v[NK][RQ];
-    uint32_t left[NK];   // entries not in the merged list yet (bit q)
-#pragma unroll
-    for (int j = 0; j < NK; ++j) left[j] = 0u;
-#pragma unroll
-    for (int q = 0; q < RQ; ++q) {
-        if (q >= 2 && q >= qtop) {
-#pragma unroll
-            for (int j = 0; j < NK; ++j) { g[j][q] = 0u; v[j][q] = TV(0); }
-            continue;
-        }
-        // slot 0 of the cell in place of a slot it does not use: no branch between the loads
-#pragma unroll
-        for (int j = 0; j < NK; ++j) {
-            const int64_t at = (q < m[j] ? static_cast<int64_t>(q) * N : 0) + nb[j];
-            g[j][q] = A.id_in[at];
-            v[j][q] = load_val<TV>(A.val_in, at);
-        }
-    }
-    double phi = 0.0;
-    uint32_t eid = 0u;
-    if (l < n0 && l < CAP) {
-        eid = A.id_in[static_cast<int64_t>(l) * N + cc];
-        if (!(IMPL && l == imp0)) phi = static_cast<double>(load_val<TV>(A.val_in, static_cast<int64_t>(l) * N + cc));
-    }
-#pragma unroll
-    for (int j = 0; j < NK; ++j)
-#pragma unroll
-        for (int q = 0; q < RQ; ++q) {
-            // a lone implicit entry (FP32) has no stored value: it is 1
-            if (IMPL && q == 0 && m[j] == 1 && ListCode<TV>::implicit(code[j]) == 0) v[j][q] = TV(1);
-            if (q < m[j] && v[j][q] != TV(0)) left[j] |= 1u << q;
-        }
-    if (l < CAP) { M.phi[l] = phi; M.eid[l] = eid; }
-    __syncthreads();
-    if (IMPL) {
-        double others = 0.0;
-        for (int t = 0; t < CAP; ++t)
-            if (t < n0 && t != imp0) others += M.phi[t];
-        __syncthreads();
-        if (l < n0 && l == imp0) {
-            phi = 1.0 - others;
-            M.phi[l] = phi;
-        }
-    }
-
-    // ---- merged list: the own entries, then grains new to the box in stencil order. Row t of
-    // M.a: the value of entry t at every box position
-    int ne = over ? 0 : n0;
-    if (!wide || over) {
-#pragma unroll
-        for (int j = 0; j < NK; ++j) left[j] = 0u;
-    }
-    auto row = [&](int t, uint32_t gid, bool on) {
-#pragma unroll
-        for (int j = 0; j < NK; ++j) {
-            TC a = TC(0);
-#pragma unroll
-            for (int q = 0; q < RQ; ++q)
-                if (((left[j] >> q) & 1u) && g[j][q] == gid && on) {
-                    a = static_cast<TC>(v[j][q]);
-                    left[j] &= ~(1u << q);
-                }
-            const int k = l + j * G;
-            if (on && k < 27) M.a[t][k] = a;
-        }
-    };
-    const int own_top = wave_max<G>(wide ? ne : 0);
-    for (int t = 0; t < own_top; ++t) row(t, M.eid[t], wide && t < ne);
-    while (true) {
-        uint32_t cand = 0u;
-        unsigned long long who = 0ull;
-#pragma unroll
-        for (int j = NK - 1; j >= 0; --j) {
-            const unsigned long long b = group_bits<G>(__ballot(left[j] != 0u));
-            if (b) {
-                who = b;
-                const int q = __ffs(static_cast<int>(left[j])) - 1;
-                cand = 0u;
-#pragma unroll
-                for (int r = 0; r < RQ; ++r) cand = r == q ? g[j][r] : cand;
-            }
-        }
-        if (!__any(who != 0ull)) break;
-        const int leader = who ? __ffsll(static_cast<long long>(who)) - 1 : 0;
-        const uint32_t gid = static_cast<uint32_t>(__shfl(static_cast<int>(cand), (lane & ~(G - 1)) + leader));
-        bool on = who != 0ull;
-        if (on && ne >= CAP) {
-            over = true;
-            on = false;
-#pragma unroll
-            for (int j = 0; j < NK; ++j) left[j] = 0u;
-        }
-        row(ne, gid, on);
-        if (on) {
-            if (l == ne) eid = gid;
-            ++ne;
-        }
-    }
-    if (l < CAP) M.eid[l] = eid;
-    const bool go = run && !over;            // the cell's result is written by this call
-    const bool work = go && wide;
+    const GroupList<TC> L = group_gather<TV, TC, GRAD, G, CAP>(A, run, c, M);
+    const int n0 = L.n0, ne = L.ne;
+    const uint32_t eid = L.eid;
+    double phi = L.phi;
+    const bool go = run && !L.over;          // the cell's result is written by this call
+    const bool work = go && L.wide;
     if (work && ne > 6 && count_long && l == 0) atomicAdd(&A.work_count[3], 1u);
     const int top = wave_max<G>(work ? ne : 0);
-    __syncthreads();
-
-    // ---- Laplacian (gradient) of entry l, in stencil order
-    TC lap = TC(0), gx = TC(0), gy = TC(0), gz = TC(0);
-    if (work && l < ne) {
-#pragma unroll
-        for (int k = 0; k < 27; ++k) {
-            const int ii = k / 9 - 1, jj = (k / 3) % 3 - 1, kk = k % 3 - 1;
-            const int nz = (ii != 0) + (jj != 0) + (kk != 0);
-            const TC a = M.a[l][k];
-            lap += static_cast<TC>(A.wl[nz]) * a;
-            if (GRAD && k != 13) {
-                const TC w = static_cast<TC>(A.wg[nz]);
-                if (ii) gx = gx + (ii < 0 ? -w : w) * a;
-                if (jj) gy = gy + (jj < 0 ? -w : w) * a;
-                if (kk) gz = gz + (kk < 0 ? -w : w) * a;
-            }
-        }
-    }
-    __syncthreads();  // M.p takes M.a's place
     double vr = 0.0;
     int ph = 0;
     if (work && l < ne) {
@@ -284,11 +88,11 @@ __device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t 
     }
     const TC ev = static_cast<TC>(phi);
     if (l < CAP) {
-        M.lap[l] = lap;
+        M.lap[l] = L.lap;
         M.ev[l] = ev;
         M.ph[l] = ph;
         M.vr[l] = vr;
-        if (GRAD) { M.gr[GRAD ? l : 0][0] = gx; M.gr[GRAD ? l : 0][1] = gy; M.gr[GRAD ? l : 0][2] = gz; }
+        if (GRAD) { M.gr[GRAD ? l : 0][0] = L.gx; M.gr[GRAD ? l : 0][1] = L.gy; M.gr[GRAD ? l : 0][2] = L.gz; }
     }
     __syncthreads();
 
@@ -544,7 +348,7 @@ __device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t 
         }
     }
     if (keep) table_volume_add(V, eid, phi, A.vol_acc, bad);
-    return run && over;
+    return run && L.over;
 }
 
 // One wavefront per block; wavefront i of a domain takes the i-th part of its deferred cells (the
@@ -553,11 +357,8 @@ template <typename TV, typename TC, bool GRAD, bool DG>
 __global__ __launch_bounds__(64) void deferred_kernel(const StepArgs* __restrict__ batch, int32_t ndom)
 {
     constexpr int G = kGroupLanes, C = 64 / G;
-    __shared__ union Arena {
-        GroupMem<TC, GRAD, kGroupCap> cell[C];
-        GroupMem<TC, GRAD, kWideSlots> one;
-    } mem;
-    __shared__ uint16_t pairs[kWideSlots * (kWideSlots - 1) / 2];
+    __shared__ GroupArena<TC, GRAD> mem;
+    __shared__ uint16_t pairs[kPairTable];
     __shared__ VolTable V;
     const unsigned per = gridDim.x / static_cast<unsigned>(ndom);
     const unsigned dom = blockIdx.x / per, part = blockIdx.x - dom * per;
@@ -570,11 +371,7 @@ __global__ __launch_bounds__(64) void deferred_kernel(const StepArgs* __restrict
     const unsigned begin = min(n, part * chunk), end = min(n, begin + chunk);
     if (begin >= end) return;
     const int lane = static_cast<int>(threadIdx.x);
-    for (int p = lane; p < kWideSlots * (kWideSlots - 1) / 2; p += 64) {
-        int b = 1;
-        while (b * (b + 1) / 2 <= p) ++b;
-        pairs[p] = static_cast<uint16_t>((p - b * (b - 1) / 2) | (b << 8));
-    }
+    fill_pairs(pairs);
     if (lane < kVolSlots) V.key[lane] = -1;
     for (int i = lane; i < kVolSlots * kLimbs; i += 64) (&V.acc[0][0])[i] = 0ull;
     __syncthreads();

@@ -213,6 +213,8 @@ struct EnergyArgs {
     const uint8_t* ip_cnt;
     const uint16_t* ip_id;
     const void* ip_val;
+    int32_t full;                // 1: pair energies need the list IP.Set saw (orientation-dependent or
+                                 // asymmetric tables), 0: they follow from the pair's phases
     double eta;                  // interface width
     double pref;                 // Eta^2 / Pi^2
     double* partial;             // energy_blocks(ncells) per-block sums
