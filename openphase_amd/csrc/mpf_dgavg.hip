@@ -20,6 +20,7 @@
 #include <stdint.h>
 
 #include "mpf_device.h"
+#include "mpf_group.h"
 #include "mpf_lists.h"
 #include "mpf_step_ops.h"
 
@@ -178,106 +179,115 @@ __global__ __launch_bounds__(kAvgBlock) void dg_average_kernel(const SphereArgs 
 
 // ---- interface regularization (FP64 state) -------------------------------------------------
 
-constexpr int kCurvBlock = 256;
+constexpr int kRawCells = 256;     // cells per block (one wavefront) of the raw pass
 
 // The curvature DoubleObstacle's regularization overload adds per pair of non-zero entries of a
 // wide-interface cell (src/DoubleObstacle.cpp:702-763): loc_increment (the pair's increment before
 // the mobility, over the neighbour-merged list) * Eta/Pi * scale * norm_1 / sqrt(phi_a phi_b) *
 // (CurvatureFactor - RegularizationFactor). Only own entries are non-zero, so only interface cells
-// (more than one own entry) hold such pairs. The list of up to K merged entries is gathered as the
-// step's deferred path does and kept in registers (loops fully unrolled over K, guarded by the
-// counts); energies per pair from the phase-pair table (GRAD false) or the orientation. Returns
-// false when the cell has more than K merged entries.
-template <int K, bool GRAD>
-__device__ __forceinline__ bool raw_cell(const CurvArgs& P, int64_t c)
+// (more than one own entry) hold such pairs. A group of lanes takes the cell (group_gather), its
+// own pairs dealt to the lanes; energies per pair from the phase-pair table (GRAD false) or the
+// orientation. Returns true when the cell needs more than CAP entries: nothing was written then.
+template <bool GRAD, int G, int CAP>
+__device__ __forceinline__ bool raw_cell(const CurvArgs& P, bool run, int64_t c, GroupMem<double, GRAD, CAP>& M,
+                                         const uint16_t* pairs)
 {
     const StepArgs& A = P.s;
     const int64_t N = A.ncells;
-    CellList<K, double, GRAD> L;
-#pragma unroll
-    for (int t = 0; t < K; ++t) L.eid[t] = 0u;
-    const int r = gather_cell<K, double, double, GRAD>(A, c, L);
-    if (r == kCellDeferred) return false;
-    if (r != kCellWide) return true;
-    const int ne = L.ne, n0 = L.n0, NP = A.nphases;
-    int ph[K];
-    double vr[K];
-    double localn = 0.0;
-#pragma unroll
-    for (int t = 0; t < K; ++t) {
-        ph[t] = 0; vr[t] = 0.0;
-        if (t < ne) { ph[t] = A.gphase[L.eid[t]]; vr[t] = A.gvr[L.eid[t]]; }
+    const int l = static_cast<int>(threadIdx.x) & (G - 1), NP = A.nphases;
+    const GroupList<double> L = group_gather<double, double, GRAD, G, CAP>(A, run, c, M);
+    const bool work = run && !L.over && L.wide;
+    const int ne = work ? L.ne : 0, n0 = work ? L.n0 : 0;
+    if (l < CAP) {
+        M.lap[l] = L.lap;
+        M.phi[l] = L.phi;
+        M.ph[l] = l < ne ? A.gphase[L.eid] : 0;
+        M.vr[l] = l < ne ? A.gvr[L.eid] : 0.0;
+        if (GRAD) { M.gr[GRAD ? l : 0][0] = L.gx; M.gr[GRAD ? l : 0][1] = L.gy; M.gr[GRAD ? l : 0][2] = L.gz; }
     }
+    __syncthreads();
+    double localn = 0.0;
     if (A.consider_nucleus) {
-#pragma unroll
-        for (int t = 0; t < K; ++t) if (t < ne) localn += vr[t];
+        for (int t = 0; t < ne; ++t) localn += M.vr[t];
     } else {
         localn = static_cast<double>(ne);
     }
     const double norm_1 = 1.0 / localn;
     const double Pf = A.prefactor;
     // InterfaceProperties energy of a pair (the lower list position first)
-    auto sigma_of = [&](int x, int y) -> double {
-        const int lo = x < y ? x : y, hi = x < y ? y : x;
-        const int k = ph[lo] * NP + ph[hi];
-        if (!GRAD) return A.sigma[k];
-        return ip_pair_energy<double>(A, k, L.eid[lo], L.eid[hi], L.phi[lo], L.phi[hi], L.gr[GRAD ? lo : 0],
-                                      L.gr[GRAD ? hi : 0]);
-    };
-#pragma unroll
-    for (int b = 1; b < K; ++b)
-#pragma unroll
-        for (int a = 0; a < b; ++a) {
-            if (b >= n0) continue;
-            const double scale = sqrt(vr[a] * vr[b]);
-            const double cf = 0.5 * (1.0 + scale) * Pf;
-            double d = sigma_of(a, b) * ((L.lap[a] + cf * L.phi[a]) - (L.lap[b] + cf * L.phi[b]));
-            if (ne > 2) {
-#pragma unroll
-                for (int g = 0; g < K; ++g) {
-                    if (g == a || g == b || g >= ne) continue;
-                    d += (sigma_of(b, g) - sigma_of(a, g)) * (L.lap[g] + cf * L.phi[g]);
-                    if (A.tj_model == 0) {
-                        if (A.tj_factor != 0.0 || scale < 1.0) {
-                            const double e3 = A.sigma[ph[a] * NP + ph[b]] + A.sigma[ph[b] * NP + ph[g]] + A.sigma[ph[a] * NP + ph[g]];
-                            d += smax(A.tj_factor, (1.0 - scale)) * Pf * e3 * (L.phi[a] * L.phi[g] - L.phi[b] * L.phi[g]);
-                        }
-                    } else if (A.tj_model == 1) {
-                        d += A.tj_energy * Pf * (L.phi[a] * L.phi[g] - L.phi[b] * L.phi[g]);
-                    }
-                }
-            }
-            double kappa = d * P.prefactor2 * scale * norm_1 / sqrt(L.phi[a] * L.phi[b]);
-            kappa *= P.factor;
-            P.sphere.raw[static_cast<int64_t>(pair_plane(a, b)) * N + c] = kappa;
+    for (int p = l; p < ne * (ne - 1) / 2; p += G) {
+        const int a = pairs[p] & 255, b = pairs[p] >> 8;
+        double en;
+        if (GRAD) {
+            double da[3], db[3];
+            for (int d = 0; d < 3; ++d) { da[d] = M.gr[GRAD ? a : 0][d]; db[d] = M.gr[GRAD ? b : 0][d]; }
+            en = ip_pair_energy<double>(A, M.ph[a] * NP + M.ph[b], M.eid[a], M.eid[b], M.phi[a], M.phi[b], da, db);
+        } else {
+            en = A.sigma[M.ph[a] * NP + M.ph[b]];
         }
-    return true;
-}
-
-constexpr int kRawCells = 4 * kCurvBlock;  // cells per block of the raw pass
-
-// A block takes kRawCells consecutive cells, collects its interface cells in LDS (in any order:
-// each cell's result is its own) and gives one to each thread in turn, so no lane idles on bulk
-// cells. Lists of up to 8 merged entries in registers, longer ones (more than 16: the step
-// itself reports the overflow) with 16.
-template <bool GRAD>
-__global__ __launch_bounds__(kCurvBlock) void curvature_raw_kernel(const CurvArgs P)
-{
-    __shared__ uint16_t s_list[kRawCells];
-    __shared__ int s_n;
-    const int tid = static_cast<int>(threadIdx.x);
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * kRawCells;
-    if (tid == 0) s_n = 0;
-    __syncthreads();
-    for (int k = tid; k < kRawCells; k += kCurvBlock) {
-        const int64_t c = base + k;
-        if (c < P.s.ncells && ListCode<double>::count(P.s.cnt_in[c]) >= 2) s_list[atomicAdd(&s_n, 1)] = static_cast<uint16_t>(k);
+        M.p.sig[a][b] = en;
+        M.p.sig[b][a] = en;
     }
     __syncthreads();
-    const int n = s_n;
-    for (int i = tid; i < n; i += kCurvBlock) {
-        const int64_t c = base + s_list[i];
-        if (!raw_cell<8, GRAD>(P, c)) (void)raw_cell<kWideSlots, GRAD>(P, c);
+    for (int p = l; p < n0 * (n0 - 1) / 2; p += G) {
+        const int a = pairs[p] & 255, b = pairs[p] >> 8;
+        const double scale = sqrt(M.vr[a] * M.vr[b]);
+        const double cf = 0.5 * (1.0 + scale) * Pf;
+        double d = M.p.sig[a][b] * ((M.lap[a] + cf * M.phi[a]) - (M.lap[b] + cf * M.phi[b]));
+        for (int g = 0; g < ne; ++g) {
+            if (g == a || g == b) continue;
+            d += (M.p.sig[b][g] - M.p.sig[a][g]) * (M.lap[g] + cf * M.phi[g]);
+            if (A.tj_model == 0) {
+                if (A.tj_factor != 0.0 || scale < 1.0) {
+                    const int pa = M.ph[a], pb = M.ph[b], pg = M.ph[g];
+                    const double e3 = A.sigma[pa * NP + pb] + A.sigma[pb * NP + pg] + A.sigma[pa * NP + pg];
+                    d += smax(A.tj_factor, (1.0 - scale)) * Pf * e3 * (M.phi[a] * M.phi[g] - M.phi[b] * M.phi[g]);
+                }
+            } else if (A.tj_model == 1) {
+                d += A.tj_energy * Pf * (M.phi[a] * M.phi[g] - M.phi[b] * M.phi[g]);
+            }
+        }
+        double kappa = d * P.prefactor2 * scale * norm_1 / sqrt(M.phi[a] * M.phi[b]);
+        kappa *= P.factor;
+        P.sphere.raw[static_cast<int64_t>(p) * N + c] = kappa;
+    }
+    __syncthreads();
+    return run && L.over;
+}
+
+// A wavefront collects the interface cells of its 256 cells in LDS and takes them four at a time
+// (longer lists, up to 16 merged entries, one at a time; more than that the step itself reports as
+// an overflow). What bounds it is the instructions of the list walk; one thread per cell with
+// register lists took 4.0 ms at 160^3 (256 VGPRs and spills, one wavefront per SIMD), now 1.23 ms.
+template <bool GRAD>
+__global__ __launch_bounds__(64) void curvature_raw_kernel(const CurvArgs P)
+{
+    constexpr int G = kGroupLanes, C = 64 / G;
+    __shared__ GroupArena<double, GRAD> mem;
+    __shared__ uint16_t pairs[kPairTable];
+    __shared__ uint16_t s_list[kRawCells];
+    const int lane = static_cast<int>(threadIdx.x);
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kRawCells;
+    fill_pairs(pairs);
+    int n = 0;
+    for (int k = 0; k < kRawCells; k += 64) {
+        const int64_t c = base + k + lane;
+        const bool in = c < P.s.ncells && ListCode<double>::count(P.s.cnt_in[c]) >= 2;
+        const unsigned long long m = __ballot(in);
+        if (in) s_list[n + __popcll(m & ((1ull << lane) - 1ull))] = static_cast<uint16_t>(k + lane);
+        n += __popcll(m);
+    }
+    __syncthreads();
+    for (int i0 = 0; i0 < n; i0 += C) {
+        const int i = i0 + lane / G;
+        const bool run = i < n;
+        const bool big = raw_cell<GRAD, G, kGroupCap>(P, run, base + (run ? s_list[i] : 0), mem.cell[lane / G], pairs);
+        unsigned long long todo = __ballot(big && (lane & (G - 1)) == 0);
+        while (todo) {
+            const int from = __ffsll(static_cast<long long>(todo)) - 1;
+            todo &= todo - 1ull;
+            (void)raw_cell<GRAD, 64, kWideSlots>(P, true, base + s_list[i0 + from / G], mem.one, pairs);
+        }
     }
 }
 
@@ -624,8 +634,8 @@ int launch_curvature(const CurvArgs& a, void* stream)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 raw_grid(static_cast<unsigned>((a.s.ncells + kRawCells - 1) / kRawCells));
-    if (a.grad) hipLaunchKernelGGL((curvature_raw_kernel<true>), raw_grid, dim3(kCurvBlock), 0, s, a);
-    else hipLaunchKernelGGL((curvature_raw_kernel<false>), raw_grid, dim3(kCurvBlock), 0, s, a);
+    if (a.grad) hipLaunchKernelGGL((curvature_raw_kernel<true>), raw_grid, dim3(64), 0, s, a);
+    else hipLaunchKernelGGL((curvature_raw_kernel<false>), raw_grid, dim3(64), 0, s, a);
     launch_sphere<double, true>(a.sphere, s);
     return static_cast<int>(hipGetLastError());
 }
