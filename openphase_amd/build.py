@@ -45,7 +45,7 @@ def build_hip() -> Path:
     # (source, object name, extra defines): the per-cell step kernels build as four variants
     units = [(CSRC / "mpf_kernels.hip", "mpf_kernels", []), (CSRC / "mpf_tile.hip", "mpf_tile", []),
              (CSRC / "mpf_adjoint.hip", "mpf_adjoint", []), (CSRC / "mpf_dgavg.hip", "mpf_dgavg", []),
-             (CSRC / "mpf_energy.hip", "mpf_energy", []),
+             (CSRC / "mpf_energy.hip", "mpf_energy", []), (CSRC / "mpf_pack.hip", "mpf_pack", []),
              (CSRC / "mpf_capi.cpp", "mpf_capi", [])]
     for fp32 in (0, 1):
         for full in (0, 1):

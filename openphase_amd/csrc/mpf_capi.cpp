@@ -143,6 +143,9 @@ struct mpf_ctx {
     size_t energy_cap = 0;
     double* d_fractions = nullptr;        // phase fractions for host downloads
     size_t fractions_cap = 0;
+    int64_t* d_pack_offset = nullptr;     // running sums of the entries (mpf_pack.hip), and the staging
+    unsigned char* d_pack = nullptr;      // buffer of packed lists for host downloads
+    size_t pack_cap = 0;
 
     int xcd_order = 1;               // launch shape, see StepArgs
     int deferred_grid = mpf::kWideGrid;
@@ -895,71 +898,102 @@ mpf_status mpf_synchronize(mpf_ctx* c)
     return read_status(c);
 }
 
+}  // extern "C"
+
+namespace {
+
+// Running sums of the current state's entries by block of cells, on the device.
+mpf_status pack_offsets(mpf_ctx* c)
+{
+    if (!c->d_pack_offset &&
+        c->hip(dalloc(&c->d_pack_offset, static_cast<size_t>(mpf::pack_blocks(c->ncells)) + 1), "list offsets"))
+        return MPF_ERR_NOMEM;
+    return c->hip(static_cast<hipError_t>(mpf::launch_pack_offsets(c->cnt[c->cur], c->ncells, c->fp32, c->d_pack_offset, c->stream)),
+                  "list offset kernels");
+}
+
+// Staging of packed lists: at most 128 MiB, held by the context; smaller parts where that cannot be had.
+constexpr size_t kPackStage = size_t{128} << 20;
+constexpr size_t kPackCellBytes = sizeof(int32_t) + sizeof(int8_t);                 // count, flag
+constexpr size_t kPackEntryBytes = sizeof(int32_t) + sizeof(double);                // index, value
+constexpr size_t kPackLeast = mpf::kPackCells * (kPackCellBytes + mpf::kMaxSlots * kPackEntryBytes) + 1024;  // one block
+
+mpf_status pack_stage(mpf_ctx* c, size_t want)
+{
+    want = std::max(std::min(want, kPackStage), kPackLeast);
+    if (c->pack_cap >= want) return MPF_OK;
+    for (size_t n = want; n >= std::max(kPackLeast, c->pack_cap + 1); n = n > kPackLeast ? std::max(n / 2, kPackLeast) : 0) {
+        unsigned char* p = nullptr;
+        if (dalloc(&p, n) == hipSuccess) {
+            dfree(c->d_pack);
+            c->d_pack = p;
+            c->pack_cap = n;
+            return MPF_OK;
+        }
+        (void)hipGetLastError();
+    }
+    return c->pack_cap >= kPackLeast ? MPF_OK : c->fail(MPF_ERR_NOMEM, "no device memory for the packed lists");
+}
+
+}  // namespace
+
+extern "C" {
+
 mpf_status mpf_total_entries(mpf_ctx* c, int64_t* total)
 {
     if (!c || !total) return MPF_ERR_ARG;
     if (!c->have_state) return c->fail(MPF_ERR_STATE, "no state");
-    std::vector<uint8_t> cnt(static_cast<size_t>(c->ncells));
-    mpf_status s = c->hip(hipMemcpyAsync(cnt.data(), c->cnt[c->cur], cnt.size(), hipMemcpyDeviceToHost, c->stream), "download counts");
+    mpf_status s = pack_offsets(c);
+    if (!s) s = c->hip(hipMemcpyAsync(total, c->d_pack_offset + mpf::pack_blocks(c->ncells), sizeof(*total), hipMemcpyDeviceToHost,
+                                      c->stream), "download counts");
     if (!s) s = c->hip(hipStreamSynchronize(c->stream), "sync");
-    if (s) return s;
-    int64_t t = 0;
-    for (uint8_t v : cnt) t += c->fp32 ? (v & 15) : v;
-    *total = t;
-    return MPF_OK;
+    return s;
 }
 
 mpf_status mpf_download(mpf_ctx* c, int32_t* count, int32_t* index, double* value, int8_t* flag)
 {
     if (!c) return MPF_ERR_ARG;
     if (!c->have_state) return c->fail(MPF_ERR_STATE, "no state");
-    const size_t N = static_cast<size_t>(c->ncells);
-    const int K = c->slots;
-    std::vector<uint8_t> cnt(N);
-    std::vector<uint16_t> ids(N * K);
-    std::vector<double> vd;
-    std::vector<float> vf;
-    if (c->fp32) vf.resize(N * K); else vd.resize(N * K);
-    const int b = c->cur;
-    mpf_status s = c->hip(hipMemcpyAsync(cnt.data(), c->cnt[b], N, hipMemcpyDeviceToHost, c->stream), "download");
-    if (!s) s = c->hip(hipMemcpyAsync(ids.data(), c->id[b], N * K * sizeof(uint16_t), hipMemcpyDeviceToHost, c->stream), "download");
-    if (!s) s = c->hip(hipMemcpyAsync(c->fp32 ? static_cast<void*>(vf.data()) : static_cast<void*>(vd.data()), c->val[b],
-                                      N * K * c->vsize(), hipMemcpyDeviceToHost, c->stream), "download");
-    if (!s) s = c->hip(hipStreamSynchronize(c->stream), "sync");
+    const int64_t N = c->ncells, nb = mpf::pack_blocks(N);
+    mpf_status s = pack_offsets(c);
     if (s) return s;
-    // decode FP32 states: count | (implicit slot << 4); the implicit value is 1 - sum(others)
-    std::vector<uint8_t> n(N);
-    for (size_t i = 0; i < N; ++i) n[i] = c->fp32 ? (cnt[i] & 15) : cnt[i];
-    size_t off = 0;
-    for (size_t i = 0; i < N; ++i) {
-        if (count) count[i] = n[i];
-        const int imp = c->fp32 && (cnt[i] >> 4) != 15 ? (cnt[i] >> 4) : -1;
-        double others = 0.0;
-        for (int q = 0; q < n[i]; ++q)
-            if (q != imp) others += c->fp32 ? static_cast<double>(vf[static_cast<size_t>(q) * N + i]) : vd[static_cast<size_t>(q) * N + i];
-        for (int q = 0; q < n[i]; ++q, ++off) {
-            if (index) index[off] = ids[static_cast<size_t>(q) * N + i];
-            if (!value) continue;
-            if (q == imp) value[off] = 1.0 - others;
-            else value[off] = c->fp32 ? static_cast<double>(vf[static_cast<size_t>(q) * N + i]) : vd[static_cast<size_t>(q) * N + i];
+    std::vector<int64_t> off(static_cast<size_t>(nb) + 1);
+    s = c->hip(hipMemcpyAsync(off.data(), c->d_pack_offset, off.size() * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream), "download");
+    if (!s) s = c->hip(hipStreamSynchronize(c->stream), "sync");
+    if (!s) s = pack_stage(c, static_cast<size_t>(N) * kPackCellBytes + static_cast<size_t>(off[nb]) * kPackEntryBytes + 1024);
+    if (s) return s;
+    const mpf::StepArgs a = step_args(c, 1.0, c->cur);
+    auto up = [](size_t x) { return (x + 255) & ~size_t{255}; };
+    for (int64_t b0 = 0; b0 < nb;) {
+        // as many blocks as the staging buffer holds: values, indices, counts, flags
+        size_t cells = 0, entries = 0;
+        int64_t b1 = b0;
+        while (b1 < nb) {
+            const size_t m = static_cast<size_t>(std::min(N, (b1 + 1) * mpf::kPackCells) - b0 * mpf::kPackCells);
+            const size_t n = static_cast<size_t>(off[b1 + 1] - off[b0]);
+            if (up(n * sizeof(double)) + up(n * sizeof(int32_t)) + up(m * sizeof(int32_t)) + m > c->pack_cap) break;
+            cells = m;
+            entries = n;
+            ++b1;
         }
-    }
-    if (flag) {
-        for (size_t i = 0; i < N; ++i) {
-            if (n[i] > 1) { flag[i] = 2; continue; }
-            const int x = static_cast<int>(i / (static_cast<size_t>(c->ny) * c->nz));
-            const int y = static_cast<int>((i / c->nz) % c->ny);
-            const int z = static_cast<int>(i % c->nz);
-            int8_t f = 0;
-            for (int ii = -c->dnx; ii <= c->dnx && !f; ++ii)
-                for (int jj = -c->dny; jj <= c->dny && !f; ++jj)
-                    for (int kk = -c->dnz; kk <= c->dnz && !f; ++kk) {
-                        const int xx = (x + ii + c->nx) % c->nx, yy = (y + jj + c->ny) % c->ny, zz = (z + kk + c->nz) % c->nz;
-                        const size_t nb = (static_cast<size_t>(xx) * c->ny + yy) * c->nz + zz;
-                        if (n[nb] > 1) f = 1;
-                    }
-            flag[i] = f;
-        }
+        double* d_val = reinterpret_cast<double*>(c->d_pack);
+        int32_t* d_idx = reinterpret_cast<int32_t*>(c->d_pack + up(entries * sizeof(double)));
+        int32_t* d_cnt = reinterpret_cast<int32_t*>(reinterpret_cast<unsigned char*>(d_idx) + up(entries * sizeof(int32_t)));
+        int8_t* d_flag = reinterpret_cast<int8_t*>(reinterpret_cast<unsigned char*>(d_cnt) + up(cells * sizeof(int32_t)));
+        s = c->hip(static_cast<hipError_t>(mpf::launch_pack(a, c->fp32, c->d_pack_offset, b0, b1 - b0, count ? d_cnt : nullptr,
+                                                            flag ? d_flag : nullptr, index ? d_idx : nullptr,
+                                                            value ? d_val : nullptr, c->stream)), "packing kernel");
+        auto get = [&](void* dst, const void* src, size_t bytes) {
+            if (!s && bytes) s = c->hip(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream), "download");
+        };
+        const int64_t c0 = b0 * mpf::kPackCells;
+        if (count) get(count + c0, d_cnt, cells * sizeof(int32_t));
+        if (flag) get(flag + c0, d_flag, cells);
+        if (index) get(index + off[b0], d_idx, entries * sizeof(int32_t));
+        if (value) get(value + off[b0], d_val, entries * sizeof(double));
+        if (!s) s = c->hip(hipStreamSynchronize(c->stream), "sync");
+        if (s) return s;
+        b0 = b1;
     }
     return MPF_OK;
 }
@@ -1191,7 +1225,7 @@ void mpf_destroy(mpf_ctx* c)
     dfree(c->d_args); dfree(c->d_first); dfree(c->d_gargs); dfree(c->d_gfirst);
     dfree(c->d_sigma); dfree(c->d_mu); dfree(c->d_eps); dfree(c->d_maxe);
     dfree(c->d_emodel); dfree(c->d_dgmode); dfree(c->d_dgval); dfree(c->d_dgallowed); dfree(c->d_dgmode_off);
-    dfree(c->d_energy); dfree(c->d_fractions);
+    dfree(c->d_energy); dfree(c->d_pack_offset); dfree(c->d_pack); dfree(c->d_fractions);
     dfree(c->d_status); dfree(c->d_first_overflow); dfree(c->d_warnings);
     dfree(c->d_work_list); dfree(c->d_work_count); dfree(c->d_stats); dfree(c->d_obs);
     dfree(c->d_avg_tmp); dfree(c->d_avg); free_sphere(&c->avg_sphere);

@@ -225,6 +225,15 @@ int64_t energy_blocks(int64_t ncells);
 int launch_energy(const EnergyArgs& a, bool fp32, double* out, void* stream);
 // Per-cell phase fractions of the state (cnt_in, id_in, val_in): out[phase * ncells + cell].
 int launch_fractions(const StepArgs& a, bool fp32, double* out, void* stream);
+
+// The state as concatenated lists (mpf_pack.hip). offset: pack_blocks + 1 running sums of the
+// entries of blocks of kPackCells cells.
+constexpr int kPackCells = 1024;
+int64_t pack_blocks(int64_t ncells);
+int launch_pack_offsets(const uint8_t* cnt, int64_t ncells, bool fp32, int64_t* offset, void* stream);
+// Blocks first .. first + blocks - 1 into device buffers (null: not wanted).
+int launch_pack(const StepArgs& a, bool fp32, const int64_t* offset, int64_t first, int64_t blocks, int32_t* count, int8_t* flag,
+                int32_t* index, double* value, void* stream);
 int launch_grains(const GrainArgs* args, const uint32_t* first, int ndom, unsigned blocks, void* stream);
 int launch_copy(const void* src, void* dst, int64_t bytes, void* stream);
 

@@ -70,6 +70,37 @@ def test_lists_of_every_length(model, dims, pool, longest):
         assert warn == warn_exp
 
 
+@pytest.mark.parametrize("model,precision", [("two", 0), ("cubic", 0), ("iso", 1)])
+@pytest.mark.parametrize("dims,pool,longest", [((9, 7, 0), 4, 3), ((7, 6, 5), 8, 8), ((5, 6, 7), 15, 9)])
+def test_energy_and_flags(model, precision, dims, pool, longest):
+    """The interface energy on lists of every length, with the pairs of the current state and of the
+    one before the step, and the downloaded flags."""
+    cfg = _config(model, dims, precision)
+    lists = _random_lists(cfg.shape, pool, longest, seed=7 * pool + longest)
+    if precision:
+        lists.value[:] = lists.value.astype(np.float32)
+    _, rot = random_rotations(pool, seed=3)
+    print(f"energy {model} precision {precision} {dims} pool {pool}", flush=True)
+    eng, orc = Engine(cfg), O.Oracle(_config(model, dims))
+    for e in (eng, orc):
+        e.set_grains(np.arange(pool, dtype=np.int32) % cfg.nphases, rot)
+        e.upload(lists)
+        e.finalize_initialization()
+        if e is orc:
+            orc.keep_step_start(True)
+        e.step(0.5 * cfg.max_time_step(), 1)
+    # sums of about 10^4 terms of either sign, FP32 states with 24-bit values
+    rel = 1e-11 if precision == 0 else 1e-4
+    for ip in ("current", "previous"):
+        assert eng.interface_energy(ip) == pytest.approx(orc.interface_energy(ip), rel=rel)
+    got, flags = eng.download(with_flags=True)
+    exp, flags_exp = orc.download(with_flags=True)
+    if precision == 0:
+        assert np.array_equal(got.count, exp.count) and np.array_equal(flags, flags_exp)
+    eng.close()
+    orc.close()
+
+
 @pytest.mark.parametrize("pool,longest", [(3, 3), (8, 5), (15, 9)])
 def test_single_precision_lists(pool, longest):
     cfg = _config("two", (7, 6, 5), precision=1)
