@@ -265,7 +265,7 @@ mpf_status mpf_adjoint_step(mpf_ctx* ctx, double dt, const double* lam_next, dou
 /* Launch-shape autotuner (no reference counterpart): times `steps` steps of each candidate on the
  * context's own state (saved and restored around every trial, so the state is unchanged
  * afterwards) and keeps the fastest, in two rounds: (1) the step kernel's tile (grids with two or
- * three active axes) - plane tiles of 64-256 cells (2D: 64 / 128 / 256 along the active plane
+ * three active axes) - plane tiles of 64-256 cells (2D: 16 / 32 / 64 / 128 / 256 along the active plane
  * axis; 3D: 4x64, 8x32, 16x16, 4x32) times 1 / 4 / 16 / the default number of planes per block,
  * and the per-cell kernel; (2) the XCD-contiguous block order of the step kernel on/off times
  * 256 / 1024 / 4096 / 16384 blocks for the deferred-cell kernel. Results do not depend on the
@@ -277,7 +277,8 @@ mpf_status mpf_set_launch_shape(mpf_ctx* ctx, int32_t xcd_order, int32_t deferre
 /* Shape of the LDS-tiled step kernel (no reference counterpart): a block holds a tile_y x tile_z
  * tile of the (y, z) plane (at most 256 cells, its halo plane at most 396 cells; 1 on reduced
  * axes; 0 = the default for that axis) and marches through tile_x planes along x (0 = about 8192
- * blocks). tile_x < 0 selects the per-cell step kernel. Contexts with two or three active axes
+ * blocks in 3D, 16 planes in 2D). 2D tiles of at most 256 cells (396 with their halo), x included,
+ * are staged whole instead. tile_x < 0 selects the per-cell step kernel. Contexts with two or three active axes
  * start with the default tile; 1D grids always use the per-cell kernel. Results do not depend on
  * the shape. */
 mpf_status mpf_set_tile_shape(mpf_ctx* ctx, int32_t tile_x, int32_t tile_y, int32_t tile_z);

@@ -183,7 +183,7 @@ struct mpf_ctx {
 // Members of one kernel variant (precision, orientation/driving-force terms, equal-energy form)
 // share every launch: device arrays of their arguments for the two captured steps.
 struct mpf_group {
-    bool fp32 = false, full = false, uni = false, tiled = false;
+    bool fp32 = false, full = false, uni = false, tiled = false, flat = false;
     std::vector<int> members;
     std::vector<mpf::StepArgs> h_a1, h_a2;
     std::vector<mpf::GrainArgs> h_g;
@@ -286,29 +286,37 @@ mpf::GrainArgs grain_args(const mpf_ctx* c)
 
 unsigned step_blocks(const mpf_ctx* c) { return static_cast<unsigned>((c->ncells + mpf::kBlock - 1) / mpf::kBlock); }
 
-// Tile shape of the LDS-tiled step kernel for this grid: z (the contiguous axis) up to 64 cells
-// wide in 3D (256 when y is reduced), y filling 256 threads, the halo plane within kTileHalo; x
-// chunks sized for about 8192 blocks (256^3 FP64: 2.38 ms at 8 planes per block, 2.42 at 4, 2.45
-// at 16, 2.61 at 32). 1D grids keep the per-cell kernel (tile_x = 0).
+// Tile shape of the LDS-tiled step kernel for this grid. 3D: 16 x 16 cells of the (y, z) plane (a
+// smaller halo than 4 x 64) and chunks of x sized for about 8192 blocks (256^3 FP64: 2.38 ms at 8
+// planes per block, 2.42 at 4, 2.45 at 16, 2.61 at 32). 2D grids that hold x: 16 x 16 cells of the
+// plane, one tile per block (flat_tile); a (y, z) plane: 64 cells along z. 1D grids keep the per-cell
+// kernel (tile_x = 0). The halo plane stays within kTileHalo.
 void tile_shape(const mpf_ctx* c, int tile_x, int* ty, int* tz, int* tx)
 {
     *ty = *tz = *tx = 0;
     if (c->active < 2) return;
-    // 16 x 16 in 3D (the tile the autotuner picks at 256^3: a smaller halo than 4 x 64), 64 cells
-    // along z in 2D (y, z) planes, whole z rows otherwise
-    int z = c->dnz ? std::min(c->nz, c->dny ? (c->dnx ? 16 : 64) : 256) : 1;
-    int y = c->dny ? std::min(c->ny, std::max(1, mpf::kBlock / z)) : 1;
+    int z = c->dnz ? std::min(c->nz, c->dnx ? 16 : 64) : 1;
+    int y = c->dny ? std::min(c->ny, c->dnx ? 16 : std::max(1, mpf::kBlock / z)) : 1;
     while ((y + 2 * c->dny) * (z + 2 * c->dnz) > mpf::kTileHalo && y > 1) --y;
     while ((y + 2 * c->dny) * (z + 2 * c->dnz) > mpf::kTileHalo && z > 1) --z;
     int x = tile_x;
     if (x <= 0) {
         const int64_t per = static_cast<int64_t>(y) * z * 8192;
-        x = static_cast<int>(std::min<int64_t>(32, std::max<int64_t>(1, c->ncells / per)));
+        x = c->active == 2 ? 16 : static_cast<int>(std::min<int64_t>(32, std::max<int64_t>(1, c->ncells / per)));
     }
     if (!c->dnx) x = 1;
     *ty = y;
     *tz = z;
     *tx = std::min(x, c->nx);
+}
+
+// A 2D grid that holds x, whose tile of tile_x cells along x and tile_y (tile_z) along the other axis
+// fits one block with its halo: staged at once. A longer tile marches along x.
+bool flat_tile(const mpf_ctx* c)
+{
+    const int other = c->dny ? c->tile_y : c->tile_z;
+    return c->active == 2 && c->dnx && c->tile_x > 0 && c->tile_x * other <= mpf::kBlock &&
+           (c->tile_x + 2) * (other + 2) <= mpf::kTileHalo;
 }
 
 unsigned tile_blocks(const mpf_ctx* c)
@@ -323,7 +331,8 @@ unsigned tile_blocks(const mpf_ctx* c)
 hipError_t launch_main(const mpf_ctx* c, const mpf::StepArgs& a, hipStream_t stream)
 {
     const bool full = full_variant(c);
-    if (c->tile_x > 0) return static_cast<hipError_t>(mpf::launch_tile(a, tile_blocks(c), c->fp32, full, c->uniform, stream));
+    if (c->tile_x > 0) return static_cast<hipError_t>(mpf::launch_tile(a, tile_blocks(c), c->fp32, full, c->uniform,
+                                                                           flat_tile(c), stream));
     return static_cast<hipError_t>(mpf::launch_step(a, nullptr, nullptr, 1, step_blocks(c), c->fp32, full, c->uniform, stream));
 }
 unsigned grain_blocks(const mpf_ctx* c)
@@ -1452,8 +1461,8 @@ mpf_status mpf_autotune(mpf_ctx* c, double dt, int32_t steps, int32_t* xcd_order
     if (c->active >= 2 && !st) {
         std::vector<std::array<int, 2>> planes;
         if (c->dny && c->dnz) planes = {{4, 64}, {8, 32}, {16, 16}, {4, 32}};
-        else if (c->dny) planes = {{64, 1}, {128, 1}, {256, 1}};
-        else planes = {{1, 64}, {1, 128}, {1, 256}};
+        else if (c->dny) planes = {{16, 1}, {32, 1}, {64, 1}, {128, 1}, {256, 1}};
+        else planes = {{1, 16}, {1, 32}, {1, 64}, {1, 128}, {1, 256}};
         std::vector<std::array<int, 3>> cands = {{0, 0, 0}};  // tile_x 0: the per-cell kernel
         std::vector<std::array<int, 2>> seen;
         for (auto pl : planes) {
@@ -1462,7 +1471,9 @@ mpf_status mpf_autotune(mpf_ctx* c, double dt, int32_t steps, int32_t* xcd_order
             if ((ty + 2 * c->dny) * (tz + 2 * c->dnz) > mpf::kTileHalo) continue;
             if (std::find(seen.begin(), seen.end(), std::array<int, 2>{ty, tz}) != seen.end()) continue;
             seen.push_back({ty, tz});
-            for (int xs : {0, 1, 4, 16}) {
+            // 2D: 8 rows complete the 8 x 32 tile
+            for (int xs : {0, 1, 4, 8, 16}) {
+                if (xs == 8 && c->active != 2) continue;
                 int dy = 0, dz = 0, tx = 0;
                 tile_shape(c, xs, &dy, &dz, &tx);
                 cands.push_back({tx, ty, tz});
@@ -1624,10 +1635,10 @@ bool build_args(mpf_ensemble* e, const double* dt)
 
 // Group of a member: kernel variant (precision; a member with a driving force runs the full
 // variant whether mpf_set_step_terms switched it on or off - off: an all-zero mode table - so the
-// grouping holds across switches; uniform tables) and step kernel (tiled or per-cell).
-std::array<bool, 4> group_key(const mpf_ctx* c)
+// grouping holds across switches; uniform tables) and step kernel (tiled, flat or marching, or per-cell).
+std::array<bool, 5> group_key(const mpf_ctx* c)
 {
-    return {c->fp32, c->grad || c->dg, c->uniform, c->tile_x > 0};
+    return {c->fp32, c->grad || c->dg, c->uniform, c->tile_x > 0, flat_tile(c)};
 }
 
 // Sorts the members into groups by group_key; drops the graph.
@@ -1637,10 +1648,10 @@ void regroup(mpf_ensemble* e)
     for (auto& g : e->groups) free_group(g);
     e->groups.clear();
     for (size_t i = 0; i < e->members.size(); ++i) {
-        const std::array<bool, 4> k = group_key(e->members[i]);
+        const std::array<bool, 5> k = group_key(e->members[i]);
         mpf_group* g = nullptr;
         for (auto& q : e->groups)
-            if (std::array<bool, 4>{q.fp32, q.full, q.uni, q.tiled} == k) g = &q;
+            if (std::array<bool, 5>{q.fp32, q.full, q.uni, q.tiled, q.flat} == k) g = &q;
         if (!g) {
             e->groups.emplace_back();
             g = &e->groups.back();
@@ -1648,6 +1659,7 @@ void regroup(mpf_ensemble* e)
             g->full = k[1];
             g->uni = k[2];
             g->tiled = k[3];
+            g->flat = k[4];
         }
         g->members.push_back(static_cast<int>(i));
     }
@@ -1658,7 +1670,7 @@ bool regroup_needed(const mpf_ensemble* e)
 {
     for (const auto& g : e->groups)
         for (int m : g.members)
-            if (group_key(e->members[m]) != std::array<bool, 4>{g.fp32, g.full, g.uni, g.tiled}) return true;
+            if (group_key(e->members[m]) != std::array<bool, 5>{g.fp32, g.full, g.uni, g.tiled, g.flat}) return true;
     return false;
 }
 
@@ -1697,7 +1709,7 @@ mpf_status capture(mpf_ensemble* e)
                 if ((half == 0 ? g.h_a1[k] : g.h_a2[k]).dg_avg) rc = mpf::launch_dg_average(avg_args(c, half == 0 ? g.h_a1[k] : g.h_a2[k]), g.fp32, e->stream);
             }
             if (!rc)
-                rc = g.tiled ? mpf::launch_tile_batch(args, g.d_first, n, blocks, g.fp32, g.full, g.uni, e->stream)
+                rc = g.tiled ? mpf::launch_tile_batch(args, g.d_first, n, blocks, g.fp32, g.full, g.uni, g.flat, e->stream)
                              : mpf::launch_step(half == 0 ? g.h_a1[0] : g.h_a2[0], args, g.d_first, n, blocks, g.fp32,
                                                 g.full, g.uni, e->stream);
             if (!rc) rc = mpf::launch_deferred(args, n, g.per_domain, g.fp32, g.full, e->stream);

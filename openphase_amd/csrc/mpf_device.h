@@ -133,12 +133,13 @@ int launch_adjoint(const AdjointArgs& a, bool fp32, void* stream);
 constexpr int kGrainBlock = 256;                     // threads per block of the grain kernel
 constexpr int kTileHalo = 396;                       // cells of a tile plane with its halo, at most (6 x 66)
 
-// LDS-tiled step kernel over one domain (mpf_tile.hip); `blocks` = tiles x x-chunks.
-int launch_tile(const StepArgs& a, unsigned blocks, bool fp32, bool full, bool uni, void* stream);
+// LDS-tiled step kernel over one domain (mpf_tile.hip); `blocks` = tiles x x-chunks. flat: a 2D grid
+// in tiles of tile_x cells along x and tile_y (or tile_z) along its other active axis.
+int launch_tile(const StepArgs& a, unsigned blocks, bool fp32, bool full, bool uni, bool flat, void* stream);
 // The same over several domains (device array `args`, first[d] = the first block of domain d,
 // ndom + 1 prefix sums of the domains' tile counts), each with its own tile shape.
 int launch_tile_batch(const StepArgs* args, const uint32_t* first, int ndom, unsigned blocks, bool fp32, bool full,
-                      bool uni, void* stream);
+                      bool uni, bool flat, void* stream);
 
 // Averaging over the interface (mpf_dgavg.hip): CollectAverage into `tmp`, DistributeAverage into
 // `avg`, both [pairs][ncells] with pair a < b of the own entries at b(b-1)/2 + a.

@@ -6,7 +6,8 @@
 // include/Containers/NodePF.h:214-255) on the neighbour-merged lists of CalculateDerivativesSR
 // (src/PhaseField.cpp:566-615), with a different way of reading the neighbourhood.
 //
-// A block owns a TY x TZ tile of the (y, z) plane and marches along x through CH planes. Each
+// A block owns a TY x TZ tile of the (y, z) plane and marches along x through CH planes (2D grids: a tile
+// of the whole plane, no marching). Each
 // plane of the tile plus a one-cell halo is staged in LDS once (a ring of three planes: x-1, x,
 // x+1), so every state entry is read from memory about (CH + 2) / CH x (halo area) times instead of
 // 27 times. Grains are renamed to local ids 0..31 per block (an LDS hash table filled as planes are
@@ -96,12 +97,19 @@ __device__ __forceinline__ void lds_unit_add(unsigned long long (*acc)[kCopies][
     }
 }
 
+// Whether the box has offset (dx, dy, dz). FLAT: the tile's plane is the whole of a 2D grid.
+template <bool FLAT> __device__ __forceinline__ bool box_in(const StepArgs& A, int dx, int dy, int dz)
+{
+    if (FLAT) return dx == 0;
+    return (dx == 0 || A.dnx) && (dy == 0 || A.dny) && (dz == 0 || A.dnz);
+}
+
 // Laplacians (and gradients) of the first T merged entries of a cell in stencil order (x outer, z
 // inner; inactive axes skipped): entry t of neighbour k contributes w_k * value, the value staged
 // at rank popcount(mask & lm[t]) when bit bm[t] is set and a zero otherwise (adding w * 0 leaves a
 // sum unchanged: the sums are never -0). pl: ring slots of the planes x-1, x, x+1; wh: the cell's
 // index in its halo plane.
-template <int T, int K, typename TV, typename TC, bool GRAD>
+template <int T, int K, typename TV, typename TC, bool GRAD, bool FLAT>
 __device__ __forceinline__ void tile_derivatives(const StepArgs& A, const uint32_t (*s_mask)[kTileHalo],
                                                  const TV (*s_val)[kRanks][kTileHalo], const TV* zero, const int pl[3],
                                                  int wh, int HZ, const uint32_t bm[K], const uint32_t lm[K],
@@ -110,7 +118,7 @@ __device__ __forceinline__ void tile_derivatives(const StepArgs& A, const uint32
 #pragma unroll
     for (int k = 0; k < 27; ++k) {
         const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
-        if (!((dx == 0 || A.dnx) && (dy == 0 || A.dny) && (dz == 0 || A.dnz))) continue;
+        if (!box_in<FLAT>(A, dx, dy, dz)) continue;
         const int p = pl[dx + 1];
         const int hh = wh + dy * HZ + dz;
         const uint32_t m = s_mask[p][hh];
@@ -137,12 +145,19 @@ __device__ __forceinline__ void tile_derivatives(const StepArgs& A, const uint32
 
 // One block of the tiled step: tile `b` of the domain A (tiles numbered z fastest, then y, then
 // the x-chunk).
-template <typename TV, typename TC, bool GRAD, bool DG, bool UNI>
+// FLAT: a 2D grid whose active axes are x and one of y and z, taken as the plane of one tile per
+// block (its cells are laid out like those of a grid reduced in x), so that a block stages its tile
+// once, in two memory round trips, and walks 9 neighbours of one plane. As a row of y marching
+// through planes of x a block staged three rows one after the other for each row of cells: 53 us at
+// 512^2 FP64, 86 us at 331 x 257 with orientation-dependent energies (FP32), 686 us for 64 FP32 domains
+// of 128^2 to 512^2 in one launch; now 26, 43 and 266 us.
+template <typename TV, typename TC, bool GRAD, bool DG, bool UNI, bool FLAT>
 __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
 {
-    __shared__ uint32_t s_info[3][kTileHalo];
-    __shared__ uint32_t s_mask[3][kTileHalo];
-    __shared__ TV s_val[3][kRanks][kTileHalo];
+    constexpr int kPlanes = FLAT ? 1 : 3;
+    __shared__ uint32_t s_info[kPlanes][kTileHalo];
+    __shared__ uint32_t s_mask[kPlanes][kTileHalo];
+    __shared__ TV s_val[kPlanes][kRanks][kTileHalo];
     __shared__ TV s_zero;
     __shared__ int32_t s_key[kLocal];
     __shared__ unsigned long long s_acc[kLocal][kCopies][kLimbs];
@@ -157,15 +172,16 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
     constexpr int K = kMainSlots;
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
     const int64_t N = A.ncells;
-    const int NY = A.ny, NZ = A.nz;
-    const int TY = A.tile_y, TZ = A.tile_z;
-    const int HZ = TZ + 2 * A.dnz, HP = (TY + 2 * A.dny) * HZ;
+    const int NX = FLAT ? 1 : A.nx, NY = FLAT ? A.nx : A.ny, NZ = FLAT ? A.ny * A.nz : A.nz;
+    const int TX = FLAT ? 1 : A.tile_x, TY = FLAT ? A.tile_x : A.tile_y, TZ = FLAT ? A.tile_y * A.tile_z : A.tile_z;
+    const int DX = FLAT ? 0 : A.dnx, DY = FLAT ? 1 : A.dny, DZ = FLAT ? 1 : A.dnz;
+    const int HZ = TZ + 2 * DZ, HP = (TY + 2 * DY) * HZ;
     const int nty = (NY + TY - 1) / TY, ntz = (NZ + TZ - 1) / TZ;
     const int tz = static_cast<int>(b % static_cast<unsigned>(ntz));
     const int ty = static_cast<int>((b / static_cast<unsigned>(ntz)) % static_cast<unsigned>(nty));
     const int xc = static_cast<int>(b / static_cast<unsigned>(ntz * nty));
     const int y0 = ty * TY, z0 = tz * TZ;
-    const int x0 = xc * A.tile_x, x1 = min(x0 + A.tile_x, A.nx);
+    const int x0 = xc * TX, x1 = min(x0 + TX, NX);
 
     if (tid < kLocal) s_key[tid] = -1;
     if (tid < 2) s_ndefer[tid] = 0;
@@ -197,7 +213,7 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
         const int h = tid + j * kBlock;
         hv[j] = h < HP;
         const int hy = h / HZ, hz = h - hy * HZ;
-        int yg = y0 - A.dny + hy, zg = z0 - A.dnz + hz;
+        int yg = y0 - DY + hy, zg = z0 - DZ + hz;
         yg = yg < 0 ? yg + NY : (yg >= NY ? yg - NY : yg);
         zg = zg < 0 ? zg + NZ : (zg >= NZ ? zg - NZ : zg);
         yz[j] = hv[j] ? static_cast<uint32_t>(yg * NZ + zg) : 0u;
@@ -261,33 +277,33 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
         }
     };
 
-    auto ring = [&](int x) { return (x - x0 + 1) % 3; };
-    auto wrapx = [&](int x) { return x < 0 ? x + A.nx : (x >= A.nx ? x - A.nx : x); };
+    auto ring = [&](int x) { return FLAT ? 0 : (x - x0 + 1) % 3; };
+    auto wrapx = [&](int x) { return x < 0 ? x + NX : (x >= NX ? x - NX : x); };
     uint8_t codes[2];
-    if (A.dnx) {
+    if (DX) {
         fetch(wrapx(x0 - 1), codes);
         stage(ring(x0 - 1), wrapx(x0 - 1), codes);
     }
     fetch(x0, codes);
     stage(ring(x0), x0, codes);
-    if (A.dnx) fetch(wrapx(x0 + 1), codes);
+    if (DX) fetch(wrapx(x0 + 1), codes);
     __syncthreads();
 
 #pragma unroll 1
     for (int x = x0; x < x1; ++x) {
-        if (A.dnx) {
+        if (DX) {
             stage(ring(x + 1), wrapx(x + 1), codes);
             if (x + 1 < x1) fetch(wrapx(x + 2), codes);
         }
         __syncthreads();
-        const int pl0 = A.dnx ? ring(x - 1) : ring(x), pl1 = ring(x), pl2 = A.dnx ? ring(x + 1) : ring(x);
+        const int pl0 = DX ? ring(x - 1) : ring(x), pl1 = ring(x), pl2 = DX ? ring(x + 1) : ring(x);
         const int par = (x - x0) & 1;
 
         // ---- classify the tile's cells: bulk cells are copied, wide cells compacted for the
         // second phase, cells the tile cannot hold deferred
         const int ly = tid / TZ, lz = tid - (tid / TZ) * TZ;
         const bool own = tid < TY * TZ && y0 + ly < NY && z0 + lz < NZ;
-        const int oh = (ly + A.dny) * HZ + lz + A.dnz;
+        const int oh = (ly + DY) * HZ + lz + DZ;
         const int64_t c = own ? (static_cast<int64_t>(x) * NY + (y0 + ly)) * NZ + (z0 + lz) : 0;
         bool wide = false, single = false;
         int slid = 0;
@@ -300,7 +316,7 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
             for (int k = 0; k < 27; ++k) {
                 if (k == 13) continue;
                 const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
-                if (!((dx == 0 || A.dnx) && (dy == 0 || A.dny) && (dz == 0 || A.dnz))) continue;
+                if (!box_in<FLAT>(A, dx, dy, dz)) continue;
                 const uint32_t inf = s_info[dx < 0 ? pl0 : (dx > 0 ? pl2 : pl1)][oh + dy * HZ + dz];
                 multi = multi || (inf & 15u) > 1u;
                 bad = bad || ((inf >> kInfoBad) & 1u) != 0u;
@@ -363,7 +379,7 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
             const int pl[3] = {pl0, pl1, pl2};
             const int local = tid < nwide ? s_list[tid] : 0;
             const int wy = local / TZ, wz = local - (local / TZ) * TZ;
-            const int wh = (wy + A.dny) * HZ + wz + A.dnz;
+            const int wh = (wy + DY) * HZ + wz + DZ;
             const int64_t cw = (static_cast<int64_t>(x) * NY + (y0 + wy)) * NZ + (z0 + wz);
             const uint32_t inf0 = s_info[pl1][wh];
             const uint32_t m0 = s_mask[pl1][wh];
@@ -381,7 +397,7 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
 #pragma unroll
             for (int k = 0; k < 27; ++k) {
                 const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
-                if (k == 13 || !((dx == 0 || A.dnx) && (dy == 0 || A.dny) && (dz == 0 || A.dnz))) continue;
+                if (k == 13 || !box_in<FLAT>(A, dx, dy, dz)) continue;
                 const int p = pl[dx + 1];
                 const int hh = wh + dy * HZ + dz;
                 const uint32_t nw = s_mask[p][hh] & ~seen;
@@ -414,9 +430,19 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
                 lm[t] = bm[t] - 1u;
             }
             // Laplacians (and gradients) for as many entries as the wavefront's longest list
-            if (__any(go && ne > 3)) tile_derivatives<4>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
-            else if (__any(go && ne > 2)) tile_derivatives<3>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
-            else if (__any(go)) tile_derivatives<2>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
+            if (__any(go && ne > 3)) tile_derivatives<4, K, TV, TC, GRAD, FLAT>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
+            else if (__any(go && ne > 2)) tile_derivatives<3, K, TV, TC, GRAD, FLAT>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
+            else if (__any(go)) tile_derivatives<2, K, TV, TC, GRAD, FLAT>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
+            if (GRAD && FLAT) {
+                // the plane's axes are x and the grid's second active one
+#pragma unroll
+                for (int t = 0; t < K; ++t) {
+                    TC (&gr)[3] = L.gr[GRAD ? t : 0];
+                    gr[0] = gr[1];
+                    gr[1] = A.dny ? gr[2] : TC(0);
+                    gr[2] = A.dny ? TC(0) : gr[2];
+                }
+            }
             if (go) {
                 // own values (FP64; the FP32 implicit entry as 1 - sum of the others in slot order)
                 const int imp0 = static_cast<int>((inf0 >> kInfoImp) & 15u);
@@ -512,58 +538,57 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
     if (bad_volume) atomicOr(&A.status[kStatusVolumeRange], 1);
 }
 
-template <typename TV, typename TC, bool GRAD, bool DG, bool UNI>
+template <typename TV, typename TC, bool GRAD, bool DG, bool UNI, bool FLAT>
 __global__ __launch_bounds__(kBlock, sizeof(TV) == 4 && !GRAD ? 4 : 1) void tile_kernel(const StepArgs A)
 {
-    tile_block<TV, TC, GRAD, DG, UNI>(A, A.xcd_order ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x);
+    tile_block<TV, TC, GRAD, DG, UNI, FLAT>(A, A.xcd_order ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x);
 }
 
 // Several domains in one launch (ensembles): block b belongs to the domain d with
 // first[d] <= b < first[d+1], each with its own tile shape.
-template <typename TV, typename TC, bool GRAD, bool DG, bool UNI>
+template <typename TV, typename TC, bool GRAD, bool DG, bool UNI, bool FLAT>
 __global__ __launch_bounds__(kBlock, sizeof(TV) == 4 && !GRAD ? 4 : 1) void tile_batch_kernel(
     const StepArgs* __restrict__ batch, const uint32_t* __restrict__ first, int32_t ndom)
 {
     const int dom = batch_domain(first, ndom, blockIdx.x);
-    tile_block<TV, TC, GRAD, DG, UNI>(batch[dom], blockIdx.x - first[dom]);
+    tile_block<TV, TC, GRAD, DG, UNI, FLAT>(batch[dom], blockIdx.x - first[dom]);
 }
 
 }  // namespace
 
-int launch_tile(const StepArgs& a, unsigned blocks, bool fp32, bool full, bool uni, void* stream)
+// The variants of a precision, by the macro LAUNCH(type, gradients, driving force, uniform).
+#define MPF_TILE_VARIANTS(LAUNCH)                  \
+    if (fp32) {                                    \
+        if (full) { LAUNCH(float, true, true, false); }   \
+        else if (uni) { LAUNCH(float, false, false, true); }  \
+        else { LAUNCH(float, false, false, false); } \
+    } else {                                       \
+        if (full) { LAUNCH(double, true, true, false); }  \
+        else if (uni) { LAUNCH(double, false, false, true); } \
+        else { LAUNCH(double, false, false, false); }\
+    }
+
+int launch_tile(const StepArgs& a, unsigned blocks, bool fp32, bool full, bool uni, bool flat, void* stream)
 {
     const dim3 grid(blocks);
     hipStream_t s = static_cast<hipStream_t>(stream);
-#define MPF_TILE(TV, G, D, U) hipLaunchKernelGGL((tile_kernel<TV, TV, G, D, U>), grid, dim3(kBlock), 0, s, a)
-    if (fp32) {
-        if (full)     MPF_TILE(float, true, true, false);
-        else if (uni) MPF_TILE(float, false, false, true);
-        else          MPF_TILE(float, false, false, false);
-    } else {
-        if (full)     MPF_TILE(double, true, true, false);
-        else if (uni) MPF_TILE(double, false, false, true);
-        else          MPF_TILE(double, false, false, false);
-    }
+#define MPF_TILE(TV, G, D, U)                                                                                     \
+    if (flat) hipLaunchKernelGGL((tile_kernel<TV, TV, G, D, U, true>), grid, dim3(kBlock), 0, s, a);              \
+    else hipLaunchKernelGGL((tile_kernel<TV, TV, G, D, U, false>), grid, dim3(kBlock), 0, s, a)
+    MPF_TILE_VARIANTS(MPF_TILE)
 #undef MPF_TILE
     return static_cast<int>(hipGetLastError());
 }
 
 int launch_tile_batch(const StepArgs* args, const uint32_t* first, int ndom, unsigned blocks, bool fp32, bool full,
-                      bool uni, void* stream)
+                      bool uni, bool flat, void* stream)
 {
     const dim3 grid(blocks);
     hipStream_t s = static_cast<hipStream_t>(stream);
-#define MPF_TILE(TV, G, D, U) \
-    hipLaunchKernelGGL((tile_batch_kernel<TV, TV, G, D, U>), grid, dim3(kBlock), 0, s, args, first, ndom)
-    if (fp32) {
-        if (full)     MPF_TILE(float, true, true, false);
-        else if (uni) MPF_TILE(float, false, false, true);
-        else          MPF_TILE(float, false, false, false);
-    } else {
-        if (full)     MPF_TILE(double, true, true, false);
-        else if (uni) MPF_TILE(double, false, false, true);
-        else          MPF_TILE(double, false, false, false);
-    }
+#define MPF_TILE(TV, G, D, U)                                                                                           \
+    if (flat) hipLaunchKernelGGL((tile_batch_kernel<TV, TV, G, D, U, true>), grid, dim3(kBlock), 0, s, args, first, ndom); \
+    else hipLaunchKernelGGL((tile_batch_kernel<TV, TV, G, D, U, false>), grid, dim3(kBlock), 0, s, args, first, ndom)
+    MPF_TILE_VARIANTS(MPF_TILE)
 #undef MPF_TILE
     return static_cast<int>(hipGetLastError());
 }
