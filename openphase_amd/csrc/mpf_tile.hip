@@ -11,9 +11,10 @@
 // plane of the tile plus a one-cell halo is staged in LDS once (a ring of three planes: x-1, x,
 // x+1), so every state entry is read from memory about (CH + 2) / CH x (halo area) times instead of
 // 27 times. Grains are renamed to local ids 0..31 per block (an LDS hash table filled as planes are
-// staged); a staged cell is a presence mask over local ids, its list order (up to three local ids)
-// and its values ordered by local id. A cell's merged list is then the OR of 27 masks, walked in
-// stencil order only where a new grain appears (to keep the reference's insertion order), and the
+// staged); a staged cell is a presence mask over local ids, its list order (up to four local ids)
+// and its values ordered by local id. A cell's merged list is then the OR of 27 masks (one plane's
+// nine formed per plane, the other two kept), walked in stencil order only where neighbours add
+// more than one grain (to keep the reference's insertion order), and the
 // Laplacian (and gradient) of merged entry t is a sum over the 27 neighbours of one LDS value each,
 // at rank popcount(mask & below(t)) or a zero when the bit is clear: no list searches.
 //
@@ -40,14 +41,14 @@ namespace {
 
 constexpr int kRanks = 4;        // entries per staged cell (longer lists make their neighbourhood deferred)
 constexpr int kLocal = 32;       // local grain ids per block
-constexpr int kCopies = 4;       // copies of the volume accumulators (lanes spread over them)
+constexpr int kCopies = 2;       // copies of the volume accumulators (lanes spread over them)
 constexpr int kTileWaves = kBlock / 64;
 static_assert(kTileHalo <= 2 * kBlock, "a thread stages at most two cells of a plane");
 
 // info word of a staged cell: bits 0-3 entry count, bit 4 unusable (more than kRanks entries or
 // an unmapped grain), bits 5-8 the FP32 implicit slot (15: none), bits 9-28 the local ids of the
-// first four entries in list order (5 bits each)
-constexpr int kInfoBad = 4, kInfoImp = 5, kInfoOrd = 9;
+// first four entries in list order (5 bits each), bit 29 more than one entry
+constexpr int kInfoBad = 4, kInfoImp = 5, kInfoOrd = 9, kInfoMulti = 29;
 
 // Local id of grain g in the block's table (open addressing over 32 slots; the slot is the id),
 // inserting it when absent. -1 when the table is full.
@@ -97,47 +98,70 @@ __device__ __forceinline__ void lds_unit_add(unsigned long long (*acc)[kCopies][
     }
 }
 
-// Whether the box has offset (dx, dy, dz). FLAT: the tile's plane is the whole of a 2D grid.
-template <bool FLAT> __device__ __forceinline__ bool box_in(const StepArgs& A, int dx, int dy, int dz)
+// Whether a plane of the box has offset (dy, dz). FLAT: the tile's plane is the whole of a 2D grid.
+template <bool FLAT> __device__ __forceinline__ bool box_in(const StepArgs& A, int dy, int dz)
 {
-    if (FLAT) return dx == 0;
-    return (dx == 0 || A.dnx) && (dy == 0 || A.dny) && (dz == 0 || A.dnz);
+    return FLAT || ((dy == 0 || A.dny) && (dz == 0 || A.dnz));
+}
+
+// OR of the cells of a staged plane within the box around cell h.
+template <bool FLAT> __device__ __forceinline__ uint2 plane_union(const StepArgs& A, const uint2* plane, int h, int HZ)
+{
+    uint2 u = make_uint2(0u, 0u);
+#pragma unroll
+    for (int j = 0; j < 9; ++j) {
+        const int dy = j / 3 - 1, dz = j % 3 - 1;
+        if (!box_in<FLAT>(A, dy, dz)) continue;
+        const uint2 cell = plane[h + dy * HZ + dz];
+        u.x |= cell.x;
+        u.y |= cell.y;
+    }
+    return u;
 }
 
 // Laplacians (and gradients) of the first T merged entries of a cell in stencil order (x outer, z
 // inner; inactive axes skipped): entry t of neighbour k contributes w_k * value, the value staged
 // at rank popcount(mask & lm[t]) when bit bm[t] is set and a zero otherwise (adding w * 0 leaves a
-// sum unchanged: the sums are never -0). pl: ring slots of the planes x-1, x, x+1; wh: the cell's
-// index in its halo plane.
+// sum unchanged: the sums are never -0). pl0-2: ring slots of the planes x-1, x, x+1; wh: the cell's
+// index in its halo plane. A loop over the planes, not unrolled: see tile_block.
 template <int T, int K, typename TV, typename TC, bool GRAD, bool FLAT>
-__device__ __forceinline__ void tile_derivatives(const StepArgs& A, const uint32_t (*s_mask)[kTileHalo],
-                                                 const TV (*s_val)[kRanks][kTileHalo], const TV* zero, const int pl[3],
+__device__ __forceinline__ void tile_derivatives(const StepArgs& A, const uint2 (*s_cell)[kTileHalo],
+                                                 const TV (*s_val)[kRanks][kTileHalo], const TV* zero, int pl0, int pl1, int pl2,
                                                  int wh, int HZ, const uint32_t bm[K], const uint32_t lm[K],
                                                  CellList<K, TC, GRAD>& L)
 {
+#pragma unroll 1
+    for (int dx = FLAT ? 0 : -A.dnx; dx <= (FLAT ? 0 : A.dnx); ++dx) {
+        const int p = dx < 0 ? pl0 : (dx > 0 ? pl2 : pl1);
+        TC wl[3], wg[3];
 #pragma unroll
-    for (int k = 0; k < 27; ++k) {
-        const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
-        if (!box_in<FLAT>(A, dx, dy, dz)) continue;
-        const int p = pl[dx + 1];
-        const int hh = wh + dy * HZ + dz;
-        const uint32_t m = s_mask[p][hh];
-        const int nj = (dy != 0) + (dz != 0);
-        const TC w = static_cast<TC>(dx != 0 ? A.wl[nj + 1] : A.wl[nj]);
-        const TC gw = static_cast<TC>(dx != 0 ? A.wg[nj + 1] : A.wg[nj]);
-        const TC gwx = dx == 0 ? TC(0) : (dx < 0 ? -gw : gw);
-        const TC gwy = dy == 0 ? TC(0) : (dy < 0 ? -gw : gw);
-        const TC gwz = dz == 0 ? TC(0) : (dz < 0 ? -gw : gw);
+        for (int nj = 0; nj < 3; ++nj) {
+            wl[nj] = static_cast<TC>(dx != 0 ? A.wl[nj + 1] : A.wl[nj]);
+            wg[nj] = static_cast<TC>(dx != 0 ? A.wg[nj + 1] : A.wg[nj]);
+        }
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-            const bool pres = (m & bm[t]) != 0u;
-            const TV* src = pres ? &s_val[p][__popc(m & lm[t])][hh] : zero;
-            const TC a = static_cast<TC>(*src);
-            L.lap[t] += w * a;
-            if (GRAD && k != 13) {
-                L.gr[GRAD ? t : 0][0] = L.gr[GRAD ? t : 0][0] + gwx * a;
-                L.gr[GRAD ? t : 0][1] = L.gr[GRAD ? t : 0][1] + gwy * a;
-                L.gr[GRAD ? t : 0][2] = L.gr[GRAD ? t : 0][2] + gwz * a;
+        for (int j = 0; j < 9; ++j) {
+            const int dy = j / 3 - 1, dz = j % 3 - 1;
+            if (!box_in<FLAT>(A, dy, dz)) continue;
+            const int hh = wh + dy * HZ + dz;
+            const uint32_t m = s_cell[p][hh].y;
+            const int nj = (dy != 0) + (dz != 0);
+            const TC w = wl[nj], gw = wg[nj];
+            const TC gwx = dx == 0 ? TC(0) : (dx < 0 ? -gw : gw);
+            const TC gwy = dy == 0 ? TC(0) : (dy < 0 ? -gw : gw);
+            const TC gwz = dz == 0 ? TC(0) : (dz < 0 ? -gw : gw);
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const bool pres = (m & bm[t]) != 0u;
+                const TV* src = pres ? &s_val[p][__popc(m & lm[t])][hh] : zero;
+                const TC a = static_cast<TC>(*src);
+                L.lap[t] += w * a;
+                if (GRAD) {
+                    // the cell itself (all weights 0) adds 0
+                    if (!FLAT) L.gr[GRAD ? t : 0][0] = L.gr[GRAD ? t : 0][0] + gwx * a;
+                    if (dy != 0) L.gr[GRAD ? t : 0][1] = L.gr[GRAD ? t : 0][1] + gwy * a;
+                    if (dz != 0) L.gr[GRAD ? t : 0][2] = L.gr[GRAD ? t : 0][2] + gwz * a;
+                }
             }
         }
     }
@@ -145,6 +169,12 @@ __device__ __forceinline__ void tile_derivatives(const StepArgs& A, const uint32
 
 // One block of the tiled step: tile `b` of the domain A (tiles numbered z fastest, then y, then
 // the x-chunk).
+// What bounds it is latency - LDS lookups, barriers, divisions - at the three (FP64) or four
+// (FP32) wavefronts per SIMD that 52 KiB of LDS and the registers leave; two took 3.00 ms at 256^3
+// where three take 2.08. Cells go to the second phase sorted by merged length, so that a wavefront
+// runs the lookups and the update of one length, with the masks' OR deciding the length: 2.28 ->
+// 2.08 ms FP64, 1.89 -> 1.73 ms FP32, orientation variant 1.53 -> 1.39 ms at 160^3. The loops over
+// the box's planes are not unrolled (92 instead of 156 KB of code in the orientation variant).
 // FLAT: a 2D grid whose active axes are x and one of y and z, taken as the plane of one tile per
 // block (its cells are laid out like those of a grid reduced in x), so that a block stages its tile
 // once, in two memory round trips, and walks 9 neighbours of one plane. As a row of y marching
@@ -155,13 +185,14 @@ template <typename TV, typename TC, bool GRAD, bool DG, bool UNI, bool FLAT>
 __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
 {
     constexpr int kPlanes = FLAT ? 1 : 3;
-    __shared__ uint32_t s_info[kPlanes][kTileHalo];
-    __shared__ uint32_t s_mask[kPlanes][kTileHalo];
+    __shared__ uint2 s_cell[kPlanes][kTileHalo];   // info word, presence mask
     __shared__ TV s_val[kPlanes][kRanks][kTileHalo];
     __shared__ TV s_zero;
     __shared__ int32_t s_key[kLocal];
     __shared__ unsigned long long s_acc[kLocal][kCopies][kLimbs];
+    // wide cells of the plane, by merged length: tile-local index, and the grains their neighbours add
     __shared__ uint16_t s_list[kBlock];
+    __shared__ uint32_t s_new[kBlock];
     __shared__ uint32_t s_nwide[kTileWaves];
     // cells of a plane for the deferred-cell kernel, by plane parity: appended in LDS, moved to
     // the global work list by wavefront 0 after the plane (one global atomic per plane)
@@ -181,7 +212,7 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
     const int ty = static_cast<int>((b / static_cast<unsigned>(ntz)) % static_cast<unsigned>(nty));
     const int xc = static_cast<int>(b / static_cast<unsigned>(ntz * nty));
     const int y0 = ty * TY, z0 = tz * TZ;
-    const int x0 = xc * TX, x1 = min(x0 + TX, NX);
+    const int x0 = FLAT ? 0 : xc * TX, x1 = FLAT ? 1 : min(x0 + TX, NX);
 
     if (tid < kLocal) s_key[tid] = -1;
     if (tid < 2) s_ndefer[tid] = 0;
@@ -271,59 +302,71 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
                 for (int q = 0; q < kRanks; ++q)
                     if (q < n && v[j][q] != TV(0)) s_val[slot][__popc(mask & ((1u << lid[q]) - 1u))][h] = v[j][q];
             }
-            s_mask[slot][h] = bad ? 0u : mask;
-            s_info[slot][h] = static_cast<uint32_t>(n) | (bad ? 1u << kInfoBad : 0u) |
-                              (static_cast<uint32_t>(imp & 15) << kInfoImp) | ord;
+            const uint32_t info = static_cast<uint32_t>(n) | (bad ? 1u << kInfoBad : 0u) |
+                                  (static_cast<uint32_t>(imp & 15) << kInfoImp) | ord | (n > 1 ? 1u << kInfoMulti : 0u);
+            s_cell[slot][h] = make_uint2(info, bad ? 0u : mask);
         }
     };
 
-    auto ring = [&](int x) { return FLAT ? 0 : (x - x0 + 1) % 3; };
+    auto ring = [&](int x) { return FLAT ? 0 : (x - x0 + 1) % 3; };  // x >= x0 - 1
     auto wrapx = [&](int x) { return x < 0 ? x + NX : (x >= NX ? x - NX : x); };
     uint8_t codes[2];
-    if (DX) {
-        fetch(wrapx(x0 - 1), codes);
-        stage(ring(x0 - 1), wrapx(x0 - 1), codes);
-    }
-    fetch(x0, codes);
-    stage(ring(x0), x0, codes);
-    if (DX) fetch(wrapx(x0 + 1), codes);
-    __syncthreads();
-
+    uint2 below = make_uint2(0u, 0u), here = below, above = below;
+    fetch(wrapx(x0 - DX), codes);
+    if (FLAT) stage(0, x0, codes);
+    // plane x + 1 is staged before plane x is computed; the first planes are staged by the same code
 #pragma unroll 1
-    for (int x = x0; x < x1; ++x) {
-        if (DX) {
+    for (int x = FLAT ? x0 : x0 - 1 - DX; x < x1; ++x) {
+        if (!FLAT && x + 1 < x1 + DX) {
             stage(ring(x + 1), wrapx(x + 1), codes);
-            if (x + 1 < x1) fetch(wrapx(x + 2), codes);
+            if (x + 2 < x1 + DX) fetch(wrapx(x + 2), codes);
         }
         __syncthreads();
+        // what the cell's box holds in plane x + 1 (grains, multi-entry and unusable cells), with the two
+        // planes before it the whole box
+        const int ly = tid / TZ, lz = tid - (tid / TZ) * TZ;
+        const bool own = tid < TY * TZ && y0 + ly < NY && z0 + lz < NZ;
+        const int oh = (ly + DY) * HZ + lz + DZ;
+        if (!FLAT) {
+            below = here;
+            here = above;
+            above = make_uint2(0u, 0u);
+        }
+        if (own && (FLAT || x + 1 < x1 + DX)) above = plane_union<FLAT>(A, s_cell[FLAT ? 0 : ring(x + 1)], oh, HZ);
+        if (x < x0) continue;
         const int pl0 = DX ? ring(x - 1) : ring(x), pl1 = ring(x), pl2 = DX ? ring(x + 1) : ring(x);
         const int par = (x - x0) & 1;
 
         // ---- classify the tile's cells: bulk cells are copied, wide cells compacted for the
-        // second phase, cells the tile cannot hold deferred
-        const int ly = tid / TZ, lz = tid - (tid / TZ) * TZ;
-        const bool own = tid < TY * TZ && y0 + ly < NY && z0 + lz < NZ;
-        const int oh = (ly + DY) * HZ + lz + DZ;
+        // second phase by their merged length, cells the tile cannot hold deferred
         const int64_t c = own ? (static_cast<int64_t>(x) * NY + (y0 + ly)) * NZ + (z0 + lz) : 0;
-        bool wide = false, single = false;
+        bool single = false;
+        int ne = 0;                 // merged length of a wide cell
+        uint32_t fresh = 0u;        // grains that its neighbours add
         int slid = 0;
         double sv = 0.0;
         if (own) {
-            const uint32_t inf0 = s_info[pl1][oh];
+            const uint32_t inf0 = s_cell[pl1][oh].x;
             const int n0 = static_cast<int>(inf0 & 15u);
-            bool multi = n0 > 1, bad = ((inf0 >> kInfoBad) & 1u) != 0u;
+            const uint2 box = FLAT ? above : make_uint2(below.x | here.x | above.x, below.y | here.y | above.y);
+            if ((box.x >> kInfoMulti) & 1u) {
+                int dest = -1;      // the deferred-cell list of a cell the tile cannot hold
+                if (((box.x >> kInfoBad) & 1u) != 0u || n0 > K) {
+                    dest = 0;
+                } else {
+                    uint32_t listed = 0u;
 #pragma unroll
-            for (int k = 0; k < 27; ++k) {
-                if (k == 13) continue;
-                const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
-                if (!box_in<FLAT>(A, dx, dy, dz)) continue;
-                const uint32_t inf = s_info[dx < 0 ? pl0 : (dx > 0 ? pl2 : pl1)][oh + dy * HZ + dz];
-                multi = multi || (inf & 15u) > 1u;
-                bad = bad || ((inf >> kInfoBad) & 1u) != 0u;
-            }
-            if (multi) {
-                if (bad || n0 > K) s_defer[par][atomicAdd(&s_ndefer[par], 1)] = static_cast<uint16_t>(tid);
-                else wide = true;
+                    for (int t = 0; t < kRanks; ++t)
+                        if (t < n0) listed |= 1u << ((inf0 >> (kInfoOrd + 5 * t)) & 31u);
+                    fresh = box.y & ~listed;
+                    ne = n0 + __popc(fresh);
+                    // by merged length: 5-6 (and fewer than 2) entries, 7-8, 9 and more
+                    if (ne > K || ne < 2) dest = ne <= 6 ? 0 : (ne <= 8 ? 1 : 2);
+                }
+                if (dest >= 0) {
+                    ne = 0;
+                    s_defer[par][atomicAdd(&s_ndefer[par], 1)] = static_cast<uint16_t>(tid | (dest << 8));
+                }
             } else if (n0 == 1 && ((inf0 >> kInfoBad) & 1u) != 0u) {
                 // a lone entry whose grain did not fit the local ids
                 s_defer[par][atomicAdd(&s_ndefer[par], 1)] = static_cast<uint16_t>(tid);
@@ -347,17 +390,31 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
         lds_unit_add(s_acc, single && sv == 1.0, slid);
         if (single && sv != 1.0) lds_volume_add(s_acc, slid, sv, bad_volume);
 
-        const unsigned long long wm = __ballot(wide);
-        if (lane == 0) s_nwide[wave] = static_cast<uint32_t>(__popcll(wm));
+        // lists of 4, 3 and 2 merged entries in this order, so that a wavefront of the second phase
+        // holds one length as far as possible (its work grows with the longest list it holds)
+        unsigned long long wm[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) wm[q] = __ballot(ne == 4 - q);
+        if (lane == 0)
+            s_nwide[wave] = static_cast<uint32_t>(__popcll(wm[0]) | __popcll(wm[1]) << 10 | __popcll(wm[2]) << 20);
         __syncthreads();
-        int offset = __popcll(wm & ((1ull << lane) - 1ull)), nwide = 0;
+        uint32_t before = 0u, all = 0u;
 #pragma unroll
         for (int w = 0; w < kTileWaves; ++w) {
-            const int n = static_cast<int>(s_nwide[w]);
-            offset += w < wave ? n : 0;
-            nwide += n;
+            const uint32_t n = s_nwide[w];
+            before += w < wave ? n : 0u;
+            all += n;
         }
-        if (wide) s_list[offset] = static_cast<uint16_t>(tid);
+        const int n4 = static_cast<int>(all & 1023u), n3 = static_cast<int>((all >> 10) & 1023u);
+        const int nwide = n4 + n3 + static_cast<int>(all >> 20);
+        if (ne) {
+            const unsigned long long lower = (1ull << lane) - 1ull;
+            const int at = ne == 4   ? static_cast<int>(before & 1023u) + __popcll(wm[0] & lower)
+                           : ne == 3 ? n4 + static_cast<int>((before >> 10) & 1023u) + __popcll(wm[1] & lower)
+                                     : n4 + n3 + static_cast<int>(before >> 20) + __popcll(wm[2] & lower);
+            s_list[at] = static_cast<uint16_t>(tid);
+            s_new[at] = fresh;
+        }
         __syncthreads();
 
         // ---- wide cells: merged list, Laplacians (gradients) from the staged planes, then the
@@ -376,52 +433,51 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
             L.n0 = 0;
             L.ne = 0;
             bool empty = false;
-            const int pl[3] = {pl0, pl1, pl2};
             const int local = tid < nwide ? s_list[tid] : 0;
             const int wy = local / TZ, wz = local - (local / TZ) * TZ;
             const int wh = (wy + DY) * HZ + wz + DZ;
             const int64_t cw = (static_cast<int64_t>(x) * NY + (y0 + wy)) * NZ + (z0 + wz);
-            const uint32_t inf0 = s_info[pl1][wh];
-            const uint32_t m0 = s_mask[pl1][wh];
+            const uint2 cell0 = s_cell[pl1][wh];
+            const uint32_t inf0 = cell0.x, m0 = cell0.y;
             const int n0 = static_cast<int>(inf0 & 15u);
-            uint32_t seen = 0u;
+            const bool go = tid < nwide;
+            uint32_t left = go ? s_new[tid] : 0u;   // grains not in the merged list yet
+            const int ne = go ? n0 + __popc(left) : 0;
 #pragma unroll
             for (int t = 0; t < kRanks; ++t)
-                if (t < n0) {
-                    lid[t] = static_cast<int>((inf0 >> (kInfoOrd + 5 * t)) & 31u);
-                    seen |= 1u << lid[t];
-                }
+                if (t < n0) lid[t] = static_cast<int>((inf0 >> (kInfoOrd + 5 * t)) & 31u);
             // merged order: own entries, then grains new to the box in stencil order (x outer,
-            // z inner), within one neighbour in its list order
-            int ne = n0;
+            // z inner), within one neighbour in its list order; a single new grain needs no search
+            int at = n0;
+            if (__any(__popc(left) > 1)) {
+#pragma unroll 1
+                for (int dx = -DX; dx <= DX; ++dx) {
+                    const int p = dx < 0 ? pl0 : (dx > 0 ? pl2 : pl1);
 #pragma unroll
-            for (int k = 0; k < 27; ++k) {
-                const int dx = k / 9 - 1, dy = (k / 3) % 3 - 1, dz = k % 3 - 1;
-                if (k == 13 || !box_in<FLAT>(A, dx, dy, dz)) continue;
-                const int p = pl[dx + 1];
-                const int hh = wh + dy * HZ + dz;
-                const uint32_t nw = s_mask[p][hh] & ~seen;
-                if (nw) {
-                    const uint32_t inf = s_info[p][hh];
-                    const int nk = static_cast<int>(inf & 15u);
+                    for (int j = 0; j < 9; ++j) {
+                        const int dy = j / 3 - 1, dz = j % 3 - 1;
+                        if (!box_in<FLAT>(A, dy, dz)) continue;
+                        const uint2 nc = s_cell[p][wh + dy * HZ + dz];
+                        const uint32_t nw = nc.y & left;
+                        if (nw) {
+                            const int nk = static_cast<int>(nc.x & 15u);
 #pragma unroll
-                    for (int q = 0; q < kRanks; ++q) {
-                        const int l = static_cast<int>((inf >> (kInfoOrd + 5 * q)) & 31u);
-                        if (q < nk && ((nw >> l) & 1u)) {
+                            for (int q = 0; q < kRanks; ++q) {
+                                const int l = static_cast<int>((nc.x >> (kInfoOrd + 5 * q)) & 31u);
+                                if (q < nk && ((nw >> l) & 1u)) {
 #pragma unroll
-                            for (int t = 0; t < K; ++t) lid[t] = t == ne ? l : lid[t];
-                            ++ne;
+                                    for (int t = 0; t < K; ++t) lid[t] = t == at ? l : lid[t];
+                                    ++at;
+                                }
+                            }
+                            left &= ~nw;
                         }
                     }
-                    seen |= nw;
                 }
-            }
-            const bool go = tid < nwide && ne <= K && ne >= 2;
-            if (tid < nwide && !go) {
-                // the deferred-cell lists by merged length: 5-6 (and fewer than 2) entries, 7-8, 9 and
-                // more
-                const int dest = ne <= 6 ? 0 : (ne <= 8 ? 1 : 2);
-                s_defer[par][atomicAdd(&s_ndefer[par], 1)] = static_cast<uint16_t>(local | (dest << 8));
+            } else if (left) {
+                const int l = __ffs(static_cast<int>(left)) - 1;
+#pragma unroll
+                for (int t = 0; t < K; ++t) lid[t] = t == at ? l : lid[t];
             }
             uint32_t bm[K], lm[K];
 #pragma unroll
@@ -430,9 +486,9 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
                 lm[t] = bm[t] - 1u;
             }
             // Laplacians (and gradients) for as many entries as the wavefront's longest list
-            if (__any(go && ne > 3)) tile_derivatives<4, K, TV, TC, GRAD, FLAT>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
-            else if (__any(go && ne > 2)) tile_derivatives<3, K, TV, TC, GRAD, FLAT>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
-            else if (__any(go)) tile_derivatives<2, K, TV, TC, GRAD, FLAT>(A, s_mask, s_val, &s_zero, pl, wh, HZ, bm, lm, L);
+            if (__any(go && ne > 3)) tile_derivatives<4, K, TV, TC, GRAD, FLAT>(A, s_cell, s_val, &s_zero, pl0, pl1, pl2, wh, HZ, bm, lm, L);
+            else if (__any(go && ne > 2)) tile_derivatives<3, K, TV, TC, GRAD, FLAT>(A, s_cell, s_val, &s_zero, pl0, pl1, pl2, wh, HZ, bm, lm, L);
+            else if (__any(go)) tile_derivatives<2, K, TV, TC, GRAD, FLAT>(A, s_cell, s_val, &s_zero, pl0, pl1, pl2, wh, HZ, bm, lm, L);
             if (GRAD && FLAT) {
                 // the plane's axes are x and the grid's second active one
 #pragma unroll
