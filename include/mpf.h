@@ -307,7 +307,7 @@ void mpf_ensemble_destroy(mpf_ensemble* ens);
  * the context's own state is not touched, its grain records (Volume, VolumeRatio, ...) become
  * those of the output state. The step's scratch (deferred-cell work lists, volume accumulators,
  * status words) is one static device array per GPU, cleared at the start of every call: at most
- * 2^19 cells per call (MPF_ERR_UNSUPPORTED beyond, and with driving-force averaging), 8 MiB per
+ * 2^19 cells per call (MPF_ERR_UNSUPPORTED beyond, and with driving-force averaging), 4 MiB per
  * GPU held until the process ends. Calls that overlap on one GPU (other threads, other streams)
  * race on that array. Synchronises on the context's stream and returns the step's status. */
 mpf_status mpf_step_into(mpf_ctx* ctx, double dt, const void* count_in, const void* index_in, const void* value_in,

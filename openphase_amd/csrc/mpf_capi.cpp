@@ -345,7 +345,7 @@ unsigned grain_blocks(const mpf_ctx* c)
 // per round of four cells while up to an eighth of the cells are deferred.
 int deferred_blocks(const mpf_ctx* c)
 {
-    return static_cast<int>(std::min<int64_t>(c->deferred_grid, (c->ncells + 31) / 32));
+    return static_cast<int>(std::min<int64_t>(c->deferred_grid, (c->ncells + 255) / 256 * 8));
 }
 
 // Makes the device copies of the kernel arguments current for time step dt (both parities).
@@ -556,8 +556,9 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
         return bail(MPF_ERR_UNSUPPORTED, "at most 2^28 - 1 cells per device (e.g. 645^3)");
     c->slots = grid->slots;
     c->fp32 = grid->precision == MPF_FP32;
-    // deferred-cell grid: 16384 wavefronts from 4M cells on, 4096 below
-    c->deferred_grid = c->ncells >= (int64_t{1} << 22) ? 4 * mpf::kWideGrid : mpf::kWideGrid;
+    // twice the wavefronts that fit the chip at a time (256^3 FP64: 2.21 ms at 1024 wavefronts, 1.19 at
+    // 4096, 1.07 at 6144, 1.14 at 8192, 1.33 at 16384)
+    c->deferred_grid = mpf::kWideGrid;
     c->nphases = params->nphases;
     const size_t np2 = static_cast<size_t>(c->nphases) * c->nphases;
     c->sigma.assign(params->sigma, params->sigma + np2);
@@ -674,7 +675,7 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
         c->hip(dalloc(&c->d_dgmode_off, np2), "tables") ||
         c->hip(dalloc(&c->d_status, mpf::kStatusWords), "status") ||
         c->hip(dalloc(&c->d_first_overflow, 1), "status") || c->hip(dalloc(&c->d_warnings, 1), "status") ||
-        c->hip(dalloc(&c->d_work_list, 3 * N), "work list") || c->hip(dalloc(&c->d_work_count, 4), "work list") ||
+        c->hip(dalloc(&c->d_work_list, N), "work list") || c->hip(dalloc(&c->d_work_count, 3), "work list") ||
         c->hip(dalloc(&c->d_stats, 2), "statistics") || c->hip(dalloc(&c->d_obs, 4), "statistics"))
         return bail(MPF_ERR_NOMEM, c->err.c_str());
     if (c->reg_active && c->reg_average) {
@@ -707,8 +708,8 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
     h2d(e, c->d_status, zeros, mpf::kStatusWords);
     h2d(e, c->d_first_overflow, &none, 1);
     h2d(e, c->d_warnings, &zero, 1);
-    const unsigned zero_u[4] = {0u, 0u, 0u, 0u};
-    h2d(e, c->d_work_count, zero_u, 4);
+    const unsigned zero_u[3] = {0u, 0u, 0u};
+    h2d(e, c->d_work_count, zero_u, 3);
     const unsigned long long zero_s[4] = {0ull, 0ull, 0ull, 0ull};
     h2d(e, c->d_stats, zero_s, 2);
     h2d(e, c->d_obs, zero_s, 4);
@@ -1494,7 +1495,7 @@ mpf_status mpf_autotune(mpf_ctx* c, double dt, int32_t steps, int32_t* xcd_order
         c->tile_z = best_tz;
     }
     // 2. block order of the step kernel x grid of the deferred-cell kernel
-    const int grids[4] = {256, 1024, mpf::kWideGrid, 4 * mpf::kWideGrid};
+    const int grids[4] = {256, 1024, 4096, 16384};
     best = 1e30f;
     int best_x = x0, best_g = g0;
     for (int x = 0; x < 2 && !st; ++x)
@@ -1818,14 +1819,14 @@ constexpr size_t align256(size_t x) { return (x + 255) & ~size_t{255}; }
 constexpr size_t kOffStepArgs = 0;
 constexpr size_t kOffGrainArgs = align256(kOffStepArgs + sizeof(mpf::StepArgs));
 constexpr size_t kOffFirst = align256(kOffGrainArgs + sizeof(mpf::GrainArgs));      // 2 x uint32
-constexpr size_t kOffCount = align256(kOffFirst + 2 * sizeof(uint32_t));            // 4 x uint32
-constexpr size_t kOffStatus = align256(kOffCount + 4 * sizeof(unsigned));           // 4 x int32
+constexpr size_t kOffCount = align256(kOffFirst + 2 * sizeof(uint32_t));            // 3 x uint32
+constexpr size_t kOffStatus = align256(kOffCount + 3 * sizeof(unsigned));           // 4 x int32
 constexpr size_t kOffWords = align256(kOffStatus + mpf::kStatusWords * sizeof(int32_t));  // 8 x u64
 constexpr size_t kOffAcc = align256(kOffWords + 8 * sizeof(unsigned long long));
 constexpr size_t kOffList = align256(kOffAcc + size_t{kScratchGrains} * mpf::kLimbs * sizeof(unsigned long long));
-constexpr size_t kScratchBytes = align256(kOffList + 3 * size_t{kScratchCells} * sizeof(uint32_t));
+constexpr size_t kScratchBytes = align256(kOffList + size_t{kScratchCells} * sizeof(uint32_t));
 
-// 8 MiB + 2.2 KiB per GPU
+// 4 MiB + 2.2 KiB per GPU
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -1868,7 +1869,7 @@ __global__ void scratch_setup_kernel(unsigned char* base, int32_t ngrains, mpf::
         auto* cnt = reinterpret_cast<unsigned*>(base + kOffCount);
         auto* st = reinterpret_cast<int32_t*>(base + kOffStatus);
         auto* w = reinterpret_cast<unsigned long long*>(base + kOffWords);
-        for (int i = 0; i < 4; ++i) cnt[i] = 0u;
+        for (int i = 0; i < 3; ++i) cnt[i] = 0u;
         for (int i = 0; i < mpf::kStatusWords; ++i) st[i] = 0;
         w[0] = ~0ull;                       // first overflowing cell: none
         for (int i = 1; i < 8; ++i) w[i] = 0ull;  // warnings, IP.Set maxima (4), statistics (2)

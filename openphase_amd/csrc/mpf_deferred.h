@@ -12,9 +12,10 @@
 // Lists are held in LDS with run-time lengths, so one kernel takes every length: a cell of more
 // than kGroupCap merged entries, or next to a list of more than kGroupCap, is done again by the
 // whole wavefront with room for kWideSlots. Measured against one thread per cell with register
-// lists in three launches (2-6, 7-10 and up to 16 entries), mid-run states, FP64: 20 us instead of
-// 114 at 2D 512^2 and 22 instead of 120 at 96^2 (a few hundred cells that waited on their own
-// latency), 1.56 ms instead of 2.62 at 256^3; 64 FP32 domains in one launch 84 us instead of 354.
+// lists in three launches (2-6, 7-10 and up to 16 entries), mid-run states, FP64: 16 us instead of
+// 114 at 2D 512^2 and 18 instead of 120 at 96^2 (a few hundred cells that waited on their own
+// latency), 1.07 ms instead of 2.62 at 256^3; 64 FP32 domains in one launch 60 us instead of 354.
+// Three wavefronts per SIMD: four spill (256^3: 1.44 ms FP64, 1.58 FP32 where three took 1.41, 1.42).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -78,7 +79,7 @@ __device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t 
     double phi = L.phi;
     const bool go = run && !L.over;          // the cell's result is written by this call
     const bool work = go && L.wide;
-    if (work && ne > 6 && count_long && l == 0) atomicAdd(&A.work_count[3], 1u);
+    if (work && ne > 6 && count_long && l == 0) atomicAdd(&A.work_count[2], 1u);
     const int top = wave_max<G>(work ? ne : 0);
     double vr = 0.0;
     int ph = 0;
@@ -191,7 +192,9 @@ __device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t 
     }
     __syncthreads();
 
-    // ---- limiter (FP64). A pair the reference drops from the increment list holds 0 here
+    // ---- limiter (FP64): lane t holds the increments psi of (t, u) in registers, 0 where there is
+    // none (the reference drops such a pair from the increment list; adding 0 changes no sum). Both
+    // lanes of a pair scale it by the same factors, so the two stay exact negatives
     const double dt = A.dt;
     if (work && ne == 2 && l == 0) {
         double d = M.p.psi[0][1];
@@ -210,66 +213,57 @@ __device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t 
         M.p.psi[0][1] = d;
         M.p.psi[1][0] = -d;
     }
+    __syncthreads();
+    double psi[CAP];
+#pragma unroll
+    for (int u = 0; u < CAP; ++u) psi[u] = work && l < ne && u < ne && u != l ? M.p.psi[l][u] : 0.0;
     const bool many = work && ne > 2;
     if (__any(many)) {
         // zero the pairs that would push a field at 0 below or at 1 above, entry after entry
         int done = -1;
         while (true) {
-            bool stop = false;
-            if (many && l < ne && l > done) {
-                double dpsi = 0.0;
-                for (int u = 0; u < ne; ++u)
-                    if (u != l) dpsi += M.p.psi[l][u];
-                stop = (phi == 0.0 && dpsi < 0.0) || (phi == 1.0 && dpsi > 0.0);
-            }
+            double dpsi = 0.0;
+#pragma unroll
+            for (int u = 0; u < CAP; ++u) dpsi += psi[u];
+            const bool stop = many && l < ne && l > done && ((phi == 0.0 && dpsi < 0.0) || (phi == 1.0 && dpsi > 0.0));
             const unsigned long long b = group_bits<G>(__ballot(stop));
             if (!__any(stop)) break;
-            __syncthreads();
             if (b) {
                 done = __ffsll(static_cast<long long>(b)) - 1;
-                if (l < ne && l != done) {
-                    M.p.psi[l][done] = 0.0;
-                    M.p.psi[done][l] = 0.0;
-                }
+#pragma unroll
+                for (int u = 0; u < CAP; ++u) psi[u] = u == done || l == done ? 0.0 : psi[u];
             }
-            __syncthreads();
         }
         bool needed = many;
         for (int iter = 1; iter <= 25 && __any(needed); ++iter) {
+            double pos = 0.0, neg = 0.0;
+#pragma unroll
+            for (int u = 0; u < CAP; ++u) {
+                pos += fmax(psi[u], 0.0);
+                neg += fmin(psi[u], 0.0);
+            }
+            double lim1 = 1.0, lim2 = 1.0;
             if (needed && l < ne) {
-                double pos = 0.0, neg = 0.0;
-                for (int u = 0; u < ne; ++u) {
-                    if (u == l) continue;
-                    const double x = M.p.psi[l][u];
-                    if (x < 0.0) neg += x;
-                    if (x > 0.0) pos += x;
-                }
-                double lim1 = 1.0, lim2 = 1.0;
                 const double npf = phi + (pos + neg) * dt;
                 if (npf < 0.0) lim2 = smin(lim2, -(phi + pos * dt) / (neg * dt));
                 if (npf > 1.0) lim1 = smin(lim1, (1.0 - (phi + neg * dt)) / (pos * dt));
+            }
+            // factors of 1 all over leave every increment as it is
+            needed = needed && group_bits<G>(__ballot(lim1 < 1.0 || lim2 < 1.0)) != 0ull;
+            if (!__any(needed)) break;
+            if (l < CAP) {
                 M.lim1[l] = lim1;
                 M.lim2[l] = lim2;
             }
             __syncthreads();
             bool again = false;
-            for (int p0 = 0; p0 < ptop; p0 += G) {
-                const int p = p0 + l;
-                if (needed && p < np) {
-                    const int a = pairs[p] & 255, b = pairs[p] >> 8;
-                    double x = M.p.psi[a][b];
-                    if (x < 0.0) {
-                        const double t = smin(M.lim2[a], M.lim1[b]);
-                        x *= t;
-                        if (t < 1.0) again = true;
-                    }
-                    if (x > 0.0) {
-                        const double t = smin(M.lim1[a], M.lim2[b]);
-                        x *= t;
-                        if (t < 1.0) again = true;
-                    }
-                    M.p.psi[a][b] = x;
-                    M.p.psi[b][a] = -x;
+            if (needed && l < ne) {
+#pragma unroll
+                for (int u = 0; u < CAP; ++u) {
+                    // (a negative increment: entry l loses, u gains)
+                    const double t = psi[u] < 0.0 ? smin(lim2, M.lim1[u]) : smin(lim1, M.lim2[u]);
+                    again = again || (psi[u] != 0.0 && t < 1.0);
+                    psi[u] = psi[u] != 0.0 ? psi[u] * t : 0.0;
                 }
             }
             needed = needed && group_bits<G>(__ballot(again)) != 0ull;
@@ -278,24 +272,19 @@ __device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t 
         // plausibility check of the limited increments (warning count)
         if (many && l < ne) {
             double tv = phi;
-            for (int u = 0; u < ne; ++u) {
-                if (u == l) continue;
-                const double x = M.p.psi[l][u];
-                if (x == 0.0 || fabs(x * dt) < DBL_EPSILON) continue;
-                tv += x * dt;
-            }
+#pragma unroll
+            for (int u = 0; u < CAP; ++u) tv += fabs(psi[u] * dt) < DBL_EPSILON ? 0.0 : psi[u] * dt;
             if (tv < -FLT_EPSILON || tv > 1.0 + FLT_EPSILON) atomicAdd(A.warnings, 1ull);
         }
     }
-    __syncthreads();
 
     // ---- merge, then finalize (NodePF::finalize); a bulk cell keeps its list
     bool keep = go && l < ne;
     if (work && l < ne) {
-        for (int u = 0; u < ne; ++u) {
-            if (u == l) continue;
-            const double value = M.p.psi[l][u] * dt;
-            if (fabs(value) >= DBL_EPSILON) phi += value;
+#pragma unroll
+        for (int u = 0; u < CAP; ++u) {
+            const double value = psi[u] * dt;
+            phi += fabs(value) >= DBL_EPSILON ? value : 0.0;
         }
         if (phi >= 1.0 - DBL_EPSILON) phi = 1.0;
         if (phi <= 0.0 + DBL_EPSILON) { phi = 0.0; keep = false; }
@@ -351,10 +340,9 @@ __device__ __forceinline__ bool group_cell(const StepArgs& A, bool run, int64_t 
     return run && L.over;
 }
 
-// One wavefront per block; wavefront i of a domain takes the i-th part of its deferred cells (the
-// concatenated lists), neighbours in the list being neighbours in the grid.
+// One wavefront per block; neighbours in a domain's list of deferred cells are neighbours in the grid.
 template <typename TV, typename TC, bool GRAD, bool DG>
-__global__ __launch_bounds__(64) void deferred_kernel(const StepArgs* __restrict__ batch, int32_t ndom)
+__global__ __launch_bounds__(64, 3) void deferred_kernel(const StepArgs* __restrict__ batch, int32_t ndom)
 {
     constexpr int G = kGroupLanes, C = 64 / G;
     __shared__ GroupArena<TC, GRAD> mem;
@@ -363,13 +351,17 @@ __global__ __launch_bounds__(64) void deferred_kernel(const StepArgs* __restrict
     const unsigned per = gridDim.x / static_cast<unsigned>(ndom);
     const unsigned dom = blockIdx.x / per, part = blockIdx.x - dom * per;
     const StepArgs& A = batch[dom];
-    const unsigned n0 = A.work_count[0], n1 = A.work_count[1], n2 = A.work_count[2];
-    const unsigned n = n0 + n1 + n2;
+    const unsigned n = A.work_count[0];
     if (n == 0u) return;
-    // whole rounds of C cells per wavefront
-    const unsigned rounds = (n + C - 1) / C, chunk = (rounds + per - 1) / per * C;
-    const unsigned begin = min(n, part * chunk), end = min(n, begin + chunk);
-    if (begin >= end) return;
+    // Runs of up to four rounds of C cells. Blocks go to the eight XCDs in turn; each XCD takes one
+    // eighth of the list and its wavefronts take that part's runs in turn, so that what is worked on
+    // at a time is one stretch of the list, whose neighbourhoods overlap in the XCD's L2 (256^3 FP64,
+    // 750,000 cells: 0.81 instead of 2.7 GB from memory, 1.07 instead of 1.41 ms)
+    const unsigned rounds = (n + C - 1) / C, length = min(4u, max(1u, rounds / per)), runs = (rounds + length - 1) / length;
+    const unsigned xcds = per % 8u == 0u ? 8u : 1u, xcd = part % xcds;
+    const unsigned last = static_cast<unsigned>(static_cast<uint64_t>(runs) * (xcd + 1u) / xcds);
+    unsigned turn = static_cast<unsigned>(static_cast<uint64_t>(runs) * xcd / xcds) + part / xcds;
+    if (turn >= last) return;
     const int lane = static_cast<int>(threadIdx.x);
     fill_pairs(pairs);
     if (lane < kVolSlots) V.key[lane] = -1;
@@ -377,39 +369,44 @@ __global__ __launch_bounds__(64) void deferred_kernel(const StepArgs* __restrict
     __syncthreads();
     double emax = 0.0, mmax = 0.0;
     bool bad = false;
-    auto cell_of = [&](unsigned i) -> int64_t {
-        if (i < n0) return A.work_list[i];
-        if (i < n0 + n1) return A.work_list[A.ncells + (i - n0)];
-        return A.work_list[2 * A.ncells + (i - n0 - n1)];
-    };
-    for (unsigned base = begin; base < end; base += C) {
-        const unsigned i = base + static_cast<unsigned>(lane / G);
-        const bool run = i < end;
-        const int64_t c = run ? cell_of(i) : 0;
-        const bool big = group_cell<TV, TC, GRAD, DG, G, kGroupCap>(A, run, c, mem.cell[lane / G], i < n0, pairs, V, emax,
-                                                                    mmax, bad);
-        unsigned long long todo = __ballot(big && (lane & (G - 1)) == 0);
-        __syncthreads();
-        while (todo) {
-            const int from = __ffsll(static_cast<long long>(todo)) - 1;
-            todo &= todo - 1ull;
-            const int64_t cb = static_cast<int64_t>(__shfl(static_cast<int>(c), from));
-            const bool first = base + static_cast<unsigned>(from / G) < n0;
-            if (group_cell<TV, TC, GRAD, DG, 64, kWideSlots>(A, true, cb, mem.one, first, pairs, V, emax, mmax, bad) &&
-                lane == 0) {
-                atomicOr(&A.status[kStatusOverflow], 1);
-                atomicMin(A.first_overflow, static_cast<unsigned long long>(cb));
-            }
+    for (; turn < last; turn += per / xcds) {
+        const unsigned begin = turn * length * C, end = min(n, begin + length * C);
+        for (unsigned base = begin; base < end; base += C) {
+            const unsigned i = base + static_cast<unsigned>(lane / G);
+            const bool run = i < end;
+            const uint32_t entry = run ? A.work_list[i] : 0u;
+            const int64_t c = entry & ~(1u << 31);
+            const bool uncounted = (entry >> 31) == 0u;   // as more than six merged entries
+            const bool big = group_cell<TV, TC, GRAD, DG, G, kGroupCap>(A, run, c, mem.cell[lane / G], uncounted, pairs, V, emax,
+                                                                        mmax, bad);
+            unsigned long long todo = __ballot(big && (lane & (G - 1)) == 0);
             __syncthreads();
+            while (todo) {
+                const int from = next_long(todo);
+                const int64_t cb = static_cast<int64_t>(__shfl(static_cast<int>(c), from));
+                const bool first = __shfl(uncounted ? 1 : 0, from) != 0;
+                if (group_cell<TV, TC, GRAD, DG, kLongLanes, kWideSlots>(A, true, cb, mem.longer[lane / kLongLanes], first, pairs,
+                                                                         V, emax, mmax, bad) &&
+                    (lane & (kLongLanes - 1)) == 0) {
+                    atomicOr(&A.status[kStatusOverflow], 1);
+                    atomicMin(A.first_overflow, static_cast<unsigned long long>(cb));
+                }
+                __syncthreads();
+            }
         }
+        // the run's volumes; another run's grains are others
+        for (int i = lane; i < kVolSlots * kLimbs; i += 64) {
+            const int s = i / kLimbs;
+            const unsigned long long x = V.acc[s][i - s * kLimbs];
+            if (x) atomicAdd(&A.vol_acc[static_cast<int64_t>(V.key[s]) * kLimbs + (i - s * kLimbs)], x);
+            V.acc[s][i - s * kLimbs] = 0ull;
+        }
+        __syncthreads();
+        if (lane < kVolSlots) V.key[lane] = -1;
+        __syncthreads();
     }
     note_maxima(A.obs, emax, mmax);
     if (__any(bad) && lane == 0) atomicOr(&A.status[kStatusVolumeRange], 1);
-    for (int i = lane; i < kVolSlots * kLimbs; i += 64) {
-        const int s = i / kLimbs;
-        const unsigned long long x = V.acc[s][i - s * kLimbs];
-        if (x) atomicAdd(&A.vol_acc[static_cast<int64_t>(V.key[s]) * kLimbs + (i - s * kLimbs)], x);
-    }
 }
 
 }  // namespace

@@ -7,7 +7,7 @@ namespace mpf {
 
 constexpr int kMaxSlots = 16;                        // largest per-cell list capacity of the stored state
 constexpr int kBlock = 256;                          // threads per block of the step kernels
-constexpr int kWideGrid = 4096;                      // blocks (wavefronts) of the deferred-cell kernel
+constexpr int kWideGrid = 6144;                      // blocks (wavefronts) of the deferred-cell kernel
 constexpr int kLimbs = 4;                            // 32-bit limbs of the exact per-grain volume sums
 
 // Device status words (one int each).
@@ -73,9 +73,9 @@ struct StepArgs {
     // largest interface energy and mobility of the pairs this step's IP.Set evaluates (FP64 bit
     // patterns of non-negative values, atomicMax): InterfaceProperties maxEnergies/maxMobilities
     unsigned long long* obs;
-    uint32_t* work_list;         // deferred cells: three lists of ncells each, by merged length where it is
-                                 // known (up to 6 or unknown; 7-8; more)
-    unsigned* work_count;        // [4] their lengths, and the cells of list 0 that have more than 6 entries
+    uint32_t* work_list;         // [ncells] deferred cells; bit 31: known to merge more than six entries
+    unsigned* work_count;        // [3] its length, how many of them have bit 31, and how many others turned
+                                 // out to merge more than six
     // launch shape (chosen by mpf_autotune): XCD-contiguous block order of the step kernel, and
     // the number of blocks of the deferred-cell kernel
     int32_t xcd_order;
@@ -94,8 +94,8 @@ struct GrainArgs {
     double* vr;
     uint8_t* exist;
     int32_t* stage;              // 0 seed, 1 nucleus, 2 stable
-    unsigned* work_count;        // [4], reset here for the next step
-    unsigned long long* stats;   // [2] cumulative lengths of work lists 0 and 1
+    unsigned* work_count;        // [3], reset here for the next step
+    unsigned long long* stats;   // [2] cumulative deferred cells not known to be long, and long ones
     unsigned long long* obs;     // [4] this step's maxima (StepArgs::obs, cleared here) and the last step's
 };
 

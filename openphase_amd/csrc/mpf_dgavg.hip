@@ -284,9 +284,8 @@ __global__ __launch_bounds__(64) void curvature_raw_kernel(const CurvArgs P)
         const bool big = raw_cell<GRAD, G, kGroupCap>(P, run, base + (run ? s_list[i] : 0), mem.cell[lane / G], pairs);
         unsigned long long todo = __ballot(big && (lane & (G - 1)) == 0);
         while (todo) {
-            const int from = __ffsll(static_cast<long long>(todo)) - 1;
-            todo &= todo - 1ull;
-            (void)raw_cell<GRAD, 64, kWideSlots>(P, true, base + s_list[i0 + from / G], mem.one, pairs);
+            const int from = next_long(todo);
+            (void)raw_cell<GRAD, kLongLanes, kWideSlots>(P, true, base + s_list[i0 + from / G], mem.longer[lane / kLongLanes], pairs);
         }
     }
 }

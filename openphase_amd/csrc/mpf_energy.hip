@@ -190,12 +190,12 @@ __global__ __launch_bounds__(64) void energy_kernel(const EnergyArgs E)
                                                   pairs, over);
         unsigned long long todo = __ballot(over && (lane & (G - 1)) == 0);
         while (todo) {
-            const int from = __ffsll(static_cast<long long>(todo)) - 1;
-            todo &= todo - 1ull;
+            const int from = next_long(todo);
             const int64_t cb = base + s_list[i0 + from / G];
             bool none = false;
-            e += group_energy<TV, FULL, 64, kWideSlots>(E, B, true, cb, mem.one, FULL ? &old->one : nullptr, pairs, none);
-            if (none && lane == 0) atomicOr(E.status, 1);
+            e += group_energy<TV, FULL, kLongLanes, kWideSlots>(E, B, true, cb, mem.longer[lane / kLongLanes],
+                                                                FULL ? &old->longer[lane / kLongLanes] : nullptr, pairs, none);
+            if (none && (lane & (kLongLanes - 1)) == 0) atomicOr(E.status, 1);
         }
     }
 #pragma unroll

@@ -19,6 +19,7 @@ namespace {
 
 constexpr int kGroupLanes = 16;  // lanes per cell
 constexpr int kGroupCap = 8;     // merged entries a group has room for
+constexpr int kLongLanes = 64;   // lanes of a cell of more (up to kWideSlots)
 
 // One cell's list and tables in LDS.
 template <typename TC, bool GRAD, int CAP> struct GroupMem {
@@ -114,17 +115,15 @@ __device__ __forceinline__ GroupList<TC> group_gather(const StepArgs& A, bool ru
     for (int k = 1; k < 64; k <<= 1) mtop = max(mtop, __shfl_xor(mtop, k));
     const int qtop = min(__builtin_amdgcn_readfirstlane(mtop), RQ);
 
-    // ---- lists of the lane's neighbours, and entry l of the own list
-    uint32_t g[NK][RQ];
+    // ---- lists of the lane's neighbours, and entry l of the own list. An entry that is not there, or
+    // holds no value, or is in the merged list already, is grain -1
+    int32_t g[NK][RQ];
     TV v[NK][RQ];
-    uint32_t left[NK];   // entries not in the merged list yet (bit q)
-#pragma unroll
-    for (int j = 0; j < NK; ++j) left[j] = 0u;
 #pragma unroll
     for (int q = 0; q < RQ; ++q) {
         if (q >= 2 && q >= qtop) {
 #pragma unroll
-            for (int j = 0; j < NK; ++j) { g[j][q] = 0u; v[j][q] = TV(0); }
+            for (int j = 0; j < NK; ++j) { g[j][q] = -1; v[j][q] = TV(0); }
             continue;
         }
         // slot 0 of the cell in place of a slot it does not use: no branch between the loads
@@ -141,14 +140,17 @@ __device__ __forceinline__ GroupList<TC> group_gather(const StepArgs& A, bool ru
         eid = A.id_in[static_cast<int64_t>(l) * N + cc];
         if (!(IMPL && l == imp0)) phi = static_cast<double>(load_val<TV>(A.val_in, static_cast<int64_t>(l) * N + cc));
     }
+    const bool look = wide && !over;
 #pragma unroll
-    for (int j = 0; j < NK; ++j)
+    for (int q = 0; q < RQ; ++q) {
+        if (q >= 2 && q >= qtop) continue;
 #pragma unroll
-        for (int q = 0; q < RQ; ++q) {
+        for (int j = 0; j < NK; ++j) {
             // a lone implicit entry (FP32) has no stored value: it is 1
             if (IMPL && q == 0 && m[j] == 1 && ListCode<TV>::implicit(code[j]) == 0) v[j][q] = TV(1);
-            if (q < m[j] && v[j][q] != TV(0)) left[j] |= 1u << q;
+            if (!look || q >= m[j] || v[j][q] == TV(0)) g[j][q] = -1;
         }
+    }
     if (l < CAP) { M.phi[l] = phi; M.eid[l] = eid; }
     __syncthreads();
     if (IMPL) {
@@ -165,53 +167,64 @@ __device__ __forceinline__ GroupList<TC> group_gather(const StepArgs& A, bool ru
     // ---- merged list: the own entries, then grains new to the box in stencil order. Row t of
     // M.a: the value of entry t at every box position
     int ne = over ? 0 : n0;
-    if (!wide || over) {
+    auto row = [&](int t, int32_t gid, bool on) {
+        TC a[NK];
 #pragma unroll
-        for (int j = 0; j < NK; ++j) left[j] = 0u;
-    }
-    auto row = [&](int t, uint32_t gid, bool on) {
+        for (int j = 0; j < NK; ++j) a[j] = TC(0);
+#pragma unroll
+        for (int q = 0; q < RQ; ++q) {
+            if (q >= 2 && q >= qtop) continue;
+#pragma unroll
+            for (int j = 0; j < NK; ++j) {
+                const bool hit = g[j][q] == gid;
+                a[j] = hit ? static_cast<TC>(v[j][q]) : a[j];
+                g[j][q] = hit ? -1 : g[j][q];
+            }
+        }
 #pragma unroll
         for (int j = 0; j < NK; ++j) {
-            TC a = TC(0);
-#pragma unroll
-            for (int q = 0; q < RQ; ++q)
-                if (((left[j] >> q) & 1u) && g[j][q] == gid && on) {
-                    a = static_cast<TC>(v[j][q]);
-                    left[j] &= ~(1u << q);
-                }
             const int k = l + j * G;
-            if (on && k < 27) M.a[t][k] = a;
+            if (on && k < 27) M.a[t][k] = a[j];
         }
     };
-    const int own_top = wave_max<G>(wide ? ne : 0);
-    for (int t = 0; t < own_top; ++t) row(t, M.eid[t], wide && t < ne);
+    const int own_top = wave_max<G>(look ? ne : 0);
+    for (int t = 0; t < own_top; ++t) {
+        const bool on = look && t < ne;
+        row(t, on ? static_cast<int32_t>(M.eid[t]) : -2, on);
+    }
     while (true) {
-        uint32_t cand = 0u;
+        // the first grain left, in stencil order then list order
+        int32_t cand = -1;
         unsigned long long who = 0ull;
 #pragma unroll
         for (int j = NK - 1; j >= 0; --j) {
-            const unsigned long long b = group_bits<G>(__ballot(left[j] != 0u));
+            int32_t next = -1;
+#pragma unroll
+            for (int q = RQ - 1; q >= 0; --q) {
+                if (q >= 2 && q >= qtop) continue;
+                next = g[j][q] >= 0 ? g[j][q] : next;
+            }
+            const unsigned long long b = group_bits<G>(__ballot(next >= 0));
             if (b) {
                 who = b;
-                const int q = __ffs(static_cast<int>(left[j])) - 1;
-                cand = 0u;
-#pragma unroll
-                for (int r = 0; r < RQ; ++r) cand = r == q ? g[j][r] : cand;
+                cand = next;
             }
         }
         if (!__any(who != 0ull)) break;
         const int leader = who ? __ffsll(static_cast<long long>(who)) - 1 : 0;
-        const uint32_t gid = static_cast<uint32_t>(__shfl(static_cast<int>(cand), (lane & ~(G - 1)) + leader));
+        const int32_t gid = __shfl(cand, (lane & ~(G - 1)) + leader);
         bool on = who != 0ull;
         if (on && ne >= CAP) {
             over = true;
             on = false;
 #pragma unroll
-            for (int j = 0; j < NK; ++j) left[j] = 0u;
+            for (int q = 0; q < RQ; ++q)
+#pragma unroll
+                for (int j = 0; j < NK; ++j) g[j][q] = -1;
         }
-        row(ne, gid, on);
+        row(ne, on ? gid : -2, on);
         if (on) {
-            if (l == ne) eid = gid;
+            if (l == ne) eid = static_cast<uint32_t>(gid);
             ++ne;
         }
     }
@@ -240,13 +253,22 @@ __device__ __forceinline__ GroupList<TC> group_gather(const StepArgs& A, bool ru
     return GroupList<TC>{n0, ne, wide, over, eid, phi, lap, gx, gy, gz};
 }
 
-// The groups' memory of one wavefront, or the whole wavefront's for one long list.
+// The groups' memory of one wavefront: four cells, or one of a longer list
 template <typename TC, bool GRAD> union GroupArena {
     GroupMem<TC, GRAD, kGroupCap> cell[64 / kGroupLanes];
-    GroupMem<TC, GRAD, kWideSlots> one;
+    GroupMem<TC, GRAD, kWideSlots> longer[64 / kLongLanes];
 };
 
 constexpr int kPairTable = kWideSlots * (kWideSlots - 1) / 2;
+
+// The next cell of a wavefront's groups whose bit (at the group's first lane) is set in `todo`: that
+// lane.
+__device__ __forceinline__ int next_long(unsigned long long& todo)
+{
+    const int from = __ffsll(static_cast<long long>(todo)) - 1;
+    todo &= todo - 1ull;
+    return from;
+}
 
 // Pair p = b (b - 1) / 2 + a as a | b << 8. One wavefront.
 __device__ __forceinline__ void fill_pairs(uint16_t* pairs)

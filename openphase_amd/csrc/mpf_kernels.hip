@@ -136,12 +136,11 @@ __global__ void grains_kernel(const GrainArgs* __restrict__ batch, const uint32_
     const GrainArgs& G = batch[dom];
     const int g = static_cast<int>(blockIdx.x - first[dom]) * blockDim.x + threadIdx.x;
     if (g == 0) {
-        G.stats[0] += G.work_count[0];
-        G.stats[1] += G.work_count[1] + G.work_count[2] + G.work_count[3];
+        G.stats[0] += G.work_count[0] - G.work_count[1];
+        G.stats[1] += G.work_count[1] + G.work_count[2];
         G.work_count[0] = 0u;
         G.work_count[1] = 0u;
         G.work_count[2] = 0u;
-        G.work_count[3] = 0u;
         // this step's IP.Set maxima become the reported ones; the next step starts from 0
         G.obs[2] = G.obs[0];
         G.obs[3] = G.obs[1];

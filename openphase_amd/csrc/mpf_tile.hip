@@ -194,11 +194,12 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
     __shared__ uint16_t s_list[kBlock];
     __shared__ uint32_t s_new[kBlock];
     __shared__ uint32_t s_nwide[kTileWaves];
-    // cells of a plane for the deferred-cell kernel, by plane parity: appended in LDS, moved to
-    // the global work list by wavefront 0 after the plane (one global atomic per plane)
-    // entries: tile-local cell index (y * TZ + z) | work list << 8
-    __shared__ uint16_t s_defer[2][kBlock];
-    __shared__ int s_ndefer[2];
+    // cells for the deferred-cell kernel: appended in LDS over the planes, moved to the global work
+    // list by wavefront 0 when another plane might not fit, so that a tile's cells stay together in
+    // it (their neighbourhoods overlap). Entries: tile-local cell index (y * TZ + z) | more than six
+    // merged entries << 8 | plane of the chunk, modulo 128 << 9
+    __shared__ uint16_t s_defer[2 * kBlock];
+    __shared__ int s_ndefer;
 
     constexpr int K = kMainSlots;
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
@@ -215,7 +216,7 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
     const int x0 = FLAT ? 0 : xc * TX, x1 = FLAT ? 1 : min(x0 + TX, NX);
 
     if (tid < kLocal) s_key[tid] = -1;
-    if (tid < 2) s_ndefer[tid] = 0;
+    if (tid == 0) s_ndefer = 0;
     for (int i = tid; i < kLocal * kCopies * kLimbs; i += kBlock) (&s_acc[0][0][0])[i] = 0ull;
     if (tid == 0) s_zero = TV(0);
     __syncthreads();
@@ -335,7 +336,10 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
         if (own && (FLAT || x + 1 < x1 + DX)) above = plane_union<FLAT>(A, s_cell[FLAT ? 0 : ring(x + 1)], oh, HZ);
         if (x < x0) continue;
         const int pl0 = DX ? ring(x - 1) : ring(x), pl1 = ring(x), pl2 = DX ? ring(x + 1) : ring(x);
-        const int par = (x - x0) & 1;
+        const uint32_t plane = static_cast<uint32_t>(x - x0) & 127u;
+        auto defer = [&](bool is_long) {
+            s_defer[atomicAdd(&s_ndefer, 1)] = static_cast<uint16_t>(static_cast<uint32_t>(tid) | (is_long ? 256u : 0u) | plane << 9);
+        };
 
         // ---- classify the tile's cells: bulk cells are copied, wide cells compacted for the
         // second phase by their merged length, cells the tile cannot hold deferred
@@ -350,26 +354,23 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
             const int n0 = static_cast<int>(inf0 & 15u);
             const uint2 box = FLAT ? above : make_uint2(below.x | here.x | above.x, below.y | here.y | above.y);
             if ((box.x >> kInfoMulti) & 1u) {
-                int dest = -1;      // the deferred-cell list of a cell the tile cannot hold
-                if (((box.x >> kInfoBad) & 1u) != 0u || n0 > K) {
-                    dest = 0;
-                } else {
+                bool hold = ((box.x >> kInfoBad) & 1u) == 0u && n0 <= K;
+                if (hold) {
                     uint32_t listed = 0u;
 #pragma unroll
                     for (int t = 0; t < kRanks; ++t)
                         if (t < n0) listed |= 1u << ((inf0 >> (kInfoOrd + 5 * t)) & 31u);
                     fresh = box.y & ~listed;
                     ne = n0 + __popc(fresh);
-                    // by merged length: 5-6 (and fewer than 2) entries, 7-8, 9 and more
-                    if (ne > K || ne < 2) dest = ne <= 6 ? 0 : (ne <= 8 ? 1 : 2);
+                    hold = ne <= K && ne >= 2;
                 }
-                if (dest >= 0) {
+                if (!hold) {
+                    defer(ne > 6);
                     ne = 0;
-                    s_defer[par][atomicAdd(&s_ndefer[par], 1)] = static_cast<uint16_t>(tid | (dest << 8));
                 }
             } else if (n0 == 1 && ((inf0 >> kInfoBad) & 1u) != 0u) {
                 // a lone entry whose grain did not fit the local ids
-                s_defer[par][atomicAdd(&s_ndefer[par], 1)] = static_cast<uint16_t>(tid);
+                defer(false);
             } else if (n0 == 1) {
                 // NodePF::finalize keeps a lone entry at 1; an FP32 list stores it implicitly
                 single = true;
@@ -542,41 +543,27 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
             mmax = smax(mmax, L.mmax);
         }
         __syncthreads();  // the next plane is staged over the ring slot of x - 1
-        if (wave == 0) {
-            // this plane's deferred cells to the global work list; the other parity's LDS list
-            // is the next plane's, this one is reused two planes on (after at least one barrier)
-            const int nd = s_ndefer[par];
-            if (nd > 0) {
-                // per list: count, reserve with one atomic, write in LDS order
-                int cnt[3] = {0, 0, 0};
-                for (int i0 = 0; i0 < nd; i0 += 64) {
-                    const int i = i0 + lane;
-                    const int d = i < nd ? (s_defer[par][i] >> 8) : 3;
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) cnt[q] += __popcll(__ballot(d == q));
-                }
-                unsigned base[3] = {0u, 0u, 0u};
-                if (lane == 0)
-#pragma unroll
-                    for (int q = 0; q < 3; ++q)
-                        if (cnt[q]) base[q] = atomicAdd(&A.work_count[q], static_cast<unsigned>(cnt[q]));
-#pragma unroll
-                for (int q = 0; q < 3; ++q) base[q] = static_cast<unsigned>(__shfl(static_cast<int>(base[q]), 0));
-                for (int i0 = 0; i0 < nd; i0 += 64) {
-                    const int i = i0 + lane;
-                    const int e = i < nd ? s_defer[par][i] : 0;
-                    const int d = i < nd ? (e >> 8) : 3, l = e & 255;
-                    const int dy = l / TZ, dz = l - (l / TZ) * TZ;
-                    const uint32_t cellv = static_cast<uint32_t>((static_cast<int64_t>(x) * NY + (y0 + dy)) * NZ + (z0 + dz));
-#pragma unroll
-                    for (int q = 0; q < 3; ++q) {
-                        const unsigned long long m = __ballot(d == q);
-                        if (d == q)
-                            A.work_list[static_cast<int64_t>(q) * N + base[q] + __popcll(m & ((1ull << lane) - 1ull))] = cellv;
-                        base[q] += static_cast<unsigned>(__popcll(m));
-                    }
-                }
-                if (lane == 0) s_ndefer[par] = 0;
+        if (wave == 0 && (s_ndefer > kBlock || plane == 127u || x + 1 == x1)) {
+            // (the other wavefronts append again only after the next barrier)
+            const int nd = s_ndefer;
+            int nlong = 0;
+            for (int i0 = 0; i0 < nd; i0 += 64) {
+                const int i = i0 + lane;
+                nlong += __popcll(__ballot(i < nd && ((s_defer[i < nd ? i : 0] >> 8) & 1) != 0));
+            }
+            unsigned base = 0u;
+            if (lane == 0) {
+                if (nd) base = atomicAdd(&A.work_count[0], static_cast<unsigned>(nd));
+                if (nlong) atomicAdd(&A.work_count[1], static_cast<unsigned>(nlong));
+                s_ndefer = 0;
+            }
+            base = static_cast<unsigned>(__shfl(static_cast<int>(base), 0));
+            const int xbase = x - static_cast<int>(plane);
+            for (int i = lane; i < nd; i += 64) {
+                const uint32_t e = s_defer[i];
+                const int l = static_cast<int>(e & 255u), dy = l / TZ, dz = l - (l / TZ) * TZ, xe = xbase + static_cast<int>(e >> 9);
+                A.work_list[base + i] = static_cast<uint32_t>((static_cast<int64_t>(xe) * NY + (y0 + dy)) * NZ + (z0 + dz)) |
+                                        (((e >> 8) & 1u) << 31);
             }
         }
     }
