@@ -215,21 +215,37 @@ MPF_HD __forceinline__ void part2(double dt, double (&psi)[NPairs<C>::value], co
 
 MPF_HD inline void gadd(double* g, int e, double v) { g[e] += v; }
 
-// Cotangent of the next state's value of grain g at cell c: by grain through S_{t+1}'s list, or
-// (no list given) by the position w among the entries the step keeps.
-MPF_HD inline double lam_of(const AdjointArgs& J, bool fp32, int64_t c, uint32_t g, int w)
-{
-    const StepArgs& A = J.s;
-    const int64_t N = A.ncells;
-    if (J.next_cnt != nullptr) {
-        const uint8_t b = J.next_cnt[c];
-        const int n = fp32 ? (b & 15) : b;
-        for (int s = 0; s < n; ++s)
-            if (J.next_id[static_cast<int64_t>(s) * N + c] == g) return J.lam_next[static_cast<int64_t>(s) * N + c];
-        return 0.0;
+// Where the entries of cell c are in S_{t+1}'s list, whose cotangents lam_next holds: its first four
+// grains are read at once (the lists are short), longer ones searched. Without a list (next_cnt
+// null) the w-th entry the step keeps is its entry w.
+struct NextList {
+    int n;
+    uint32_t id[4];
+    MPF_HD NextList(const AdjointArgs& J, bool fp32, int64_t c) : n(0)
+    {
+        const uint8_t b = J.next_cnt != nullptr ? J.next_cnt[c] : 0;
+        n = fp32 ? (b & 15) : b;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            id[s] = J.next_cnt != nullptr ? J.next_id[(s < n ? static_cast<int64_t>(s) * J.s.ncells : 0) + c] : 0u;
     }
-    return w < A.slots ? J.lam_next[static_cast<int64_t>(w) * N + c] : 0.0;
-}
+    // Slot of grain g (w: its place among the kept entries), -1: none.
+    MPF_HD int find(const AdjointArgs& J, int64_t c, uint32_t g, int w) const
+    {
+        if (J.next_cnt == nullptr) return w < J.s.slots ? w : -1;
+        int at = -1;
+#pragma unroll
+        for (int s = 3; s >= 0; --s) at = s < n && id[s] == g ? s : at;
+        for (int s = 4; s < n && at < 0; ++s)
+            if (J.next_id[static_cast<int64_t>(s) * J.s.ncells + c] == g) at = s;
+        return at;
+    }
+    MPF_HD double lam(const AdjointArgs& J, int64_t c, int at) const
+    {
+        const double v = J.lam_next[(at >= 0 ? static_cast<int64_t>(at) * J.s.ncells : 0) + c];
+        return at >= 0 ? v : 0.0;
+    }
+};
 
 // Reverse sweep through the limiter iterations of a cell of three or more entries, each
 // psi_p <- psi_p f_p (limiter_pass); the increments entering iteration k are recomputed from
@@ -450,6 +466,7 @@ MPF_HD __forceinline__ void cell_adjoint(const AdjointArgs& J, bool fp32, int64_
     const int NP = A.nphases, NP2 = NP * NP;
     const int n0 = L.n0;
     const double Pf = A.prefactor, dt = A.dt;
+    const NextList next(J, fp32, c);
     CellFwd<C, GRAD> F;
     cell_forward<C, GRAD, K>(J, L, F);
     const int (&ph)[C] = F.ph;
@@ -474,11 +491,9 @@ MPF_HD __forceinline__ void cell_adjoint(const AdjointArgs& J, bool fp32, int64_
         int w = 0;
 #pragma unroll UA
         for (int t = 0; t < C; ++t) {
-            lam_out[t] = 0.0;
-            if (R.keep >> t & 1u) {
-                lam_out[t] = lam_of(J, fp32, c, L.eid[t], w);
-                ++w;
-            }
+            const bool kept = (R.keep >> t & 1u) != 0u;
+            lam_out[t] = next.lam(J, c, kept ? next.find(J, c, L.eid[t], w) : -1);
+            w += kept ? 1 : 0;
         }
     }
 
