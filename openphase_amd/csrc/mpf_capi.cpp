@@ -1300,6 +1300,65 @@ StateLayout state_layout(const mpf_ctx* c)
     return L;
 }
 
+mpf::StateParts saved_parts(const mpf_ctx* c, void* blob)
+{
+    const StateLayout L = state_layout(c);
+    char* b = static_cast<char*>(blob);
+    return {reinterpret_cast<uint8_t*>(b + L.cnt), reinterpret_cast<uint16_t*>(b + L.id), b + L.val,
+            reinterpret_cast<double*>(b + L.volume), reinterpret_cast<double*>(b + L.maxvolume),
+            reinterpret_cast<double*>(b + L.vr), reinterpret_cast<uint8_t*>(b + L.exist), reinterpret_cast<int32_t*>(b + L.stage)};
+}
+
+mpf::StateParts context_parts(const mpf_ctx* c)
+{
+    return {c->cnt[c->cur], c->id[c->cur], c->val[c->cur], c->g_volume, c->g_maxvolume, c->g_vr, c->g_exist, c->g_stage};
+}
+
+// Whether the checkpoint kernels may access `p`: memory of the current device, where the state lies
+// too, aligned for their 16-byte accesses. Anything else takes the runtime's copies.
+bool kernel_copies(const mpf_ctx* c, const void* p)
+{
+    int dev = -1;
+    if (reinterpret_cast<uintptr_t>(p) % 16 != 0 || hipGetDevice(&dev) != hipSuccess) return false;
+    for (const void* q : {p, static_cast<const void*>(c->cnt[c->cur])}) {
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, q) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        if (at.type != hipMemoryTypeDevice || at.device != dev) return false;
+    }
+    return true;
+}
+
+mpf_status copy_parts(mpf_ctx* c, const mpf::StateParts& dst, const mpf::StateParts& src, const char* what)
+{
+    const size_t N = static_cast<size_t>(c->ncells), S = static_cast<size_t>(c->slots), G = static_cast<size_t>(c->ngrains);
+    hipError_t e = hipSuccess;
+    auto cp = [&](void* d, const void* s, size_t n) {
+        if (e == hipSuccess) e = hipMemcpyAsync(d, s, n, hipMemcpyDeviceToDevice, c->stream);
+    };
+    cp(dst.cnt, src.cnt, N);
+    cp(dst.id, src.id, S * N * sizeof(uint16_t));
+    cp(dst.val, src.val, S * N * c->vsize());
+    cp(dst.volume, src.volume, G * sizeof(double));
+    cp(dst.maxvolume, src.maxvolume, G * sizeof(double));
+    cp(dst.vr, src.vr, G * sizeof(double));
+    cp(dst.exist, src.exist, G);
+    cp(dst.stage, src.stage, G * sizeof(int32_t));
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    return c->hip(e, what);
+}
+
+mpf::StateCopy state_copy(const mpf_ctx* c)
+{
+    mpf::StateCopy a{};
+    a.ncells = c->ncells;
+    a.slots = c->slots;
+    a.ngrains = c->ngrains;
+    return a;
+}
+
 }  // namespace
 
 mpf_status mpf_state_bytes(mpf_ctx* c, int64_t* bytes)
@@ -1314,47 +1373,30 @@ mpf_status mpf_save_state(mpf_ctx* c, void* dst)
 {
     if (!c || !dst) return MPF_ERR_ARG;
     if (!c->initialized) return c->fail(MPF_ERR_STATE, "mpf_finalize_initialization first");
-    const StateLayout L = state_layout(c);
-    const size_t N = static_cast<size_t>(c->ncells), S = static_cast<size_t>(c->slots), G = static_cast<size_t>(c->ngrains);
-    char* d = static_cast<char*>(dst);
-    hipError_t e = hipSuccess;
-    auto cp = [&](size_t off, const void* src, size_t n) {
-        if (e == hipSuccess) e = hipMemcpyAsync(d + off, src, n, hipMemcpyDeviceToDevice, c->stream);
-    };
-    cp(L.cnt, c->cnt[c->cur], N);
-    cp(L.id, c->id[c->cur], S * N * sizeof(uint16_t));
-    cp(L.val, c->val[c->cur], S * N * c->vsize());
-    cp(L.volume, c->g_volume, G * sizeof(double));
-    cp(L.maxvolume, c->g_maxvolume, G * sizeof(double));
-    cp(L.vr, c->g_vr, G * sizeof(double));
-    cp(L.exist, c->g_exist, G);
-    cp(L.stage, c->g_stage, G * sizeof(int32_t));
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    return c->hip(e, "state save");
+    if (kernel_copies(c, dst)) {
+        mpf::StateCopy a = state_copy(c);
+        a.src = context_parts(c);
+        a.dst = saved_parts(c, dst);
+        const hipError_t e = static_cast<hipError_t>(mpf::launch_save(a, c->fp32, c->stream));
+        return c->hip(e == hipSuccess ? hipStreamSynchronize(c->stream) : e, "state save");
+    }
+    return copy_parts(c, saved_parts(c, dst), context_parts(c), "state save");
 }
 
 mpf_status mpf_restore_state(mpf_ctx* c, const void* src)
 {
     if (!c || !src) return MPF_ERR_ARG;
     if (!c->initialized) return c->fail(MPF_ERR_STATE, "mpf_finalize_initialization first");
-    const StateLayout L = state_layout(c);
-    const size_t N = static_cast<size_t>(c->ncells), S = static_cast<size_t>(c->slots), G = static_cast<size_t>(c->ngrains);
-    const char* s = static_cast<const char*>(src);
-    hipError_t e = hipSuccess;
-    auto cp = [&](void* dstp, size_t off, size_t n) {
-        if (e == hipSuccess) e = hipMemcpyAsync(dstp, s + off, n, hipMemcpyDeviceToDevice, c->stream);
-    };
+    const mpf::StateParts saved = saved_parts(c, const_cast<void*>(src));
     c->prev_valid = false;
-    cp(c->cnt[c->cur], L.cnt, N);
-    cp(c->id[c->cur], L.id, S * N * sizeof(uint16_t));
-    cp(c->val[c->cur], L.val, S * N * c->vsize());
-    cp(c->g_volume, L.volume, G * sizeof(double));
-    cp(c->g_maxvolume, L.maxvolume, G * sizeof(double));
-    cp(c->g_vr, L.vr, G * sizeof(double));
-    cp(c->g_exist, L.exist, G);
-    cp(c->g_stage, L.stage, G * sizeof(int32_t));
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    return c->hip(e, "state restore");
+    if (kernel_copies(c, src)) {
+        mpf::StateCopy a = state_copy(c);
+        a.src = saved;
+        a.dst = context_parts(c);
+        const hipError_t e = static_cast<hipError_t>(mpf::launch_restore(a, c->fp32, c->stream));
+        return c->hip(e == hipSuccess ? hipStreamSynchronize(c->stream) : e, "state restore");
+    }
+    return copy_parts(c, context_parts(c), saved, "state restore");
 }
 
 mpf_status mpf_adjoint_step(mpf_ctx* c, double dt, const double* lam_next, double* lam_prev, double* grad,

@@ -235,6 +235,25 @@ int launch_pack_offsets(const uint8_t* cnt, int64_t ncells, bool fp32, int64_t* 
 // Blocks first .. first + blocks - 1 into device buffers (null: not wanted).
 int launch_pack(const StepArgs& a, bool fp32, const int64_t* offset, int64_t first, int64_t blocks, int32_t* count, int8_t* flag,
                 int32_t* index, double* value, void* stream);
+
+// Device checkpoints (mpf_pack.hip).
+struct StateParts {
+    uint8_t* cnt;
+    uint16_t* id;
+    void* val;
+    double* volume;
+    double* maxvolume;
+    double* vr;
+    uint8_t* exist;
+    int32_t* stage;
+};
+struct StateCopy {
+    StateParts src, dst;
+    int64_t ncells;
+    int32_t slots, ngrains;
+};
+int launch_restore(const StateCopy& a, bool fp32, void* stream);
+int launch_save(const StateCopy& a, bool fp32, void* stream);
 int launch_grains(const GrainArgs* args, const uint32_t* first, int ndom, unsigned blocks, void* stream);
 int launch_copy(const void* src, void* dst, int64_t bytes, void* stream);
 

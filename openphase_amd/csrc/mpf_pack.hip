@@ -6,7 +6,7 @@
 // per cell, instead of every stored slot (10 bytes each) for a host loop to pick from. At 128^3 with 16
 // slots and 3.3 million entries a download took 94 ms, most of it that loop and the pages of its
 // 335 MB of buffers; now 4.2 ms (a 1.2 ms step among them not counted). The transfer to pageable
-// memory bounds it: the kernels take 50 us.
+// memory bounds it: the kernels take 50 us. Also the device checkpoints.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -113,7 +113,76 @@ __global__ __launch_bounds__(kPackBlock) void pack_write_kernel(const StepArgs A
     }
 }
 
+// Checkpoints (mpf_save_state, mpf_restore_state) in one launch each instead of eight copies, which
+// small domains feel most: 6 us of kernel for a domain of 128^2 to 512^2. 64 such domains restored and
+// stepped 40 times took 23.1 ms and take 20.1 ms; 512^2 in FP64 with 20 steps 1.11 and 1.05 ms.
+
+// A saved state into the context: counts, the entries in use, grain arrays. Slots a cell does not use
+// are never read, so they are left: at 256^3 with 16 slots a restore takes 0.26 ms, a copy of every slot
+// (the save) 1.1 ms.
+template <typename TV>
+__global__ __launch_bounds__(256) void restore_kernel(const StateCopy S)
+{
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (c < S.ncells) {
+        const uint8_t code = S.src.cnt[c];
+        S.dst.cnt[c] = code;
+        const int n = min(ListCode<TV>::count(code), S.slots);
+        for (int s = 0; s < n; ++s) {
+            const int64_t at = static_cast<int64_t>(s) * S.ncells + c;
+            S.dst.id[at] = S.src.id[at];
+            static_cast<TV*>(S.dst.val)[at] = static_cast<const TV*>(S.src.val)[at];
+        }
+    }
+    if (c < S.ngrains) {
+        S.dst.volume[c] = S.src.volume[c];
+        S.dst.maxvolume[c] = S.src.maxvolume[c];
+        S.dst.vr[c] = S.src.vr[c];
+        S.dst.exist[c] = S.src.exist[c];
+        S.dst.stage[c] = S.src.stage[c];
+    }
+}
+
+// The context's state into a checkpoint, every slot.
+__global__ __launch_bounds__(256) void save_kernel(const StateCopy S, int value_bytes)
+{
+    const int64_t i0 = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x, stride = static_cast<int64_t>(gridDim.x) * 256;
+    auto copy = [&](void* dst, const void* src, int64_t bytes) {
+        const int64_t n = bytes / 16;
+        for (int64_t i = i0; i < n; i += stride) static_cast<uint4*>(dst)[i] = static_cast<const uint4*>(src)[i];
+        for (int64_t i = 16 * n + i0; i < bytes; i += stride) static_cast<uint8_t*>(dst)[i] = static_cast<const uint8_t*>(src)[i];
+    };
+    copy(S.dst.cnt, S.src.cnt, S.ncells);
+    copy(S.dst.id, S.src.id, S.ncells * S.slots * 2);
+    copy(S.dst.val, S.src.val, S.ncells * S.slots * value_bytes);
+    for (int64_t g = i0; g < S.ngrains; g += stride) {
+        S.dst.volume[g] = S.src.volume[g];
+        S.dst.maxvolume[g] = S.src.maxvolume[g];
+        S.dst.vr[g] = S.src.vr[g];
+        S.dst.exist[g] = S.src.exist[g];
+        S.dst.stage[g] = S.src.stage[g];
+    }
+}
+
 }  // namespace
+
+int launch_restore(const StateCopy& a, bool fp32, void* stream)
+{
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int64_t n = a.ncells > a.ngrains ? a.ncells : a.ngrains;
+    const dim3 grid(static_cast<unsigned>((n + 255) / 256));
+    if (fp32) hipLaunchKernelGGL((restore_kernel<float>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((restore_kernel<double>), grid, dim3(256), 0, s, a);
+    return static_cast<int>(hipGetLastError());
+}
+
+int launch_save(const StateCopy& a, bool fp32, void* stream)
+{
+    const int64_t n = a.ncells * a.slots / 1024 + 1;
+    const dim3 grid(static_cast<unsigned>(n < 16384 ? n : 16384));
+    hipLaunchKernelGGL(save_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), a, fp32 ? 4 : 8);
+    return static_cast<int>(hipGetLastError());
+}
 
 int64_t pack_blocks(int64_t ncells) { return (ncells + kPackCells - 1) / kPackCells; }
 
