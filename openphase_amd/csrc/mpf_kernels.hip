@@ -89,7 +89,7 @@ __global__ __launch_bounds__(kBlock) void finalize_init_kernel(const StepArgs A)
     }
     // the list was validated against the capacity on upload
     if (valid) store_cell<K, TV, double, false>(A, cc, L);
-    for (int t = 0; t < K; ++t) wave_volume_add<true>(L.keep[t], L.eid[t], L.phi[t], A.vol_acc, bad_volume);
+    for (int t = 0; t < K; ++t) wave_volume_add(L.keep[t], L.eid[t], L.phi[t], A.vol_acc, bad_volume);
     if (bad_volume) atomicOr(&A.status[kStatusVolumeRange], 1);
 }
 

@@ -97,17 +97,14 @@ __device__ __forceinline__ void value_limbs(double v, unsigned long long l[kLimb
 
 // Adds the (grain, value) entries of all lanes of the wavefront to the grain accumulators with one
 // integer atomic per distinct grain and limb. Must be reached by whole wavefronts.
-// LANE_EXACT = false: the lanes' values are summed in FP64 by a butterfly (fixed lane order);
-// deterministic when the cell-to-lane mapping is (the main kernel).
-// LANE_EXACT = true: every value is converted to fixed point first and the limbs are summed as
-// integers; deterministic for any mapping (the work-list kernels, whose order varies).
-template <bool LANE_EXACT>
+// Every value is converted to fixed point first and the limbs are summed as integers, which gives
+// the same sum for any mapping of cells to lanes (the order of a work list varies).
 __device__ __forceinline__ void wave_volume_add(bool act, uint32_t g, double v,
                                                 unsigned long long* acc, bool& bad)
 {
     const int lane = static_cast<int>(threadIdx.x) & (warpSize - 1);
     unsigned long long lv[kLimbs] = {0ull, 0ull, 0ull, 0ull};
-    if (LANE_EXACT && act) value_limbs(v, lv, bad);
+    if (act) value_limbs(v, lv, bad);
     while (true) {
         unsigned long long m = __ballot(act);
         if (m == 0ull) break;
@@ -115,19 +112,12 @@ __device__ __forceinline__ void wave_volume_add(bool act, uint32_t g, double v,
         uint32_t g0 = static_cast<uint32_t>(__shfl(static_cast<int>(g), leader));
         bool sel = act && (g == g0);
         unsigned long long l[kLimbs];
-        if (LANE_EXACT) {
 #pragma unroll
-            for (int i = 0; i < kLimbs; ++i) {
-                unsigned long long s = sel ? lv[i] : 0ull;
-#pragma unroll
-                for (int k = 32; k >= 1; k >>= 1) s += __shfl_xor(s, k);
-                l[i] = s;
-            }
-        } else {
-            double s = sel ? v : 0.0;
+        for (int i = 0; i < kLimbs; ++i) {
+            unsigned long long s = sel ? lv[i] : 0ull;
 #pragma unroll
             for (int k = 32; k >= 1; k >>= 1) s += __shfl_xor(s, k);
-            if (lane == leader) value_limbs(s, l, bad);
+            l[i] = s;
         }
         if (lane == leader) {
 #pragma unroll
@@ -403,9 +393,9 @@ __device__ __forceinline__ void merge_entry(CellList<K, TC, GRAD>& L, int& ne, b
 // gradients); appended entries start at value 0 (CalculateDerivativesSR). One plane of nine
 // neighbours per loop trip (the loop is not unrolled, which keeps the kernel within the
 // instruction cache): the first two entries of the nine are loaded together with branch-free
-// buffer loads, a third entry (rare) on demand. A list growing beyond K returns kCellDeferred.
-// Entries beyond a neighbour's third are read one by one (MANY) or defer the cell.
-template <int K, typename TV, typename TC, bool GRAD, bool MANY>
+// buffer loads, entries beyond a neighbour's third or fourth (rare) one by one on demand. A list
+// growing beyond K returns kCellDeferred.
+template <int K, typename TV, typename TC, bool GRAD>
 __device__ __forceinline__ int merge_neighbours(const StepArgs& A, const Box& B, const uint32_t codes[7],
                                                 CellList<K, TC, GRAD>& L)
 {
@@ -474,14 +464,10 @@ __device__ __forceinline__ int merge_neighbours(const StepArgs& A, const Box& B,
                 if (m > 2) {
                     const TC a2 = static_cast<TC>(v2);
                     merge_entry<K, TC, GRAD>(L, ne, over, a2 != TC(0), g2, w * a2, gwx * a2, gwy * a2, gwz * a2, side);
-                    if (!MANY) {
-                        over = over || m > 3;
-                    } else {
-                        for (int q = 3; q < m; ++q) {
-                            const TC aq = static_cast<TC>(load_val<TV>(A.val_in, static_cast<int64_t>(q) * N + nb));
-                            const uint32_t gq = A.id_in[static_cast<int64_t>(q) * N + nb];
-                            merge_entry<K, TC, GRAD>(L, ne, over, aq != TC(0), gq, w * aq, gwx * aq, gwy * aq, gwz * aq, side);
-                        }
+                    for (int q = 3; q < m; ++q) {
+                        const TC aq = static_cast<TC>(load_val<TV>(A.val_in, static_cast<int64_t>(q) * N + nb));
+                        const uint32_t gq = A.id_in[static_cast<int64_t>(q) * N + nb];
+                        merge_entry<K, TC, GRAD>(L, ne, over, aq != TC(0), gq, w * aq, gwx * aq, gwy * aq, gwz * aq, side);
                     }
                 }
             }
@@ -511,14 +497,11 @@ __device__ __forceinline__ int merge_neighbours(const StepArgs& A, const Box& B,
                 v0[j] = lone ? TV(1) : buffer_load<TV>(rv0, m > 0 ? nb * SV : kNoLoad);
                 g1[j] = buffer_load<uint16_t>(ri1, m > 1 ? nb * 2u : kNoLoad);
                 v1[j] = buffer_load<TV>(rv1, m > 1 ? nb * SV : kNoLoad);
-                // the work-list kernels (MANY) load a third and fourth entry with the first two,
-                // so a neighbour of four entries costs no extra round trip (256^3 deferred-cell
-                // kernels 0.80 -> 0.77 ms)
+                // a third and fourth entry are loaded with the first two, so a neighbour of four
+                // entries costs no extra round trip
                 g2p[j] = 0u; v2p[j] = TV(0); g3p[j] = 0u; v3p[j] = TV(0);
-                if (MANY) {
-                    if (m > 2) { g2p[j] = A.id_in[2 * N + nb]; v2p[j] = load_val<TV>(A.val_in, 2 * N + nb); }
-                    if (m > 3) { g3p[j] = A.id_in[3 * N + nb]; v3p[j] = load_val<TV>(A.val_in, 3 * N + nb); }
-                }
+                if (m > 2) { g2p[j] = A.id_in[2 * N + nb]; v2p[j] = load_val<TV>(A.val_in, 2 * N + nb); }
+                if (m > 3) { g3p[j] = A.id_in[3 * N + nb]; v3p[j] = load_val<TV>(A.val_in, 3 * N + nb); }
             }
             const int dx = ip - 1, jj = r - 1;
 #pragma unroll
@@ -533,30 +516,19 @@ __device__ __forceinline__ int merge_neighbours(const StepArgs& A, const Box& B,
                 const TC gwx = dx == 0 ? TC(0) : (dx < 0 ? -gw : gw);
                 const TC gwy = jj == 0 ? TC(0) : (jj < 0 ? -gw : gw);
                 const TC gwz = kk == 0 ? TC(0) : (kk < 0 ? -gw : gw);
-                // entries beyond the second (rare), loaded on demand
-                TV v2 = TV(0);
-                uint32_t g2 = 0u;
-                if (m > 2) {
-                    g2 = MANY ? g2p[j] : A.id_in[2 * N + nb];
-                    v2 = MANY ? v2p[j] : load_val<TV>(A.val_in, 2 * N + nb);
-                }
                 const TC a0 = static_cast<TC>(v0[j]), a1 = static_cast<TC>(v1[j]);
                 merge_entry<K, TC, GRAD>(L, ne, over, m > 0 && a0 != TC(0), g0[j], w * a0,
                                          gwx * a0, gwy * a0, gwz * a0, side);
                 merge_entry<K, TC, GRAD>(L, ne, over, m > 1 && a1 != TC(0), g1[j], w * a1,
                                          gwx * a1, gwy * a1, gwz * a1, side);
                 if (m > 2) {
-                    const TC a2 = static_cast<TC>(v2);
-                    merge_entry<K, TC, GRAD>(L, ne, over, a2 != TC(0), g2, w * a2, gwx * a2, gwy * a2, gwz * a2, side);
-                    if (!MANY) {
-                        over = over || m > 3;
-                    } else {
-                        for (int q = 3; q < m; ++q) {
-                            const TC aq = q == 3 ? static_cast<TC>(v3p[j])
-                                                 : static_cast<TC>(load_val<TV>(A.val_in, static_cast<int64_t>(q) * N + nb));
-                            const uint32_t gq = q == 3 ? g3p[j] : A.id_in[static_cast<int64_t>(q) * N + nb];
-                            merge_entry<K, TC, GRAD>(L, ne, over, aq != TC(0), gq, w * aq, gwx * aq, gwy * aq, gwz * aq, side);
-                        }
+                    const TC a2 = static_cast<TC>(v2p[j]);
+                    merge_entry<K, TC, GRAD>(L, ne, over, a2 != TC(0), g2p[j], w * a2, gwx * a2, gwy * a2, gwz * a2, side);
+                    for (int q = 3; q < m; ++q) {
+                        const TC aq = q == 3 ? static_cast<TC>(v3p[j])
+                                             : static_cast<TC>(load_val<TV>(A.val_in, static_cast<int64_t>(q) * N + nb));
+                        const uint32_t gq = q == 3 ? g3p[j] : A.id_in[static_cast<int64_t>(q) * N + nb];
+                        merge_entry<K, TC, GRAD>(L, ne, over, aq != TC(0), gq, w * aq, gwx * aq, gwy * aq, gwz * aq, side);
                     }
                 }
             }
@@ -576,7 +548,7 @@ __device__ __forceinline__ int gather_cell(const StepArgs& A, int64_t cc, CellLi
     const Box B = make_box(A, cc);
     uint32_t codes[7];
     if (!load_codes<TV>(A, B, code, codes)) return kCellBulk;
-    return merge_neighbours<K, TV, TC, GRAD, true>(A, B, codes, L);
+    return merge_neighbours<K, TV, TC, GRAD>(A, B, codes, L);
 }
 
 }  // namespace

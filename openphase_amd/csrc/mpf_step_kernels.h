@@ -33,7 +33,7 @@ __device__ __forceinline__ void wave_volume_add_split(bool act, uint32_t g, doub
         if (lane == leader) atomicAdd(&acc[static_cast<int64_t>(g0) * kLimbs + 3], cells << 20);
         one = one && !sel;
     }
-    wave_volume_add<true>(act && v != 1.0, g, v, acc, bad);
+    wave_volume_add(act && v != 1.0, g, v, acc, bad);
 }
 
 // One block = kBlock consecutive cells. Phase 1 classifies every cell from the count bytes of its
@@ -125,7 +125,7 @@ __device__ __forceinline__ void step_block(const StepArgs& A, int64_t base, uint
         for (int w = 0; w < 7; ++w) codes[w] = s_codes[w][local];
         bool empty = false;
         load_own<K, TV, TC, GRAD>(A, cw, box_code(codes, 13), L);
-        int r = merge_neighbours<K, TV, TC, GRAD, true>(A, make_box(A, cw), codes, L);
+        int r = merge_neighbours<K, TV, TC, GRAD>(A, make_box(A, cw), codes, L);
         if (r == kCellWide) {
             // merged lists of 2-4 entries here; longer ones (few cells) are deferred
             // UNI: the equal-energy form only; cells next to a grain below its reference volume
@@ -133,9 +133,9 @@ __device__ __forceinline__ void step_block(const StepArgs& A, int64_t base, uint
             constexpr int PATH = UNI ? 1 : 2;
             bool done = false;
             switch (L.ne) {
-            case 2: done = compute_cell<2, true, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
-            case 3: done = compute_cell<3, true, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
-            case 4: done = compute_cell<4, true, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
+            case 2: done = compute_cell<2, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
+            case 3: done = compute_cell<3, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
+            case 4: done = compute_cell<4, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
             default: break;
             }
             if (!done) r = kCellDeferred;

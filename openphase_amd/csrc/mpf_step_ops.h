@@ -27,16 +27,16 @@ __device__ __forceinline__ TC dg_local(const StepArgs& A, int a, int b, int n0, 
 }
 
 // IP.Set + increments + normalize + merge + finalize of a wide cell whose merged list has C
-// entries (EXACT) or at most C entries (ne at run time). Only entries < C are touched.
+// entries. Only entries < C are touched.
 // PATH selects the increment formula at compile time: 0 both (chosen per cell), 1 only the
 // equal-energy form (returns false, doing nothing, for a cell that needs the general one), 2 only
 // the general form (exact for every cell: the equal-energy form drops exact zero terms).
-template <int C, bool EXACT, int K, typename TC, bool GRAD, bool DG, int PATH = 0>
+template <int C, int K, typename TC, bool GRAD, bool DG, int PATH = 0>
 __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, GRAD>& L, bool& empty, int64_t cell)
 {
     constexpr int U = C <= kFastSlots ? C : 1;
     constexpr int NPC = C * (C - 1) / 2;
-    const int ne = EXACT ? C : L.ne;
+    constexpr int ne = C;
     const int n0 = L.n0;
     const int NP = A.nphases;
 
@@ -45,20 +45,20 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
     double vr[C];
 #pragma unroll U
     for (int t = 0; t < C; ++t) {
-        ph[t] = 0; vr[t] = 0.0;
-        if (EXACT || t < ne) { ph[t] = A.gphase[L.eid[t]]; vr[t] = A.gvr[L.eid[t]]; }
+        ph[t] = A.gphase[L.eid[t]];
+        vr[t] = A.gvr[L.eid[t]];
     }
     double localn = 0.0;
     if (A.consider_nucleus) {
 #pragma unroll U
-        for (int t = 0; t < C; ++t) if (EXACT || t < ne) localn += vr[t];
+        for (int t = 0; t < C; ++t) localn += vr[t];
     } else {
         localn = static_cast<double>(ne);
     }
     const double norm_1 = 1.0 / localn;
     bool uni = A.uniform != 0;
 #pragma unroll U
-    for (int t = 0; t < C; ++t) uni = uni && (!(EXACT || t < ne) || vr[t] == 1.0);
+    for (int t = 0; t < C; ++t) uni = uni && vr[t] == 1.0;
     if (PATH == 1 && !uni) return false;
     if (PATH == 2) uni = false;
 
@@ -83,7 +83,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
         for (int a = 0; a < C; ++a)
 #pragma unroll U
         for (int b = 0; b < C; ++b) {
-            if (b <= a || !(EXACT || b < ne)) continue;
+            if (b <= a) continue;
             TC d = s0 * (X[a] - X[b]);
             d *= mf;
             if (DG && n0 > 1 && A.dg_mode[ph[a] * NP + ph[b]] == 1) {
@@ -103,7 +103,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
             for (int a = 0; a < C; ++a)
 #pragma unroll U
             for (int b = 0; b < C; ++b) {
-                if (b <= a || !(EXACT || b < ne)) continue;
+                if (b <= a) continue;
                 const int k = ph[a] * NP + ph[b];
                 const TC en = ip_pair_energy<TC>(A, k, L.eid[a], L.eid[b], L.ev(a), L.ev(b), L.gr[GRAD ? a : 0],
                                                  L.gr[GRAD ? b : 0]);
@@ -118,7 +118,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
         for (int a = 0; a < C; ++a)
 #pragma unroll U
         for (int b = 0; b < C; ++b) {
-            if (b <= a || !(EXACT || b < ne)) continue;
+            if (b <= a) continue;
             const double scaled = sqrt(vr[a] * vr[b]);
             const TC scale = static_cast<TC>(scaled);
             const TC cf = TC(0.5) * (TC(1.0) + scale) * P;
@@ -126,7 +126,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
             if (ne > 2) {
 #pragma unroll U
                 for (int g = 0; g < C; ++g) {
-                    if (g == a || g == b || !(EXACT || g < ne)) continue;
+                    if (g == a || g == b) continue;
                     d += (sigma_of(b, g) - sigma_of(a, g)) * (L.lap[g] + cf * L.ev(g));
                     if (A.tj_model == 0) {
                         if (A.tj_factor != 0.0 || scaled < 1.0) {
@@ -195,17 +195,16 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
         // zero the pairs that would push a field at 0 below or at 1 above
 #pragma unroll U
         for (int a = 0; a < C; ++a) {
-            if (!(EXACT || a < ne)) continue;
             double dpsi = 0.0;
 #pragma unroll U
             for (int b = 0; b < C; ++b) {
-                if (b == a || !(EXACT || b < ne)) continue;
+                if (b == a) continue;
                 dpsi += a < b ? psi[pair_index<C>(a, b)] : psi[pair_index<C>(b, a)] * (-1.0);
             }
             if ((phi[a] == 0.0 && dpsi < 0.0) || (phi[a] == 1.0 && dpsi > 0.0)) {
 #pragma unroll U
                 for (int b = 0; b < C; ++b) {
-                    if (b == a || !(EXACT || b < ne)) continue;
+                    if (b == a) continue;
                     psi[a < b ? pair_index<C>(a, b) : pair_index<C>(b, a)] = 0.0;
                 }
             }
@@ -215,7 +214,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
         for (int a = 0; a < C; ++a)
 #pragma unroll U
         for (int b = 0; b < C; ++b) {
-            if (b <= a || !(EXACT || b < ne)) continue;
+            if (b <= a) continue;
             const int p = pair_index<C>(a, b);
             alive[p] = psi[p] != 0.0;
             any = any || alive[p];
@@ -234,7 +233,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
                 for (int a = 0; a < C; ++a)
 #pragma unroll U
                 for (int b = 0; b < C; ++b) {
-                    if (b <= a || !(EXACT || b < ne)) continue;
+                    if (b <= a) continue;
                     const int p = pair_index<C>(a, b);
                     if (!alive[p]) continue;
                     const double v = psi[p];
@@ -244,7 +243,6 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
 #pragma unroll U
                 for (int t = 0; t < C; ++t) {
                     lim1[t] = 1.0; lim2[t] = 1.0;
-                    if (!(EXACT || t < ne)) continue;
                     const double npf = phi[t] + (pos[t] + neg[t]) * dt;
                     if (npf < 0.0) lim2[t] = smin(lim2[t], -(phi[t] + pos[t] * dt) / (neg[t] * dt));
                     if (npf > 1.0) lim1[t] = smin(lim1[t], (1.0 - (phi[t] + neg[t] * dt)) / (pos[t] * dt));
@@ -253,7 +251,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
                 for (int a = 0; a < C; ++a)
 #pragma unroll U
                 for (int b = 0; b < C; ++b) {
-                    if (b <= a || !(EXACT || b < ne)) continue;
+                    if (b <= a) continue;
                     const int p = pair_index<C>(a, b);
                     if (!alive[p]) continue;
                     if (psi[p] < 0.0) {
@@ -281,7 +279,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
             for (int a = 0; a < C; ++a)
 #pragma unroll U
             for (int b = 0; b < C; ++b) {
-                if (b <= a || !(EXACT || b < ne)) continue;
+                if (b <= a) continue;
                 const int p = pair_index<C>(a, b);
                 if (!alive[p] || psi[p] == 0.0) continue;
                 tv[a] += psi[p] * dt;
@@ -290,7 +288,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
             unsigned long long warn = 0;
 #pragma unroll U
             for (int t = 0; t < C; ++t)
-                if ((EXACT || t < ne) && (tv[t] < -FLT_EPSILON || tv[t] > 1.0 + FLT_EPSILON)) ++warn;
+                if (tv[t] < -FLT_EPSILON || tv[t] > 1.0 + FLT_EPSILON) ++warn;
             if (warn) atomicAdd(A.warnings, warn);
         }
     }
@@ -300,7 +298,7 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
     for (int a = 0; a < C; ++a)
 #pragma unroll U
     for (int b = 0; b < C; ++b) {
-        if (b <= a || !(EXACT || b < ne)) continue;
+        if (b <= a) continue;
         const int p = pair_index<C>(a, b);
         if (!alive[p]) continue;
         const double value = 1.0 * psi[p] * dt;
@@ -316,7 +314,6 @@ __device__ __forceinline__ bool compute_cell(const StepArgs& A, CellList<K, TC, 
 #pragma unroll U
     for (int t = 0; t < C; ++t) {
         L.keep[t] = false;
-        if (!(EXACT || t < ne)) continue;
         double v = phi[t];
         bool erase = false;
         if (v >= 1.0 - DBL_EPSILON) v = 1.0;

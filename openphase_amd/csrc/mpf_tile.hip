@@ -526,9 +526,9 @@ __device__ __forceinline__ void tile_block(const StepArgs& A, const unsigned b)
                 L.ne = ne;
                 constexpr int PATH = UNI ? 0 : 2;
                 switch (ne) {
-                case 2: compute_cell<2, true, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
-                case 3: compute_cell<3, true, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
-                default: compute_cell<4, true, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
+                case 2: compute_cell<2, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
+                case 3: compute_cell<3, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
+                default: compute_cell<4, K, TC, GRAD, DG, PATH>(A, L, empty, cw); break;
                 }
                 if (!store_cell<K, TV, TC, GRAD>(A, cw, L)) report_overflow<K, TC, GRAD>(A, cw, L);
                 if (empty) atomicOr(&A.status[kStatusEmpty], 1);
