@@ -1496,8 +1496,8 @@ mpf_status mpf_autotune(mpf_ctx* c, double dt, int32_t steps, int32_t* xcd_order
         if (!t) t = read_status(c);
         return t;
     };
-    // 1. step-kernel tile: plane tiles of 64-256 cells x 1-16 planes per block (or the default
-    //    count), and the per-cell kernel
+    // 1. step-kernel tile: plane tiles (3D: 128-256 cells, 2D: 16-256) x 1-16 planes per block (or the
+    //    default count), and the per-cell kernel
     const int tx0 = c->tile_x, ty0 = c->tile_y, tz0 = c->tile_z;
     float best = 1e30f;
     int best_tx = tx0, best_ty = ty0, best_tz = tz0;

@@ -48,31 +48,6 @@ __device__ double entry_value(const StepArgs& A, int64_t c, uint8_t code, int t)
     return 1.0 - others;
 }
 
-// NodeDF::get_weight of pair (ga, gb) at cell nb (include/Containers/NodeDF.h:401-410): a Force
-// entry exists on an interface cell (more than one own entry) whose list holds both grains (the
-// pair's phases give the same mode everywhere); entries of zero-valued appended grains weigh 0 and
-// never count. On success: the weight, the pair plane and whether ga precedes gb in that cell's
-// list (the entry's stored order; get_raw / get_tmp flip the sign otherwise).
-template <typename TV>
-__device__ bool find_pair(const StepArgs& A, int64_t nb, uint32_t ga, uint32_t gb, double& w, int& plane, bool& fwd)
-{
-    const int64_t N = A.ncells;
-    const uint8_t code = A.cnt_in[nb];
-    const int n = ListCode<TV>::count(code);
-    if (n < 2) return false;
-    int ia = -1, ib = -1;
-    for (int s = 0; s < n; ++s) {
-        const uint32_t g = A.id_in[static_cast<int64_t>(s) * N + nb];
-        ia = g == ga ? s : ia;
-        ib = g == gb ? s : ib;
-    }
-    if (ia < 0 || ib < 0) return false;
-    w = sqrt(entry_value<TV>(A, nb, code, ia) * entry_value<TV>(A, nb, code, ib));
-    fwd = ia < ib;
-    plane = fwd ? pair_plane(ia, ib) : pair_plane(ib, ia);
-    return true;
-}
-
 // Lane l's value of x (l uniform across the wavefront).
 __device__ __forceinline__ double lane_value(double x, int l)
 {
@@ -84,24 +59,170 @@ __device__ __forceinline__ double lane_value(double x, int l)
 
 constexpr int kAvgCells = 64;                 // cells per block
 constexpr int kAvgWaves = kAvgBlock / 64;     // wavefronts per block
+constexpr int kAvgChunks = 2;                 // offsets of a lane looked up together
 
-// SECOND = false: CollectAverage into tmp; true: DistributeAverage into avg, for spheres too large
-// for staged tiles (sphere_tile_kernel). A block takes 64 consecutive cells and compacts their interface cells in LDS; its wavefronts take them in turn.
-// For one cell and pair the 64 lanes evaluate 64 sphere offsets at once (the neighbour's weight
-// and raw or tmp value), then every lane adds the terms of the lanes that count in lane order,
-// chunk after chunk: the sums are formed in the reference's offset order, and a wavefront waits
-// on a few memory round trips per chunk instead of one chain per offset.
-template <typename TV, bool SECOND>
-__global__ __launch_bounds__(kAvgBlock) void dg_average_kernel(const SphereArgs P)
+// The lists of the cells at the sphere's offsets t0 + 64 u + lane: all chunks' counts are loaded
+// together, then their first four grains (branch-free buffer loads).
+struct NearLists {
+    uint32_t nb[kAvgChunks];
+    uint8_t code[kAvgChunks];
+    int n[kAvgChunks];            // entries of an interface cell, else 0
+    uint32_t g[kAvgChunks][4];
+};
+
+template <typename TV>
+__device__ __forceinline__ void near_lists(const SphereArgs& P, int x, int y, int z, int t0, NearLists& L)
+{
+    const StepArgs& A = P.s;
+    const int64_t N = A.ncells;
+    const uint32_t N32 = static_cast<uint32_t>(N);
+    const int lane = static_cast<int>(threadIdx.x) & 63;
+#pragma unroll
+    for (int u = 0; u < kAvgChunks; ++u) {
+        const int t = min(t0 + 64 * u + lane, P.noff - 1);
+        const int ii = P.off[3 * t], jj = P.off[3 * t + 1], kk = P.off[3 * t + 2];
+        L.nb[u] = (static_cast<uint32_t>(wrap1(x + ii, A.nx)) * static_cast<uint32_t>(A.ny) + static_cast<uint32_t>(wrap1(y + jj, A.ny))) *
+                      static_cast<uint32_t>(A.nz) + static_cast<uint32_t>(wrap1(z + kk, A.nz));
+    }
+#pragma unroll
+    for (int u = 0; u < kAvgChunks; ++u) L.code[u] = A.cnt_in[L.nb[u]];
+#pragma unroll
+    for (int u = 0; u < kAvgChunks; ++u) {
+        const int n = t0 + 64 * u + lane < P.noff ? ListCode<TV>::count(L.code[u]) : 0;
+        L.n[u] = n < 2 ? 0 : n;
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+            L.g[u][s] = buffer_load<uint16_t>(plane_rsrc(A.id_in + s * N, N32 * 2u), s < L.n[u] ? L.nb[u] * 2u : kNoLoad);
+    }
+}
+
+// A pair of grains at one neighbour: NodeDF::get_weight / get_raw / get_tmp
+// (include/Containers/NodeDF.h:401-410). An entry exists on an interface cell (more than one own
+// entry) whose list holds both grains (the pair's phases give the same mode everywhere); entries of
+// zero-valued appended grains weigh 0 and never count.
+struct PairTerm {
+    bool has, fwd;   // fwd: ga precedes gb in the list (the entry's stored order; else the sign flips)
+    double w, v;     // sqrt(phi_a phi_b) and, given `src`, the pair's stored value there
+};
+
+// The pair (ga, gb) at the cells of L, its values and stored values loaded together; false when none
+// of the wavefront's cells holds it. Lanes without the pair read cell c.
+template <typename TV>
+__device__ __forceinline__ bool pair_terms(const StepArgs& A, const NearLists& L, int64_t c, uint32_t ga, uint32_t gb,
+                                           const double* src, PairTerm (&T)[kAvgChunks])
+{
+    const int64_t N = A.ncells;
+    int ia[kAvgChunks], ib[kAvgChunks];
+    bool any = false;
+#pragma unroll
+    for (int u = 0; u < kAvgChunks; ++u) {
+        ia[u] = ib[u] = -1;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            ia[u] = s < L.n[u] && L.g[u][s] == ga ? s : ia[u];
+            ib[u] = s < L.n[u] && L.g[u][s] == gb ? s : ib[u];
+        }
+        for (int s = 4; s < L.n[u]; ++s) {
+            const uint32_t gs = A.id_in[static_cast<int64_t>(s) * N + L.nb[u]];
+            ia[u] = gs == ga ? s : ia[u];
+            ib[u] = gs == gb ? s : ib[u];
+        }
+        T[u].has = ia[u] >= 0 && ib[u] >= 0;
+        T[u].fwd = ia[u] < ib[u];
+        any = any || T[u].has;
+    }
+    if (!__any(any)) return false;
+    double va[kAvgChunks], vb[kAvgChunks];
+#pragma unroll
+    for (int u = 0; u < kAvgChunks; ++u) {
+        T[u].v = 0.0;
+        if constexpr (ListCode<TV>::kImplicit) {
+            va[u] = vb[u] = 0.0;
+            if (T[u].has) {
+                va[u] = entry_value<TV>(A, L.nb[u], L.code[u], ia[u]);
+                vb[u] = entry_value<TV>(A, L.nb[u], L.code[u], ib[u]);
+            }
+        } else {
+            va[u] = load_val<TV>(A.val_in, T[u].has ? static_cast<int64_t>(ia[u]) * N + L.nb[u] : c);
+            vb[u] = load_val<TV>(A.val_in, T[u].has ? static_cast<int64_t>(ib[u]) * N + L.nb[u] : c);
+        }
+        if (src != nullptr) {
+            const int plane = T[u].fwd ? pair_plane(ia[u], ib[u]) : pair_plane(ib[u], ia[u]);
+            T[u].v = src[T[u].has ? static_cast<int64_t>(plane) * N + L.nb[u] : c];
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kAvgChunks; ++u) T[u].w = sqrt(va[u] * vb[u]);
+    return true;
+}
+
+// Adds the weights and terms that count of kAvgChunks chunks to `acc` in offset order (even lanes: the
+// sum of the weights, odd lanes: that of the terms) and returns how many there were. They are
+// compacted into LDS and added eight at a time by every lane, padded with +0, which changes no sum
+// here (none is ever -0): two instructions per term, where reading each from its lane's registers took
+// about twelve and made up half of the first pass.
+__device__ __forceinline__ int ordered_add(double (&buf)[64 * kAvgChunks + 8][2], const bool (&ok)[kAvgChunks],
+                                           const double (&wt)[kAvgChunks], const double (&term)[kAvgChunks], double& acc)
+{
+    const int lane = static_cast<int>(threadIdx.x) & 63;
+    int m = 0;
+#pragma unroll
+    for (int u = 0; u < kAvgChunks; ++u) {
+        const unsigned long long okm = __ballot(ok[u]);
+        if (ok[u]) {
+            const int at = m + __popcll(okm & ((1ull << lane) - 1ull));
+            buf[at][0] = wt[u];
+            buf[at][1] = term[u];
+        }
+        m += __popcll(okm);
+    }
+    if (m == 0) return 0;
+    if (lane < 16) buf[m + (lane >> 1)][lane & 1] = 0.0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int i = 0; i < m; i += 8) {
+        double e[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) e[q] = buf[i + q][lane & 1];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) acc += e[q];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    return m;
+}
+
+// SECOND = false: CollectAverage into tmp; true: DistributeAverage into avg, of the driving force or
+// (CURV) of the curvature, for spheres too large for staged tiles (sphere_tile_kernel). A block takes
+// 64 consecutive cells and compacts their interface cells in LDS; its wavefronts take them in turn.
+// Lane p holds pair p of the cell (64 at a time): its bounds, own value and sums. The 64 lanes look up
+// the lists at 64 kAvgChunks sphere offsets at once, every pair of the cell is matched against them, and its
+// terms are added in offset order, chunk after chunk, as the reference's sums are formed.
+//
+// The curvature: collect is InterfaceRegularization::CollectAverageSR
+// (src/InterfaceRegularization.cpp:196-223), distribute DistributeAverageSR (:225-274); the pair's
+// weight is sqrt(phi_a phi_b) (SetWeightsSR, :178-194) on interface cells. Collect: for a weight above
+// the threshold, the mean of the neighbours' raw weighted by weight * (Range - |offset|), over terms
+// above DBL_EPSILON, if their sum exceeds DBL_EPSILON (else the fresh entry's 0). Distribute: for a
+// weight above DBL_EPSILON, the plain mean of the tmp of the neighbours whose weight exceeds the
+// threshold, or the own tmp. No grain is a Seed here (grains enter as Stable; only nucleation makes
+// seeds), so the entries below those bounds keep 0.
+//
+// What bounds it is the lookups' round trips. 96^3, 485 offsets (collect / distribute): lists looked up
+// for each pair anew and terms read from lane registers 0.64 / 1.88 ms, terms added from LDS and two
+// chunks in flight 0.33 / 1.74 ms, lists looked up once for all pairs of a cell 0.31 / 1.32 ms.
+template <typename TV, bool SECOND, bool CURV>
+__global__ __launch_bounds__(kAvgBlock) void sphere_wave_kernel(const SphereArgs P)
 {
     __shared__ uint16_t s_list[kAvgCells];
     __shared__ int s_count;
+    __shared__ double s_terms[kAvgWaves][64 * kAvgChunks + 8][2];
     const StepArgs& A = P.s;
     const int64_t N = A.ncells;
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
     const int64_t base = static_cast<int64_t>(blockIdx.x) * kAvgCells;
     if (wave == 0) {
-        // Force entries live on interface cells (more than one own entry) only
+        // pairs of own entries live on interface cells (more than one own entry) only
         const int64_t c0 = base + lane;
         const bool inter = lane < kAvgCells && c0 < N && ListCode<TV>::count(A.cnt_in[c0]) >= 2;
         const unsigned long long m = __ballot(inter);
@@ -112,68 +233,95 @@ __global__ __launch_bounds__(kAvgBlock) void dg_average_kernel(const SphereArgs 
     const int ninter = s_count;
     const int64_t nyz = static_cast<int64_t>(A.ny) * A.nz;
     const int NP = A.nphases;
+    const double* src = SECOND ? P.tmp : (CURV ? P.raw : nullptr);
     for (int i = wave; i < ninter; i += kAvgWaves) {
         const int64_t c = base + s_list[i];
         const uint8_t code = A.cnt_in[c];
         const int n = ListCode<TV>::count(code);
         const int x = static_cast<int>(c / nyz), y = static_cast<int>((c / A.nz) % A.ny), z = static_cast<int>(c % A.nz);
-        for (int b = 1; b < n; ++b)
-            for (int a = 0; a < b; ++a) {
-                const uint32_t ga = A.id_in[static_cast<int64_t>(a) * N + c], gb = A.id_in[static_cast<int64_t>(b) * N + c];
-                const int pa = A.gphase[ga], pb = A.gphase[gb];
-                if (A.dg_mode[pa * NP + pb] != 1) continue;  // no Force entry for this pair
-                const int plane = pair_plane(a, b);
+        const int npairs = n * (n - 1) / 2;
+        for (int p0 = 0; p0 < npairs; p0 += 64) {
+            // ---- lane's pair (a, b), a < b, at plane b (b - 1) / 2 + a
+            const int p = p0 + lane;
+            uint32_t ga = 0u, gb = 0u;
+            double cut = 0.0, vab = 0.0, vba = 0.0, own = 0.0;
+            bool entry = false, run = false;
+            if (p < npairs) {
+                int b = 1;
+                while (b * (b + 1) / 2 <= p) ++b;
+                const int a = p - b * (b - 1) / 2;
+                ga = A.id_in[static_cast<int64_t>(a) * N + c];
+                gb = A.id_in[static_cast<int64_t>(b) * N + c];
                 const double w = sqrt(entry_value<TV>(A, c, code, a) * entry_value<TV>(A, c, code, b));
-                const double scale = A.gvr[ga] * A.gvr[gb];
-                const double cut = P.threshold * scale;
-                const double vab = A.dg_value[pa * NP + pb], vba = A.dg_value[pb * NP + pa];
-                // own value the pass falls back to: raw (collect) or tmp (distribute)
-                const double own = SECOND ? P.tmp[static_cast<int64_t>(plane) * N + c] : vab;
-                double result = 0.0;  // a fresh entry's tmp / average
-                if (SECOND ? (w > 0.0) : (w > cut)) {
-                    double value = 0.0, sum = 0.0;
-                    int counter = 0;
-                    for (int t0 = 0; t0 < P.noff; t0 += 64) {
-                        const int t = t0 + lane;
-                        bool ok = false;
-                        double wt = 0.0, term = 0.0;
-                        if (t < P.noff) {
-                            const int ii = P.off[3 * t], jj = P.off[3 * t + 1], kk = P.off[3 * t + 2];
-                            const int64_t nb = (static_cast<int64_t>(wrap1(x + ii, A.nx)) * A.ny + wrap1(y + jj, A.ny)) * A.nz +
-                                               wrap1(z + kk, A.nz);
-                            double wphi = 0.0;
-                            int np = 0;
-                            bool fwd = true;
-                            if (find_pair<TV>(A, nb, ga, gb, wphi, np, fwd) && (SECOND ? (wphi > cut) : (wphi > 0.0))) {
-                                ok = true;
-                                wt = P.weights == 1 ? P.off_w[t] : (P.weights == 0 ? wphi : 1.0);
-                                double v;
-                                if (SECOND) {
-                                    const double tn = P.tmp[static_cast<int64_t>(np) * N + nb];
-                                    v = fwd ? tn : -tn;
-                                } else {
-                                    v = fwd ? vab : -vba;
-                                }
-                                term = wt * v;
-                            }
-                        }
-                        // value += weight * v and sum += weight in offset order
-                        unsigned long long okm = __ballot(ok);
-                        while (okm) {
-                            const int l = __ffsll(static_cast<long long>(okm)) - 1;
-                            okm &= okm - 1ull;
-                            if (P.weights == 2) counter++;
-                            else sum += lane_value(wt, l);
-                            value += lane_value(term, l);
+                if (CURV) {
+                    entry = true;
+                    run = SECOND ? (w > DBL_EPSILON) : (w > P.threshold);
+                } else {
+                    const int pa = A.gphase[ga], pb = A.gphase[gb];
+                    entry = A.dg_mode[pa * NP + pb] == 1;  // else no Force entry for this pair
+                    const double scale = A.gvr[ga] * A.gvr[gb];
+                    cut = P.threshold * scale;
+                    vab = A.dg_value[pa * NP + pb];
+                    vba = A.dg_value[pb * NP + pa];
+                    run = entry && (SECOND ? (w > 0.0) : (w > cut));
+                }
+                // own value the pass falls back to: raw or 0 (collect), tmp (distribute)
+                if (entry) own = SECOND ? P.tmp[static_cast<int64_t>(p) * N + c] : (CURV ? 0.0 : vab);
+            }
+            double sum = 0.0, value = 0.0;
+            int counted = 0;
+            const unsigned long long pairs = __ballot(run);
+            for (int t0 = 0; pairs != 0ull && t0 < P.noff; t0 += 64 * kAvgChunks) {
+                NearLists L;
+                near_lists<TV>(P, x, y, z, t0, L);
+                double ow[kAvgChunks];
+#pragma unroll
+                for (int u = 0; u < kAvgChunks; ++u)
+                    ow[u] = (CURV ? !SECOND : P.weights == 1) ? P.off_w[min(t0 + 64 * u + lane, P.noff - 1)] : 1.0;
+                for (unsigned long long left = pairs; left != 0ull; left &= left - 1ull) {
+                    const int q = __ffsll(static_cast<long long>(left)) - 1;
+                    PairTerm T[kAvgChunks];
+                    if (!pair_terms<TV>(A, L, c, static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(ga), q)),
+                                        static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(gb), q)), src, T))
+                        continue;
+                    bool ok[kAvgChunks];
+                    double wt[kAvgChunks], term[kAvgChunks];
+#pragma unroll
+                    for (int u = 0; u < kAvgChunks; ++u) {
+                        if (CURV) {
+                            const double v = T[u].fwd ? T[u].v : -T[u].v;
+                            wt[u] = SECOND ? 0.0 : T[u].w * ow[u];
+                            ok[u] = T[u].has && (SECOND ? T[u].w > P.threshold : wt[u] > DBL_EPSILON);
+                            term[u] = SECOND ? v : wt[u] * v;
+                        } else {
+                            wt[u] = P.weights == 0 ? T[u].w : ow[u];
+                            ok[u] = T[u].has && (SECOND ? (T[u].w > lane_value(cut, q)) : (T[u].w > 0.0));
+                            if (SECOND) term[u] = wt[u] * (T[u].fwd ? T[u].v : -T[u].v);
+                            else term[u] = wt[u] * (T[u].fwd ? lane_value(vab, q) : -lane_value(vba, q));
                         }
                     }
-                    if (P.weights == 2) result = counter != 0 ? value / static_cast<double>(counter) : own;
-                    else result = sum > 0.0 ? value / sum : own;
+                    // value += weight * v and sum += weight in offset order
+                    double acc = lane & 1 ? lane_value(value, q) : lane_value(sum, q);
+                    const int m = ordered_add(s_terms[wave], ok, wt, term, acc);
+                    const double s0 = lane_value(acc, 0), s1 = lane_value(acc, 1);
+                    if (lane == q) {
+                        sum = s0;
+                        value = s1;
+                        counted += m;
+                    }
                 }
-                // DistributeAverage's weight-0 branch (Seed grains) cannot occur: own entries are
-                // above the finalize cutoff and no grain is a Seed
-                if (lane == 0) (SECOND ? P.avg : P.tmp)[static_cast<int64_t>(plane) * N + c] = result;
             }
+            // DistributeAverage's weight-0 branch (Seed grains) cannot occur: own entries are above the
+            // finalize cutoff and no grain is a Seed
+            if (entry) {
+                double result = 0.0;  // a fresh entry's tmp / average
+                if (run) {
+                    if (CURV ? SECOND : P.weights == 2) result = counted != 0 ? value / static_cast<double>(counted) : own;
+                    else result = sum > (CURV ? DBL_EPSILON : 0.0) ? value / sum : own;
+                }
+                (SECOND ? P.avg : P.tmp)[static_cast<int64_t>(p) * N + c] = result;
+            }
+        }
     }
 }
 
@@ -290,89 +438,6 @@ __global__ __launch_bounds__(64) void curvature_raw_kernel(const CurvArgs P)
     }
 }
 
-// SECOND = false: InterfaceRegularization::CollectAverageSR (src/InterfaceRegularization.cpp:196-223)
-// into tmp; true: DistributeAverageSR (:225-274) into avg. The pair's weight is sqrt(phi_a phi_b)
-// (SetWeightsSR, :178-194) on interface cells. Collect: for a weight above the threshold, the mean
-// of the neighbours' raw weighted by weight * (Range - |offset|), over terms above DBL_EPSILON, if
-// their sum exceeds DBL_EPSILON (else the fresh entry's 0). Distribute: for a weight above
-// DBL_EPSILON, the plain mean of the tmp of the neighbours whose weight exceeds the threshold, or
-// the own tmp. No grain is a Seed here (grains enter as Stable; only nucleation makes seeds), so
-// the entries below those bounds keep 0. Lane-parallel over the sphere, summed in offset order as
-// dg_average_kernel does.
-template <bool SECOND>
-__global__ __launch_bounds__(kAvgBlock) void curvature_average_kernel(const SphereArgs P)
-{
-    __shared__ uint16_t s_list[kAvgCells];
-    __shared__ int s_count;
-    const StepArgs& A = P.s;
-    const int64_t N = A.ncells;
-    const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * kAvgCells;
-    if (wave == 0) {
-        const int64_t c0 = base + lane;
-        const bool inter = lane < kAvgCells && c0 < N && ListCode<double>::count(A.cnt_in[c0]) >= 2;
-        const unsigned long long m = __ballot(inter);
-        if (inter) s_list[__popcll(m & ((1ull << lane) - 1ull))] = static_cast<uint16_t>(lane);
-        if (lane == 0) s_count = __popcll(m);
-    }
-    __syncthreads();
-    const int ninter = s_count;
-    const int64_t nyz = static_cast<int64_t>(A.ny) * A.nz;
-    const double* src = SECOND ? P.tmp : P.raw;
-    for (int i = wave; i < ninter; i += kAvgWaves) {
-        const int64_t c = base + s_list[i];
-        const uint8_t code = A.cnt_in[c];
-        const int n = ListCode<double>::count(code);
-        const int x = static_cast<int>(c / nyz), y = static_cast<int>((c / A.nz) % A.ny), z = static_cast<int>(c % A.nz);
-        for (int b = 1; b < n; ++b)
-            for (int a = 0; a < b; ++a) {
-                const uint32_t ga = A.id_in[static_cast<int64_t>(a) * N + c], gb = A.id_in[static_cast<int64_t>(b) * N + c];
-                const int plane = pair_plane(a, b);
-                const double w = sqrt(entry_value<double>(A, c, code, a) * entry_value<double>(A, c, code, b));
-                double result = 0.0;
-                if (SECOND ? (w > DBL_EPSILON) : (w > P.threshold)) {
-                    double value = 0.0, sum = 0.0;
-                    int counter = 0;
-                    for (int t0 = 0; t0 < P.noff; t0 += 64) {
-                        const int t = t0 + lane;
-                        bool ok = false;
-                        double wt = 0.0, term = 0.0;
-                        if (t < P.noff) {
-                            const int ii = P.off[3 * t], jj = P.off[3 * t + 1], kk = P.off[3 * t + 2];
-                            const int64_t nb = (static_cast<int64_t>(wrap1(x + ii, A.nx)) * A.ny + wrap1(y + jj, A.ny)) * A.nz +
-                                               wrap1(z + kk, A.nz);
-                            double wphi = 0.0;
-                            int np = 0;
-                            bool fwd = true;
-                            if (find_pair<double>(A, nb, ga, gb, wphi, np, fwd)) {
-                                const double v = src[static_cast<int64_t>(np) * N + nb];
-                                if (SECOND) {
-                                    ok = wphi > P.threshold;
-                                    term = fwd ? v : -v;
-                                } else {
-                                    wt = wphi * P.off_w[t];
-                                    ok = wt > DBL_EPSILON;
-                                    term = wt * (fwd ? v : -v);
-                                }
-                            }
-                        }
-                        unsigned long long okm = __ballot(ok);
-                        while (okm) {
-                            const int l = __ffsll(static_cast<long long>(okm)) - 1;
-                            okm &= okm - 1ull;
-                            if (SECOND) counter++;
-                            else sum += lane_value(wt, l);
-                            value += lane_value(term, l);
-                        }
-                    }
-                    if (SECOND) result = counter != 0 ? value / static_cast<double>(counter) : P.tmp[static_cast<int64_t>(plane) * N + c];
-                    else result = sum > DBL_EPSILON ? value / sum : 0.0;
-                }
-                if (lane == 0) (SECOND ? P.avg : P.tmp)[static_cast<int64_t>(plane) * N + c] = result;
-            }
-    }
-}
-
 // ---- both averagings on staged tiles
 
 constexpr int kSphereBlock = kSphereCells;     // threads of a block
@@ -389,7 +454,7 @@ __device__ __forceinline__ uint32_t listed_grain(const StepArgs& A, unsigned lon
 }
 
 // SECOND = false: CollectAverage into tmp; true: DistributeAverage into avg, of the driving force or
-// (CURV) of the curvature: the sums of dg_average_kernel and curvature_average_kernel, on tiles.
+// (CURV) of the curvature: the sums of sphere_wave_kernel, on tiles.
 //
 // A block stages the lists' grains of its tile plus the sphere's reach in LDS, and then takes the
 // pairs of grains its cells hold one after another (ascending): the pair's weight and value at every
@@ -400,9 +465,9 @@ __device__ __forceinline__ uint32_t listed_grain(const StepArgs& A, unsigned lon
 // and not once per cell and offset, and a wavefront holds 64 cells' sums instead of one. What
 // bounds it is the chain of the sums (an LDS read and about 11 instructions per offset) of the
 // pairs that only a few of the tile's cells hold. Collect / Distribute of the curvature, 93
-// offsets, 160^3: 7.66 / 5.70 ms a wavefront at a time, 1.68 / 1.54 ms on tiles. The driving force
-// with 485 offsets, 96^3: 0.64 / 1.88 ms a wavefront at a time, 0.61 / 2.70 ms on tiles: so tiles
-// are staged up to kSphereOffsets offsets.
+// offsets, 160^3: 7.66 / 5.70 ms when a wavefront took a cell, 1.68 / 1.54 ms on tiles. The driving
+// force with 485 offsets, 96^3: 0.31 / 1.32 ms a wavefront per cell, 0.61 / 2.70 ms on tiles: so
+// tiles are staged up to kSphereOffsets offsets.
 template <typename TV, bool CURV, bool SECOND>
 __global__ __launch_bounds__(kSphereBlock) void sphere_tile_kernel(const SphereArgs P)
 {
@@ -603,13 +668,8 @@ static void launch_sphere(const SphereArgs& a, hipStream_t s)
         hipLaunchKernelGGL((sphere_tile_kernel<TV, CURV, true>), grid, dim3(kSphereBlock), lds, s, a);
     } else {
         const dim3 grid(static_cast<unsigned>((a.s.ncells + kAvgCells - 1) / kAvgCells));
-        if constexpr (CURV) {
-            hipLaunchKernelGGL((curvature_average_kernel<false>), grid, dim3(kAvgBlock), 0, s, a);
-            hipLaunchKernelGGL((curvature_average_kernel<true>), grid, dim3(kAvgBlock), 0, s, a);
-        } else {
-            hipLaunchKernelGGL((dg_average_kernel<TV, false>), grid, dim3(kAvgBlock), 0, s, a);
-            hipLaunchKernelGGL((dg_average_kernel<TV, true>), grid, dim3(kAvgBlock), 0, s, a);
-        }
+        hipLaunchKernelGGL((sphere_wave_kernel<TV, false, CURV>), grid, dim3(kAvgBlock), 0, s, a);
+        hipLaunchKernelGGL((sphere_wave_kernel<TV, true, CURV>), grid, dim3(kAvgBlock), 0, s, a);
     }
 }
 
