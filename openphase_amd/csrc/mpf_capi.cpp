@@ -452,7 +452,8 @@ mpf_status enqueue_step(mpf_ctx* c, double dt, hipStream_t stream)
 // The sphere of radius `range`: the loop bounds and distance weights of CollectAverage /
 // DistributeAverage (src/DrivingForce.cpp:295-324, src/InterfaceRegularization.cpp:198-213), and the
 // tile the averaging kernels stage with it: 8 x 8 x 8 cells in 3D (4 x 8 x 8 where that lets a second
-// block onto a CU), 16 x 32 in 2D, 256 in 1D; none when that does not fit LDS.
+// block onto a CU), 16 x 32 in 2D, 256 in 1D; none when that does not fit LDS, on small grids and for
+// large spheres (sphere_wave_kernel has both sides' times).
 void make_sphere(const mpf_ctx* c, int range, mpf_sphere* p)
 {
     const int n[3] = {c->nx, c->ny, c->nz}, d[3] = {c->dnx, c->dny, c->dnz};
@@ -477,7 +478,8 @@ void make_sphere(const mpf_ctx* c, int range, mpf_sphere* p)
     auto box = [&](int q) { return p->tile[q] + 2 * p->reach[q]; };
     auto bytes = [&]() { return static_cast<int64_t>(box(0)) * box(1) * (box(2) * mpf::kSphereCellBytes + 4); };
     if (c->active == 3 && bytes() > 78 * 1024) p->tile[0] = std::min(4, n[0]);
-    if (p->w.size() > mpf::kSphereOffsets || bytes() > mpf::kSphereLds || box(2) > mpf::kSphereCells) {
+    const size_t most = c->active == 2 ? mpf::kSphereOffsets2d : mpf::kSphereOffsets;
+    if (c->ncells < mpf::kSphereGrid || p->w.size() > most || bytes() > mpf::kSphereLds || box(2) > mpf::kSphereCells) {
         p->tile[0] = p->tile[1] = p->tile[2] = 0;
         return;
     }

@@ -164,6 +164,8 @@ struct SphereArgs {
 };
 constexpr int kAvgBlock = 256;
 constexpr int kSphereOffsets = 256;      // offsets up to which tiles are staged
+constexpr int kSphereOffsets2d = 64;     // the same in 2D
+constexpr int64_t kSphereGrid = int64_t{1} << 18;  // cells from which tiles are staged: fewer leave CUs idle
 constexpr int kSphereCells = 512;        // cells of a staged tile at most
 constexpr int kSphereCellBytes = 25;     // LDS per staged cell
 constexpr int kSphereLds = 150 * 1024;   // LDS of a staged tile at most

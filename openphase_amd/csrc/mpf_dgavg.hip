@@ -211,6 +211,10 @@ __device__ __forceinline__ int ordered_add(double (&buf)[64 * kAvgChunks + 8][2]
 // What bounds it is the lookups' round trips. 96^3, 485 offsets (collect / distribute): lists looked up
 // for each pair anew and terms read from lane registers 0.64 / 1.88 ms, terms added from LDS and two
 // chunks in flight 0.33 / 1.74 ms, lists looked up once for all pairs of a cell 0.31 / 1.32 ms.
+// Tiles against this kernel (ms, 20 steps in 2D, 4 in 3D): curvature, 25 offsets in 2D and 93 in 3D,
+// 256^2 4.07 / 3.63, 512^2 5.36 / 6.51, 48^3 5.89 / 3.77, 64^3 5.40 / 5.91, 96^3 8.17 / 10.6: tiles from
+// kSphereGrid cells on. Driving force, 69 offsets in 2D, 128^2 3.03 / 1.95, 512^2 4.86 / 3.75: in 2D two
+// chunks hold the sphere, and tiles stay to kSphereOffsets2d.
 template <typename TV, bool SECOND, bool CURV>
 __global__ __launch_bounds__(kAvgBlock) void sphere_wave_kernel(const SphereArgs P)
 {
@@ -327,7 +331,8 @@ __global__ __launch_bounds__(kAvgBlock) void sphere_wave_kernel(const SphereArgs
 
 // ---- interface regularization (FP64 state) -------------------------------------------------
 
-constexpr int kRawCells = 256;     // cells per block (one wavefront) of the raw pass
+constexpr int kRawCells = 256;     // most cells per block (one wavefront) of the raw pass
+constexpr int kRawWaves = 8192;    // wavefronts that fill the chip: 1024 SIMDs x 8
 
 // The curvature DoubleObstacle's regularization overload adds per pair of non-zero entries of a
 // wide-interface cell (src/DoubleObstacle.cpp:702-763): loc_increment (the pair's increment before
@@ -408,19 +413,19 @@ __device__ __forceinline__ bool raw_cell(const CurvArgs& P, bool run, int64_t c,
 // an overflow). What bounds it is the instructions of the list walk; one thread per cell with
 // register lists took 4.0 ms at 160^3 (256 VGPRs and spills, one wavefront per SIMD), now 1.23 ms.
 template <bool GRAD>
-__global__ __launch_bounds__(64) void curvature_raw_kernel(const CurvArgs P)
+__global__ __launch_bounds__(64) void curvature_raw_kernel(const CurvArgs P, int cells)
 {
     constexpr int G = kGroupLanes, C = 64 / G;
     __shared__ GroupArena<double, GRAD> mem;
     __shared__ uint16_t pairs[kPairTable];
     __shared__ uint16_t s_list[kRawCells];
     const int lane = static_cast<int>(threadIdx.x);
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * kRawCells;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * cells;
     fill_pairs(pairs);
     int n = 0;
-    for (int k = 0; k < kRawCells; k += 64) {
+    for (int k = 0; k < cells; k += 64) {
         const int64_t c = base + k + lane;
-        const bool in = c < P.s.ncells && ListCode<double>::count(P.s.cnt_in[c]) >= 2;
+        const bool in = k + lane < cells && c < P.s.ncells && ListCode<double>::count(P.s.cnt_in[c]) >= 2;
         const unsigned long long m = __ballot(in);
         if (in) s_list[n + __popcll(m & ((1ull << lane) - 1ull))] = static_cast<uint16_t>(k + lane);
         n += __popcll(m);
@@ -692,9 +697,14 @@ int sphere_lds_limit()
 int launch_curvature(const CurvArgs& a, void* stream)
 {
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const dim3 raw_grid(static_cast<unsigned>((a.s.ncells + kRawCells - 1) / kRawCells));
-    if (a.grad) hipLaunchKernelGGL((curvature_raw_kernel<true>), raw_grid, dim3(64), 0, s, a);
-    else hipLaunchKernelGGL((curvature_raw_kernel<false>), raw_grid, dim3(64), 0, s, a);
+    // a wavefront takes 256 cells, whose interface cells fill its groups of lanes; fewer on a grid that
+    // would not give every SIMD eight wavefronts: 20 regularized steps 64^2 6.0 -> 2.7 ms, 512^2 6.5 -> 5.4 ms,
+    // four at 96^3 8.6 -> 8.2 ms
+    int cells = kRawCells;
+    while (cells > 64 / kGroupLanes && a.s.ncells / cells < kRawWaves) cells /= 2;
+    const dim3 raw_grid(static_cast<unsigned>((a.s.ncells + cells - 1) / cells));
+    if (a.grad) hipLaunchKernelGGL((curvature_raw_kernel<true>), raw_grid, dim3(64), 0, s, a, cells);
+    else hipLaunchKernelGGL((curvature_raw_kernel<false>), raw_grid, dim3(64), 0, s, a, cells);
     launch_sphere<double, true>(a.sphere, s);
     return static_cast<int>(hipGetLastError());
 }

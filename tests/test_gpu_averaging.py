@@ -41,3 +41,22 @@ def test_curvature(dims, reach):
                      curvature_factor=0.7, reg_range=reach, reg_threshold=0.02)
     print(f"curvature {dims} range {reach}", flush=True)
     _compare(cfg, 7, 6, seed=23 * reach)
+
+
+@pytest.mark.parametrize("dims,reach", [((521, 509, 0), 3), ((67, 61, 65), 2)])
+def test_curvature_on_tiles(dims, reach):
+    # at least 2^18 cells: the averages are formed on staged tiles, here with remainders on every axis
+    cfg = StepConfig(*dims, slots=16, nucleus_volume_factor=1e-3, regularization=True, regularization_factor=1.5,
+                     curvature_factor=0.7, reg_range=reach, reg_threshold=0.02)
+    print(f"curvature on tiles {dims} range {reach}", flush=True)
+    _compare(cfg, 4, 3, seed=23 * reach)
+
+
+@pytest.mark.parametrize("weights", [0, 1, 2])
+def test_driving_force_on_tiles(weights):
+    cfg = StepConfig(521, 509, 0, nphases=2, sigma=np.full((2, 2), 0.24), mu=np.full((2, 2), 4e-9), slots=16,
+                     nucleus_volume_factor=1e-3, dg_mode=np.array([[0, 1], [1, 0]], np.int32),
+                     dg_value=np.array([[0.0, 1e5], [-7e4, 0.0]]), dg_average=True, dg_range=3, dg_threshold=0.05,
+                     dg_weights=weights)
+    print(f"driving force on tiles, weights {weights}", flush=True)
+    _compare(cfg, 4, 3, seed=31)
