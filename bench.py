@@ -127,7 +127,7 @@ def run_gpu(precision: int, lists, steps: int, warmup: int):
 
 
 PROFILE = ROOT / "profiles" / "mpf_step_256cube_1000grains.md"
-MAIN_KERNEL = "tile_kernel<double, double, false, false, true>"
+MAIN_KERNEL = "tile_kernel<double, double, false, false, true, false>"
 
 
 def profiled_traffic(kernel: str = MAIN_KERNEL):
