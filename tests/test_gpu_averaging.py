@@ -1,5 +1,5 @@
-"""Averaging over the interface (driving force, curvature) on staged tiles and, for spheres that do not
-fit LDS, per wavefront: ragged grids, every reach, lists of up to six entries, against the oracle."""
+"""Averaging over the interface (driving force, curvature) with a wavefront per cell (small grids, large
+spheres) and on staged tiles: ragged grids, every reach, lists of up to six entries, against the oracle."""
 import numpy as np
 import pytest
 
@@ -22,7 +22,7 @@ def _compare(cfg, pool, longest, seed):
     assert np.abs(got.value - exp.value).max() <= TOL
 
 
-# Range 9 in 3D does not fit LDS, Range 6 leaves one block per CU, Range 5 takes the smaller tile
+# spheres of one chunk of offsets, of several, and longer than the grid
 @pytest.mark.parametrize("dims,reach", [((33, 19, 0), 3), ((12, 50, 0), 5), ((9, 8, 10), 3), ((13, 9, 10), 5), ((12, 9, 11), 6),
                                         ((9, 10, 11), 9), ((40, 0, 0), 4)])
 @pytest.mark.parametrize("weights", [0, 1, 2])
