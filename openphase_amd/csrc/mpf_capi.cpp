@@ -341,12 +341,7 @@ unsigned grain_blocks(const mpf_ctx* c)
     return static_cast<unsigned>((n + mpf::kGrainBlock - 1) / mpf::kGrainBlock);
 }
 
-// Wavefronts of the deferred-cell kernel: no more than one per 32 cells of the domain, which is one
-// per round of four cells while up to an eighth of the cells are deferred.
-int deferred_blocks(const mpf_ctx* c)
-{
-    return static_cast<int>(std::min<int64_t>(c->deferred_grid, (c->ncells + 255) / 256 * 8));
-}
+int deferred_blocks(const mpf_ctx* c) { return mpf::deferred_blocks(c->ncells, c->deferred_grid); }
 
 // Makes the device copies of the kernel arguments current for time step dt (both parities).
 // Uploads only when something changed (dt, tables, launch shape, grains); then it waits for the
@@ -1539,11 +1534,12 @@ mpf_status mpf_autotune(mpf_ctx* c, double dt, int32_t steps, int32_t* xcd_order
         c->tile_z = best_tz;
     }
     // 2. block order of the step kernel x grid of the deferred-cell kernel
-    const int grids[4] = {256, 1024, 4096, 16384};
+    int grids[mpf::kDeferredTrials];
+    const int ngrids = mpf::deferred_trials(c->ncells, grids);
     best = 1e30f;
     int best_x = x0, best_g = g0;
     for (int x = 0; x < 2 && !st; ++x)
-        for (int gi = 0; gi < 4 && !st; ++gi) {
+        for (int gi = 0; gi < ngrids && !st; ++gi) {
             c->xcd_order = x;
             c->deferred_grid = grids[gi];
             float ms = 0.f;

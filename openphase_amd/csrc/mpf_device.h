@@ -185,6 +185,27 @@ struct CurvArgs {
 };
 int launch_curvature(const CurvArgs& a, void* stream);
 
+// Wavefronts of the deferred-cell kernel given its grid: no more than one per 32 cells of the domain,
+// which is one per round of four cells while up to an eighth of the cells are deferred.
+inline int deferred_blocks(int64_t ncells, int grid)
+{
+    const int64_t most = (ncells + 255) / 256 * 8;
+    return static_cast<int>(grid < most ? grid : most);
+}
+
+// The grids of the deferred-cell kernel the autotuner times, the default among them (256^3 FP64: the
+// kernel takes 1.19 ms at 4096 wavefronts, 1.07 at the default 6144, 1.33 at 16384): those that are
+// another launch than the ones before. Returns how many.
+constexpr int kDeferredGrids[] = {256, 1024, 4096, kWideGrid, 16384};
+constexpr int kDeferredTrials = sizeof(kDeferredGrids) / sizeof(kDeferredGrids[0]);
+inline int deferred_trials(int64_t ncells, int (&grids)[kDeferredTrials])
+{
+    int n = 0;
+    for (int g : kDeferredGrids)
+        if (n == 0 || deferred_blocks(ncells, g) != deferred_blocks(ncells, grids[n - 1])) grids[n++] = g;
+    return n;
+}
+
 // Host-side launchers (mpf_kernels.hip); return a hipError_t value. The step, deferred-cell and
 // grain kernels run over one or several domains of the same kernel variant in one launch: `args`
 // (device memory) holds one argument block per domain and `first` (device, ndom + 1 entries) the
