@@ -158,7 +158,7 @@ __device__ __forceinline__ GroupList<TC> group_gather(const StepArgs& A, bool ru
         for (int t = 0; t < CAP; ++t)
             if (t < n0 && t != imp0) others += M.phi[t];
         __syncthreads();
-        if (l < n0 && l == imp0) {
+        if (l < CAP && l < n0 && l == imp0) {
             phi = 1.0 - others;
             M.phi[l] = phi;
         }

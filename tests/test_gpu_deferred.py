@@ -111,3 +111,20 @@ def test_single_precision_lists(pool, longest):
     exp, _ = _step(O.Oracle, _config("two", (7, 6, 5)), lists, pool, dt)
     # one step in FP32: increments of order 1 with 24-bit terms that cancel to a few per cent
     assert np.abs(_dense(got, pool) - _dense(exp, pool)).max() <= 1e-5
+
+
+# the entry an FP32 list holds implicitly (the largest) beyond the eighth slot
+@pytest.mark.parametrize("longest", [9, 15])
+def test_single_precision_lists_with_a_late_implicit_entry(longest):
+    cfg = _config("two", (7, 6, 5), precision=1)
+    lists = _random_lists(cfg.shape, 15, longest, seed=longest)
+    off = lists.offsets()
+    for c in np.flatnonzero(lists.count > 8):
+        v = lists.value[off[c]:off[c + 1]]
+        v.sort()
+    dt = 0.5 * cfg.max_time_step()
+    print(f"fp32 late implicit entry, longest {longest}", flush=True)
+    got, _ = _step(Engine, cfg, lists, 15, dt)
+    exp, _ = _step(O.Oracle, _config("two", (7, 6, 5)), lists, 15, dt)
+    # one step in FP32: increments of order 1 with 24-bit terms that cancel to a few per cent
+    assert np.abs(_dense(got, 15) - _dense(exp, 15)).max() <= 1e-5
