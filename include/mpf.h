@@ -182,7 +182,8 @@ typedef enum mpf_ip_state {
  * 4 E (phi_a phi_b - Eta^2/Pi^2 grad_a . grad_b) / Eta, E the pair's energy from the IP.Set state
  * named by ip_state (0 for a pair absent there). Summed on the device in a fixed order (the same
  * from run to run; the reference's sequential sum differs in rounding only). MPF_IP_PREVIOUS needs
- * a step since the last upload / restore / finalize. */
+ * a step since the last upload / restore / finalize. MPF_SLOT_OVERFLOW when a cell's merged list is
+ * longer than a step takes (16 entries), in the current state or the one IP.Set saw. */
 mpf_status mpf_interface_energy(mpf_ctx* ctx, int32_t ip_state, double* sum);
 
 /* PhaseField::CalculateFractions (src/PhaseField.cpp:411-423), which the reference runs in every

@@ -1090,11 +1090,23 @@ mpf_status mpf_interface_energy(mpf_ctx* c, int32_t ip_state, double* sum)
     a.status = c->d_status + 3;
     const int32_t zero = 0;
     int32_t flag = 0;
-    mpf_status st = c->hip(hipMemcpyAsync(a.status, &zero, sizeof(zero), hipMemcpyHostToDevice, c->stream), "status reset");
-    if (!st) st = c->hip(static_cast<hipError_t>(mpf::launch_energy(a, c->fp32, c->d_energy + nb, c->stream)), "energy kernels");
-    if (!st) st = c->hip(hipMemcpyAsync(sum, c->d_energy + nb, sizeof(double), hipMemcpyDeviceToHost, c->stream), "energy readback");
-    if (!st) st = c->hip(hipMemcpyAsync(&flag, a.status, sizeof(flag), hipMemcpyDeviceToHost, c->stream), "status readback");
-    if (!st) st = c->hip(hipStreamSynchronize(c->stream), "stream synchronize");
+    unsigned long long overflow = ~0ull;
+    auto sum_energy = [&]() {
+        mpf_status e = c->hip(hipMemcpyAsync(a.status, &zero, sizeof(zero), hipMemcpyHostToDevice, c->stream), "status reset");
+        if (!e) e = c->hip(static_cast<hipError_t>(mpf::launch_energy(a, c->fp32, c->d_energy + nb, c->stream)), "energy kernels");
+        if (!e) e = c->hip(hipMemcpyAsync(sum, c->d_energy + nb, sizeof(double), hipMemcpyDeviceToHost, c->stream), "energy readback");
+        if (!e) e = c->hip(hipMemcpyAsync(&flag, a.status, sizeof(flag), hipMemcpyDeviceToHost, c->stream), "status readback");
+        if (!e) e = c->hip(hipMemcpyAsync(&overflow, c->d_first_overflow, sizeof(overflow), hipMemcpyDeviceToHost, c->stream), "status readback");
+        if (!e) e = c->hip(hipStreamSynchronize(c->stream), "stream synchronize");
+        return e;
+    };
+    mpf_status st = sum_energy();
+    // only the form with the lists of the state IP.Set saw finds one that is too long there; a step from
+    // such a state has reported a cell
+    if (!st && !flag && !a.full && ip_state == MPF_IP_PREVIOUS && overflow != ~0ull) {
+        a.full = 1;
+        st = sum_energy();
+    }
     if (!st && flag) st = c->fail(MPF_SLOT_OVERFLOW, "a cell's merged list exceeds 16 entries");
     return st;
 }

@@ -128,3 +128,63 @@ def test_single_precision_lists_with_a_late_implicit_entry(longest):
     exp, _ = _step(O.Oracle, _config("two", (7, 6, 5)), lists, 15, dt)
     # one step in FP32: increments of order 1 with 24-bit terms that cancel to a few per cent
     assert np.abs(_dense(got, 15) - _dense(exp, 15)).max() <= 1e-5
+
+
+def _vanishing(grains):
+    """9 x 9 cells, an interface of grains 0 and 1 along x, and around cell (4, 4) sixteen entries of
+    `grains` other grains so small that the next step erases most of them: that cell's merged list is
+    `grains` + 2 long before the step and shorter after it."""
+    lists, n = [], 0
+    for x in range(9):
+        for y in range(9):
+            cell = {0: 1.0} if x <= 4 else ({0: 0.5, 1: 0.5} if x == 5 else {1: 1.0})
+            if max(abs(x - 4), abs(y - 4)) == 1:
+                for _ in range(2):
+                    cell[2 + n % grains] = 1e-5
+                    n += 1
+                cell[max(cell, key=cell.get)] -= 2e-5
+            lists.append(cell)
+    return Lists((9, 9, 1), np.array([len(c) for c in lists], np.int32), np.array([g for c in lists for g in c], np.int32),
+                 np.array([v for c in lists for v in c.values()]))
+
+
+@pytest.mark.parametrize("model", ["iso", "two"])
+def test_energy_of_a_vanished_list(model):
+    """Energies with the pairs of the state before the step, where one list was long (16 entries of other
+    grains in the box, 12 grains merged), against the oracle."""
+    cfg = _config(model, (9, 9, 0))
+    lists = _vanishing(10)
+    eng, orc = Engine(cfg), O.Oracle(cfg)
+    for e in (eng, orc):
+        e.set_grains(np.arange(12, dtype=np.int32) % cfg.nphases)
+        e.upload(lists)
+        e.finalize_initialization()
+        if e is orc:
+            orc.keep_step_start(True)
+        e.step(cfg.max_time_step(), 1)
+    assert np.array_equal(eng.download().index, orc.download().index)
+    for ip in ("previous", "current"):
+        # sums of about 100 terms
+        assert eng.interface_energy(ip) == pytest.approx(orc.interface_energy(ip), rel=1e-12)
+    eng.close()
+    orc.close()
+
+
+@pytest.mark.parametrize("model", ["iso", "two", "cubic"])
+def test_energy_refuses_a_list_no_step_takes(model):
+    """18 grains merged in one cell: the step reports the cell, and so does the energy with the pairs of
+    the state before that step, for every form of the tables; the lists after it are short enough."""
+    cfg = _config(model, (9, 9, 0))
+    _, rot = random_rotations(18, seed=3)
+    e = Engine(cfg)
+    e.set_grains(np.arange(18, dtype=np.int32) % cfg.nphases, rot)
+    e.upload(_vanishing(16))
+    e.finalize_initialization()
+    with pytest.raises(_capi.MpfError) as err:
+        e.step(cfg.max_time_step(), 1)
+    assert err.value.status == _capi.MPF_SLOT_OVERFLOW and e.overflow_cell() == 4 * 9 + 4
+    assert e.interface_energy("current") > 0.0
+    with pytest.raises(_capi.MpfError) as err:
+        e.interface_energy("previous")
+    assert err.value.status == _capi.MPF_SLOT_OVERFLOW
+    e.close()
