@@ -145,11 +145,13 @@ mpf_status mpf_step_async(mpf_ctx* ctx, double dt, int32_t nsteps);
 /* Blocks until all work on the context's stream is done; returns the accumulated status. */
 mpf_status mpf_synchronize(mpf_ctx* ctx);
 
-/* Total entries over all cells (size of the index/value download buffers). */
+/* Total entries over all cells (size of the index/value download buffers). Allocates nothing. */
 mpf_status mpf_total_entries(mpf_ctx* ctx, int64_t* total);
 
 /* PhaseField::Write (src/PhaseField.cpp:2340-2388) content: finalized lists in the same layout
- * as mpf_upload; flag (0/1/2) per cell may be NULL. */
+ * as mpf_upload; flag (0/1/2) per cell may be NULL. Packed on the device in a staging buffer of the
+ * lists' size but at most 128 MiB (less where memory is short), which the context keeps for the next
+ * download until mpf_destroy. */
 mpf_status mpf_download(mpf_ctx* ctx, int32_t* count, int32_t* index, double* value, int8_t* flag);
 
 /* GrainsProperties Volume and VolumeRatio per grain (either may be NULL). */

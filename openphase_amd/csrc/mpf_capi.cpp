@@ -41,6 +41,22 @@ template <typename T> void h2d(hipError_t& e, T* dst, const T* src, size_t n)
     if (e == hipSuccess) e = hipMemcpy(dst, src, n * sizeof(T), hipMemcpyHostToDevice);
 }
 
+// Makes a device current for a call that allocates or launches on it, whichever the caller's thread has.
+struct DeviceScope {
+    int back = -1;
+    explicit DeviceScope(int device)
+    {
+        int now = 0;
+        if (hipGetDevice(&now) == hipSuccess && now != device && hipSetDevice(device) == hipSuccess) back = now;
+    }
+    ~DeviceScope()
+    {
+        if (back >= 0) (void)hipSetDevice(back);
+    }
+    DeviceScope(const DeviceScope&) = delete;
+    DeviceScope& operator=(const DeviceScope&) = delete;
+};
+
 }  // namespace
 
 // Averaging sphere of a context: offsets (3 each), their distance weights, and the staged tile.
@@ -55,6 +71,7 @@ struct mpf_sphere {
 
 struct mpf_ctx {
     mpf_grid grid{};
+    int device = 0;                  // the device current at creation
     int nx = 1, ny = 1, nz = 1, dnx = 0, dny = 0, dnz = 0, active = 0;
     int64_t ncells = 0;
     int slots = 8;
@@ -500,6 +517,18 @@ void free_sphere(mpf_sphere* p)
     dfree(p->d_off); dfree(p->d_tile_off); dfree(p->d_w);
 }
 
+// Staging of packed lists for host downloads: one block of cells at creation, so that a download never
+// lacks memory, and at most 128 MiB after one.
+constexpr size_t kPackStage = size_t{128} << 20;
+constexpr size_t kPackCellBytes = sizeof(int32_t) + sizeof(int8_t);                 // count, flag
+constexpr size_t kPackEntryBytes = sizeof(int32_t) + sizeof(double);                // index, value
+
+size_t pack_least(const mpf_ctx* c)
+{
+    const size_t cells = static_cast<size_t>(std::min<int64_t>(c->ncells, mpf::kPackCells));
+    return cells * (kPackCellBytes + static_cast<size_t>(c->slots) * kPackEntryBytes) + 1024;
+}
+
 mpf_status read_status(mpf_ctx* c)
 {
     int32_t st[mpf::kStatusWords];
@@ -659,6 +688,7 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
 
     const size_t N = static_cast<size_t>(c->ncells);
     mpf_status s = MPF_OK;
+    if ((s = c->hip(hipGetDevice(&c->device), "hipGetDevice"))) return bail(s, c->err.c_str());
     if ((s = c->hip(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate"))) return bail(s, c->err.c_str());
     for (int b = 0; b < 2; ++b) {
         if ((s = c->hip(dalloc(&c->cnt[b], N), "hipMalloc counts"))) return bail(MPF_ERR_NOMEM, c->err.c_str());
@@ -673,8 +703,11 @@ mpf_status mpf_create(const mpf_grid* grid, const mpf_params* params, mpf_ctx** 
         c->hip(dalloc(&c->d_status, mpf::kStatusWords), "status") ||
         c->hip(dalloc(&c->d_first_overflow, 1), "status") || c->hip(dalloc(&c->d_warnings, 1), "status") ||
         c->hip(dalloc(&c->d_work_list, N), "work list") || c->hip(dalloc(&c->d_work_count, 3), "work list") ||
-        c->hip(dalloc(&c->d_stats, 2), "statistics") || c->hip(dalloc(&c->d_obs, 4), "statistics"))
+        c->hip(dalloc(&c->d_stats, 2), "statistics") || c->hip(dalloc(&c->d_obs, 4), "statistics") ||
+        c->hip(dalloc(&c->d_pack_offset, static_cast<size_t>(mpf::pack_blocks(c->ncells)) + 1), "list offsets") ||
+        c->hip(dalloc(&c->d_pack, pack_least(c)), "packed lists"))
         return bail(MPF_ERR_NOMEM, c->err.c_str());
+    c->pack_cap = pack_least(c);
     if (c->reg_active && c->reg_average) {
         const size_t pairs = static_cast<size_t>(c->slots) * (c->slots - 1) / 2;
         if (c->hip(dalloc(&c->d_curv_raw, pairs * N), "regularization arrays") ||
@@ -912,34 +945,25 @@ namespace {
 // Running sums of the current state's entries by block of cells, on the device.
 mpf_status pack_offsets(mpf_ctx* c)
 {
-    if (!c->d_pack_offset &&
-        c->hip(dalloc(&c->d_pack_offset, static_cast<size_t>(mpf::pack_blocks(c->ncells)) + 1), "list offsets"))
-        return MPF_ERR_NOMEM;
     return c->hip(static_cast<hipError_t>(mpf::launch_pack_offsets(c->cnt[c->cur], c->ncells, c->fp32, c->d_pack_offset, c->stream)),
                   "list offset kernels");
 }
 
-// Staging of packed lists: at most 128 MiB, held by the context; smaller parts where that cannot be had.
-constexpr size_t kPackStage = size_t{128} << 20;
-constexpr size_t kPackCellBytes = sizeof(int32_t) + sizeof(int8_t);                 // count, flag
-constexpr size_t kPackEntryBytes = sizeof(int32_t) + sizeof(double);                // index, value
-constexpr size_t kPackLeast = mpf::kPackCells * (kPackCellBytes + mpf::kMaxSlots * kPackEntryBytes) + 1024;  // one block
-
-mpf_status pack_stage(mpf_ctx* c, size_t want)
+// Grows the staging of packed lists towards `want` bytes. What cannot be had is done without: the lists
+// then go in more parts.
+void pack_stage(mpf_ctx* c, size_t want)
 {
-    want = std::max(std::min(want, kPackStage), kPackLeast);
-    if (c->pack_cap >= want) return MPF_OK;
-    for (size_t n = want; n >= std::max(kPackLeast, c->pack_cap + 1); n = n > kPackLeast ? std::max(n / 2, kPackLeast) : 0) {
+    want = std::min(want, kPackStage);
+    for (size_t n = want; n > c->pack_cap; n /= 2) {
         unsigned char* p = nullptr;
         if (dalloc(&p, n) == hipSuccess) {
             dfree(c->d_pack);
             c->d_pack = p;
             c->pack_cap = n;
-            return MPF_OK;
+            return;
         }
         (void)hipGetLastError();
     }
-    return c->pack_cap >= kPackLeast ? MPF_OK : c->fail(MPF_ERR_NOMEM, "no device memory for the packed lists");
 }
 
 }  // namespace
@@ -950,6 +974,7 @@ mpf_status mpf_total_entries(mpf_ctx* c, int64_t* total)
 {
     if (!c || !total) return MPF_ERR_ARG;
     if (!c->have_state) return c->fail(MPF_ERR_STATE, "no state");
+    const DeviceScope scope(c->device);
     mpf_status s = pack_offsets(c);
     if (!s) s = c->hip(hipMemcpyAsync(total, c->d_pack_offset + mpf::pack_blocks(c->ncells), sizeof(*total), hipMemcpyDeviceToHost,
                                       c->stream), "download counts");
@@ -961,14 +986,15 @@ mpf_status mpf_download(mpf_ctx* c, int32_t* count, int32_t* index, double* valu
 {
     if (!c) return MPF_ERR_ARG;
     if (!c->have_state) return c->fail(MPF_ERR_STATE, "no state");
+    const DeviceScope scope(c->device);
     const int64_t N = c->ncells, nb = mpf::pack_blocks(N);
     mpf_status s = pack_offsets(c);
     if (s) return s;
     std::vector<int64_t> off(static_cast<size_t>(nb) + 1);
     s = c->hip(hipMemcpyAsync(off.data(), c->d_pack_offset, off.size() * sizeof(int64_t), hipMemcpyDeviceToHost, c->stream), "download");
     if (!s) s = c->hip(hipStreamSynchronize(c->stream), "sync");
-    if (!s) s = pack_stage(c, static_cast<size_t>(N) * kPackCellBytes + static_cast<size_t>(off[nb]) * kPackEntryBytes + 1024);
     if (s) return s;
+    pack_stage(c, static_cast<size_t>(N) * kPackCellBytes + static_cast<size_t>(off[nb]) * kPackEntryBytes + 1024);
     const mpf::StepArgs a = step_args(c, 1.0, c->cur);
     auto up = [](size_t x) { return (x + 255) & ~size_t{255}; };
     for (int64_t b0 = 0; b0 < nb;) {
