@@ -6,6 +6,7 @@ import pytest
 from openphase_amd.engine import Engine, StepConfig
 import oracle as O
 from test_gpu_deferred import _random_lists, _step
+from test_gpu_deferred import _dense
 
 pytestmark = pytest.mark.gpu
 
@@ -60,3 +61,47 @@ def test_driving_force_on_tiles(weights):
                      dg_weights=weights)
     print(f"driving force on tiles, weights {weights}", flush=True)
     _compare(cfg, 4, 3, seed=31)
+
+
+# grids of at least 2^18 cells with remainders on every axis, of one, two and three axes, and lists of up to
+# six entries (beyond the four grains a staged cell holds)
+TILED = [((521, 509, 0), 4), ((521, 0, 509), 3), ((0, 521, 509), 2), ((262149, 0, 0), 5), ((67, 61, 65), 3), ((67, 61, 65), 4)]
+
+
+def _driving(dims, reach, weights, precision=0):
+    return StepConfig(*dims, nphases=2, sigma=np.full((2, 2), 0.24), mu=np.full((2, 2), 4e-9), slots=8,
+                      nucleus_volume_factor=1e-3, dg_mode=np.array([[0, 1], [1, 0]], np.int32),
+                      dg_value=np.array([[0.0, 1e5], [-7e4, 0.0]]), dg_average=True, dg_range=reach, dg_threshold=0.05,
+                      dg_weights=weights, precision=precision)
+
+
+@pytest.mark.parametrize("dims,reach", TILED)
+def test_driving_force_of_long_lists_on_tiles(dims, reach):
+    print(f"driving force of long lists on tiles {dims} range {reach}", flush=True)
+    _compare(_driving(dims, reach, reach % 3), 7, 6, seed=41 * reach)
+
+
+@pytest.mark.parametrize("dims,reach", TILED)
+def test_curvature_of_long_lists_on_tiles(dims, reach):
+    cfg = StepConfig(*dims, slots=8, nucleus_volume_factor=1e-3, regularization=True, regularization_factor=1.5,
+                     curvature_factor=0.7, reg_range=reach, reg_threshold=0.02)
+    print(f"curvature of long lists on tiles {dims} range {reach}", flush=True)
+    _compare(cfg, 7, 6, seed=43 * reach)
+
+
+@pytest.mark.parametrize("dims,reach", [TILED[0], TILED[4], ((33, 19, 0), 3)])
+def test_single_precision_driving_force(dims, reach):
+    """FP32 lists, on tiles and with a wavefront per cell. The values are multiples of 2^-16 that sum to 1,
+    which both precisions hold exactly: the weights are the same and the same terms count."""
+    lists = _random_lists((dims[0] or 1, dims[1] or 1, dims[2] or 1), 7, 6, seed=47 * reach)
+    first = np.cumsum(lists.count) - lists.count
+    v = np.maximum(np.floor(lists.value * 65536), 1.0)
+    v[first] += 65536 - np.add.reduceat(v, first)
+    lists.value[:] = v / 65536
+    assert lists.value.min() > 0
+    print(f"fp32 driving force {dims} range {reach}", flush=True)
+    dt = 0.3 * _driving(dims, reach, 0).max_time_step()
+    got, _ = _step(Engine, _driving(dims, reach, 0, precision=1), lists, 7, dt)
+    exp, _ = _step(O.Oracle, _driving(dims, reach, 0), lists, 7, dt)
+    # one step in FP32: increments of order 1 with 24-bit terms that cancel to a few per cent
+    assert np.abs(_dense(got, 7) - _dense(exp, 7)).max() <= 1e-5
