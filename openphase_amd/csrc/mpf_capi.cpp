@@ -277,7 +277,6 @@ mpf::StepArgs step_args(const mpf_ctx* c, double dt, int src)
     a.work_list = c->d_work_list;
     a.work_count = c->d_work_count;
     a.xcd_order = c->xcd_order;
-    a.deferred_grid = c->deferred_grid;
     a.tile_x = c->tile_x;
     a.tile_y = c->tile_y;
     a.tile_z = c->tile_z;
@@ -463,9 +462,8 @@ mpf_status enqueue_step(mpf_ctx* c, double dt, hipStream_t stream)
 
 // The sphere of radius `range`: the loop bounds and distance weights of CollectAverage /
 // DistributeAverage (src/DrivingForce.cpp:295-324, src/InterfaceRegularization.cpp:198-213), and the
-// tile the averaging kernels stage with it: 8 x 8 x 8 cells in 3D (4 x 8 x 8 where that lets a second
-// block onto a CU), 16 x 32 in 2D, 256 in 1D; none when that does not fit LDS, on small grids and for
-// large spheres (sphere_wave_kernel has both sides' times).
+// tile the averaging kernels stage with it: 8 x 8 x 8 cells in 3D (two blocks fit a CU), 16 x 32 in 2D,
+// 256 in 1D; none on small grids and for large spheres (sphere_wave_kernel has both sides' times).
 void make_sphere(const mpf_ctx* c, int range, mpf_sphere* p)
 {
     const int n[3] = {c->nx, c->ny, c->nz}, d[3] = {c->dnx, c->dny, c->dnz};
@@ -488,10 +486,8 @@ void make_sphere(const mpf_ctx* c, int range, mpf_sphere* p)
     }
     if (c->active == 2) p->tile[last] = std::min(32, n[last]);
     auto box = [&](int q) { return p->tile[q] + 2 * p->reach[q]; };
-    auto bytes = [&]() { return static_cast<int64_t>(box(0)) * box(1) * (box(2) * mpf::kSphereCellBytes + 4); };
-    if (c->active == 3 && bytes() > 78 * 1024) p->tile[0] = std::min(4, n[0]);
     const size_t most = c->active == 2 ? mpf::kSphereOffsets2d : mpf::kSphereOffsets;
-    if (c->ncells < mpf::kSphereGrid || p->w.size() > most || bytes() > mpf::kSphereLds || box(2) > mpf::kSphereCells) {
+    if (c->ncells < mpf::kSphereGrid || p->w.size() > most) {
         p->tile[0] = p->tile[1] = p->tile[2] = 0;
         return;
     }

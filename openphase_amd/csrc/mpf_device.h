@@ -76,10 +76,7 @@ struct StepArgs {
     uint32_t* work_list;         // [ncells] deferred cells; bit 31: known to merge more than six entries
     unsigned* work_count;        // [3] its length, how many of them have bit 31, and how many others turned
                                  // out to merge more than six
-    // launch shape (chosen by mpf_autotune): XCD-contiguous block order of the step kernel, and
-    // the number of blocks of the deferred-cell kernel
-    int32_t xcd_order;
-    int32_t deferred_grid;
+    int32_t xcd_order;           // XCD-contiguous block order of the step kernel (chosen by mpf_autotune)
     // LDS-tiled step kernel (mpf_tile.hip): tile of tile_y x tile_z cells of the (y, z) plane
     // marching through tile_x planes along x; tile_x = 0 selects the per-cell step kernel
     int32_t tile_x, tile_y, tile_z;
@@ -168,7 +165,9 @@ constexpr int kSphereOffsets2d = 64;     // the same in 2D
 constexpr int64_t kSphereGrid = int64_t{1} << 18;  // cells from which tiles are staged: fewer leave CUs idle
 constexpr int kSphereCells = 512;        // cells of a staged tile at most
 constexpr int kSphereCellBytes = 25;     // LDS per staged cell
-constexpr int kSphereLds = 150 * 1024;   // LDS of a staged tile at most
+static_assert(256 + kSphereOffsets - 1 <= kSphereCells, "a staged row of a 1D tile and its halo");
+// LDS of a staged tile at most: 3D, Range 4 (251 offsets, a reach of three cells)
+constexpr int kSphereLds = 14 * 14 * (14 * kSphereCellBytes + 4);
 int sphere_lds_limit();                  // to be called before the first launch with tx > 0
 // Averaged driving force (avg = s.dg_avg).
 int launch_dg_average(const SphereArgs& a, bool fp32, void* stream);

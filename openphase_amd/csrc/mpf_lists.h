@@ -198,7 +198,7 @@ __host__ __device__ __forceinline__ TC ip_pair_energy(const StepArgs& A, int k, 
     return en;
 }
 
-enum CellResult { kCellBulk = 0, kCellWide = 1, kCellDeferred = 2, kCellOverflow = 3 };
+enum CellResult { kCellBulk = 0, kCellWide = 1, kCellDeferred = 2 };
 
 // Count byte of a stored list. FP64 states store the entry count. FP32 states store
 // count | (implicit slot << 4): the cell's own update recovers the largest entry as

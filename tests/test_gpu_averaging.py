@@ -65,7 +65,7 @@ def test_driving_force_on_tiles(weights):
 
 # grids of at least 2^18 cells with remainders on every axis, of one, two and three axes, and lists of up to
 # six entries (beyond the four grains a staged cell holds)
-TILED = [((521, 509, 0), 4), ((521, 0, 509), 3), ((0, 521, 509), 2), ((262149, 0, 0), 5), ((67, 61, 65), 3), ((67, 61, 65), 4)]
+TILED = [((521, 509, 0), 4), ((521, 0, 509), 3), ((0, 521, 509), 2), ((262149, 0, 0), 128), ((67, 61, 65), 3), ((67, 61, 65), 4)]
 
 
 def _driving(dims, reach, weights, precision=0):
