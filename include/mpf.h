@@ -222,9 +222,9 @@ mpf_status mpf_last_timing(mpf_ctx* ctx, double* step_kernel_ms, double* rest_ms
 /* Enables/disables per-kernel HIP event timing in mpf_step (off by default). */
 mpf_status mpf_enable_timing(mpf_ctx* ctx, int32_t on);
 
-/* Cumulative number of cell-steps finished outside the main kernel since creation: merged lists
- * of 5-6 entries (or more than 8 own entries) and lists of 1, 7-16 entries (no reference
- * counterpart: the reference has one code path). */
+/* Cumulative number of cell-steps finished by the deferred-cell kernel since creation: those that the
+ * main kernel did not know to merge more than six entries, and those that merge more than six (some of
+ * the first among them; no reference counterpart: the reference has one code path). */
 mpf_status mpf_step_stats(mpf_ctx* ctx, int64_t* deferred_mid, int64_t* deferred_wide);
 
 /* Measurement helper (no reference counterpart): copies `bytes` (multiple of 16) between two

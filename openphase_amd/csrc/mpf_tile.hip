@@ -18,7 +18,7 @@
 // Laplacian (and gradient) of merged entry t is a sum over the 27 neighbours of one LDS value each,
 // at rank popcount(mask & below(t)) or a zero when the bit is clear: no list searches.
 //
-// Cells the tile cannot hold - a neighbourhood with a list of more than three entries or a grain
+// Cells the tile cannot hold - a neighbourhood with a list of more than four entries or a grain
 // that did not fit the 32 local ids, more than four merged entries, fewer than two - go to the
 // deferred-cell work list, whose kernel handles any list.
 //

@@ -271,7 +271,8 @@ class Engine:
         return a.value, b.value
 
     def step_stats(self):
-        """Cumulative (mid-kernel, wide-kernel) cell-steps since creation."""
+        """Cumulative deferred cell-steps since creation: (not known beforehand to merge more than six
+        entries, merging more than six)."""
         a, b = C.c_int64(), C.c_int64()
         self._check(self.lib.mpf_step_stats(self.h, C.byref(a), C.byref(b)), "mpf_step_stats")
         return a.value, b.value
